@@ -5,18 +5,20 @@
 // (170-219) and matmul_a_bt (221-268), and the process-wide workspace with
 // matmul_gpu / matmul_at_b_gpu / matmul_a_bt_gpu (283-327) that
 // crates/prichs-core/src/ops.rs:3, 24-31 dispatches every large matmul_2d
-// to.  Shapes are arbitrary (no multiple-of-tile requirement): the kernel
-// loads its operand tiles with bounds checks and zero fill.
+// to.  Shapes are arbitrary (no multiple-of-tile requirement).
 //
 // Arithmetic: v_mfma_f32_16x16x4f32 -- full f32 products with f32
 // accumulation (the reference's cuBLAS runs TF32 tensor cores,
 // engine.rs:370 / cublas.rs:72; this path is at least as precise and stays
 // within 1e-4 of the reference's CPU loop, crates/prichs-core/src/ops.rs:
 // 33-58, on its shapes).
+#include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <new>
 
 #include "common.hpp"
+#include "f32_tile.hpp"
 
 struct prichs_gpu_workspace {
   std::mutex mu;  // serialises the calls on this handle (the reference's Mutex<GpuWorkspace>)
@@ -29,102 +31,102 @@ struct prichs_gpu_workspace {
 namespace prichs {
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int kTile = 64;    // output tile (rows and columns)
-constexpr int kStepR = 16;   // reduction elements per LDS stage
-constexpr int kThreads = 256;
+using f32t::f32x4;
 
 // C[M, N] = sum_r opA(i, r) opB(r, j), row-major C with ldc = N.
 //   OP 0 (A B):    opA(i, r) = A[i R + r],  opB(r, j) = B[r N + j]
 //   OP 1 (A^T B):  opA(i, r) = A[r M + i],  opB(r, j) = B[r N + j]
 //   OP 2 (A B^T):  opA(i, r) = A[i R + r],  opB(r, j) = B[j R + r]
-// One workgroup per 64 x 64 tile (tiles numbered row-major over the grid),
-// 4 waves of 32 x 32 (2 x 2 MFMA blocks of 16 x 16).  The operand tiles go
-// through LDS as [row][r] with a padded row, loaded so that consecutive
-// threads read consecutive addresses of whichever index is contiguous.
-template <int OP>
-__global__ __launch_bounds__(kThreads) void f32_matmul_kernel(const float *__restrict__ A,
-                                                              const float *__restrict__ B,
-                                                              float *__restrict__ C, long long M,
-                                                              long long N, long long R,
-                                                              long long n_tiles) {
-  __shared__ float As[kTile][kStepR + 1];
-  __shared__ float Bs[kTile][kStepR + 1];
-  const long long tile = blockIdx.x;
-  const long long m0 = (tile / n_tiles) * kTile;
-  const long long n0 = (tile % n_tiles) * kTile;
+// One workgroup per tile; tiles in bands of 4 tile rows, column by column in
+// a band, each XCD taking a contiguous run of them.  Rows and columns past
+// the matrix read its last ones and are not stored.
+template <class T, int OP>
+__global__ __launch_bounds__(T::kThreads) void f32_matmul_kernel(
+    const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, long long M,
+    long long N, long long R, unsigned m_tiles, unsigned n_tiles, int vec_c) {
+  __shared__ __attribute__((aligned(16))) float lds[T::kLdsFloats];
   const int t = threadIdx.x;
-  const int lane = t & 63, wave = t >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-
-  // Loader coordinates: "rc" = the reduction index is the contiguous one.
-  constexpr bool a_rc = OP != 1, b_rc = OP == 2;
-  const int a_i = a_rc ? t >> 2 : (t & 15) * 4, a_r = a_rc ? (t & 3) * 4 : t >> 4;
-  const int b_j = b_rc ? t >> 2 : (t & 15) * 4, b_r = b_rc ? (t & 3) * 4 : t >> 4;
-
-  f32x4 acc[2][2];
+  const unsigned id = f32t::xcd_run(blockIdx.x, gridDim.x);
+  const unsigned band = id / n_tiles / 4, in = id - band * 4 * n_tiles;
+  const unsigned rows = min(4u, m_tiles - band * 4);
+  const long long m0 = (long long)(band * 4 + in % rows) * T::BM;
+  const long long n0 = (long long)(in / rows) * T::BN;
+  T tile(t);
+  typename T::OpA oa;
+  typename T::OpB ob;
+  if constexpr (OP == 1)
+    oa.init_rm(A + m0, M, M - m0, t);
+  else
+    oa.init_rc([&](int r) { return A + min(m0 + r, M - 1) * R; }, A, t);
+  if constexpr (OP == 2)
+    ob.init_rc([&](int r) { return B + min(n0 + r, N - 1) * R; }, B, t);
+  else
+    ob.init_rm(B + n0, N, N - n0, t);
+  if (!tile.run(lds, oa, ob, R, OP == 1 ? T::BK * M : T::BK, OP == 2 ? T::BK : T::BK * N, t))
+    return;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < T::MI; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  float ra[4], rb[4];
-  auto gload = [&](long long r0) {
+    for (int j = 0; j < T::NJ; ++j) {
+      const long long row = m0 + tile.wm * T::WM + 16 * i + (tile.lane & 15);
+      const long long col = n0 + tile.wn * T::WN + 16 * j + 4 * (tile.lane >> 4);
+      if (row >= M || col >= N) continue;
+      float *dst = C + row * N + col;
+      if (vec_c) {
+        *reinterpret_cast<f32x4 *>(dst) = tile.acc[i][j];
+      } else {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const long long i = m0 + a_i + (a_rc ? 0 : q), ar = r0 + a_r + (a_rc ? q : 0);
-      ra[q] = (i < M && ar < R) ? (OP == 1 ? A[ar * M + i] : A[i * R + ar]) : 0.f;
-      const long long j = n0 + b_j + (b_rc ? 0 : q), br = r0 + b_r + (b_rc ? q : 0);
-      rb[q] = (j < N && br < R) ? (OP == 2 ? B[j * R + br] : B[br * N + j]) : 0.f;
-    }
-  };
-  auto lstore = [&]() {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      As[a_i + (a_rc ? 0 : q)][a_r + (a_rc ? q : 0)] = ra[q];
-      Bs[b_j + (b_rc ? 0 : q)][b_r + (b_rc ? q : 0)] = rb[q];
-    }
-  };
-
-  // MFMA operands (v_mfma_f32_16x16x4f32): lane l holds A[row l%16][k l/16]
-  // and B[k l/16][col l%16]; the result lane holds rows 4 (l/16) + 0..3 of
-  // column l%16.
-  const int fr = lane & 15, fk = lane >> 4;
-  gload(0);
-  for (long long r0 = 0; r0 < R; r0 += kStepR) {
-    __syncthreads();  // the previous stage's reads are done
-    lstore();
-    __syncthreads();
-    if (r0 + kStepR < R) gload(r0 + kStepR);
-#pragma unroll
-    for (int ks = 0; ks < kStepR / 4; ++ks) {
-      const int kk = ks * 4 + fk;
-      float af[2], bf[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) af[i] = As[wm * 32 + i * 16 + fr][kk];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) bf[j] = Bs[wn * 32 + j * 16 + fr][kk];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i], bf[j], acc[i][j], 0, 0, 0);
-    }
-  }
-
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const long long col = n0 + wn * 32 + j * 16 + fr;
-      if (col >= N) continue;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const long long row = m0 + wm * 32 + i * 16 + 4 * fk + r;
-        if (row < M) C[row * N + col] = acc[i][j][r];
+        for (int e = 0; e < 4; ++e)
+          if (col + e < N) dst[e] = tile.acc[i][j][e];
       }
     }
+}
+
+// The tile shapes, from large outputs to outputs of a few tiles with a long
+// reduction (waves m x n x k: the last split the reduction).
+template <int CFG, int OP, int W> struct MatmulCfg;
+#define PRICHS_MATMUL_CFG(I, BM, BN, BK, WM, WN, WK)                                      \
+  template <int OP, int W> struct MatmulCfg<I, OP, W> {                                   \
+    typedef f32t::Tile<BM, BN, BK, WM, WN, WK, OP != 1, OP == 2, W> T;                    \
+  };
+PRICHS_MATMUL_CFG(0, 128, 128, 32, 2, 2, 1)
+PRICHS_MATMUL_CFG(1, 64, 64, 64, 2, 2, 2)
+PRICHS_MATMUL_CFG(2, 32, 64, 64, 1, 2, 2)
+PRICHS_MATMUL_CFG(3, 32, 32, 64, 2, 2, 2)
+PRICHS_MATMUL_CFG(4, 16, 16, 256, 1, 1, 8)
+#undef PRICHS_MATMUL_CFG
+constexpr int kMatmulCfgs = 5;
+
+// Nanoseconds per reduction element of one tile on a CU: alone, and each of
+// several on the same CU (measured on MI355X at 512 x 512 x 2048, 128 x 128 x
+// 4096, 1024^3, 2048 x 1280 x 1536 and 4096 x 4096 x 1024; the single-element
+// loads at 145 x 58 x 1895 and 1001 x 777 x 333, where they bound the small
+// tiles).  The shape with the least whole rounds x time wins: at 1024^3 64 x
+// 64 tiles take 22.0 us against 69.5 (128 x 128, 64 CUs busy) and 25.6 (32 x
+// 32), at 4096 x 4096 x 1024 288 against 258 and 356, at 128 x 128 x 4096 72
+// against 256 and 26, and 16 x 16 with the reduction over 8 waves 10.2.
+struct MatmulTileCost {
+  int bm, bn, bk;
+  double alone[2], shared[2];  // [0] 16-byte, [1] single-element loads
+};
+constexpr MatmulTileCost kMatmulCost[kMatmulCfgs] = {
+    {128, 128, 32, {63.0, 78.0}, {63.0, 78.0}}, {64, 64, 64, {18.6, 30.0}, {17.8, 30.0}},
+    {32, 64, 64, {12.7, 18.0}, {9.7, 20.0}},    {32, 32, 64, {7.2, 10.5}, {5.6, 11.0}},
+    {16, 16, 256, {2.5, 5.7}, {2.6, 10.0}},
+};
+
+int matmul_cfg(size_t M, size_t N, size_t R, bool vec, int cus) {
+  int best = 0;
+  double best_t = 0;
+  for (int c = 0; c < kMatmulCfgs; ++c) {
+    const MatmulTileCost &k = kMatmulCost[c];
+    const double tiles = (double)cdiv(M, k.bm) * (double)cdiv(N, k.bn);
+    if (c > 0 && tiles > (double)INT32_MAX) continue;
+    const double rounds = std::ceil(tiles / cus);
+    const double t = (double)roundup(R, k.bk) * std::max(k.alone[!vec], rounds * k.shared[!vec]);
+    if (c == 0 || t < best_t) best = c, best_t = t;
+  }
+  return best;
 }
 
 // Product of two sizes, or SIZE_MAX when it overflows.
@@ -157,20 +159,52 @@ int check_matmul(int op, size_t m, size_t k, size_t n, const char *who, MatmulDi
   return PRICHS_OK;
 }
 
+template <int CFG, int OP, int W>
+void launch_matmul_kernel(const float *a, const float *b, float *c, const MatmulDims &d, int vec_c,
+                          hipStream_t s) {
+  typedef typename MatmulCfg<CFG, OP, W>::T T;
+  const unsigned mt = (unsigned)cdiv(d.M, T::BM), nt = (unsigned)cdiv(d.N, T::BN);
+  hipLaunchKernelGGL((f32_matmul_kernel<T, OP>), dim3(mt * nt), dim3(T::kThreads), 0, s, a, b, c,
+                     (long long)d.M, (long long)d.N, (long long)d.R, mt, nt, vec_c);
+}
+
+template <int OP, int W>
+void launch_matmul_cfg(int cfg, const float *a, const float *b, float *c, const MatmulDims &d,
+                       int vec_c, hipStream_t s) {
+  switch (cfg) {
+    case 0: return launch_matmul_kernel<0, OP, W>(a, b, c, d, vec_c, s);
+    case 1: return launch_matmul_kernel<1, OP, W>(a, b, c, d, vec_c, s);
+    case 2: return launch_matmul_kernel<2, OP, W>(a, b, c, d, vec_c, s);
+    case 3: return launch_matmul_kernel<3, OP, W>(a, b, c, d, vec_c, s);
+    default: return launch_matmul_kernel<4, OP, W>(a, b, c, d, vec_c, s);
+  }
+}
+
 int launch_matmul(int op, const float *a, const float *b, float *c, const MatmulDims &d,
                   hipStream_t s) {
   if (d.M == 0 || d.N == 0) return PRICHS_OK;
-  const long long mt = (long long)cdiv(d.M, kTile), nt = (long long)cdiv(d.N, kTile);
-  PRICHS_REQUIRE(mt * nt <= (long long)INT32_MAX, "matmul: %zu x %zu output has too many tiles",
-                 d.M, d.N);
-  const dim3 grid((unsigned)(mt * nt));
-  const long long M = (long long)d.M, N = (long long)d.N, R = (long long)d.R;
+  PRICHS_REQUIRE(cdiv(d.M, 64) * cdiv(d.N, 64) <= (size_t)INT32_MAX,
+                 "matmul: %zu x %zu output has too many tiles", d.M, d.N);
+  const int cus = device_cu_count();
+  if (cus <= 0) return fail(PRICHS_ERR_HIP, "matmul: cannot query the device");
+  // 16-byte loads where every row of both operands starts 16-byte aligned,
+  // 16-byte stores where every row of C does.
+  auto aligned = [](const float *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  const size_t lda = op == PRICHS_MATMUL_ATB ? d.M : d.R;
+  const size_t ldb = op == PRICHS_MATMUL_ABT ? d.R : d.N;
+  const bool vec = lda % 4 == 0 && ldb % 4 == 0 && aligned(a) && aligned(b);
+  const int vec_c = d.N % 4 == 0 && aligned(c);
+  const int cfg = matmul_cfg(d.M, d.N, d.R, vec, cus);
+#define PRICHS_MATMUL_OP(OP)                                     \
+  (vec ? launch_matmul_cfg<OP, 4>(cfg, a, b, c, d, vec_c, s)     \
+       : launch_matmul_cfg<OP, 1>(cfg, a, b, c, d, vec_c, s))
   if (op == PRICHS_MATMUL_ATB)
-    hipLaunchKernelGGL(f32_matmul_kernel<1>, grid, dim3(kThreads), 0, s, a, b, c, M, N, R, nt);
+    PRICHS_MATMUL_OP(1);
   else if (op == PRICHS_MATMUL_ABT)
-    hipLaunchKernelGGL(f32_matmul_kernel<2>, grid, dim3(kThreads), 0, s, a, b, c, M, N, R, nt);
+    PRICHS_MATMUL_OP(2);
   else
-    hipLaunchKernelGGL(f32_matmul_kernel<0>, grid, dim3(kThreads), 0, s, a, b, c, M, N, R, nt);
+    PRICHS_MATMUL_OP(0);
+#undef PRICHS_MATMUL_OP
   PRICHS_LAUNCH_CHECK("matmul launch");
   return PRICHS_OK;
 }

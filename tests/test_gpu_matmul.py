@@ -191,3 +191,39 @@ def test_matmul_device_entry_on_stream_and_big_reduction(cuda, orc):
         out = ops.matmul_f32(L.MATMUL_AB, ta, tb, stream=s)
     s.synchronize()
     assert rel_err(out.cpu().numpy(), orc.matmul_2d(a, b)) <= TOL
+
+
+# (M, N, R) of the output and the reduction: each tile shape of the kernel
+# with 16-byte loads (every row start a multiple of 4 elements) and with
+# single-element ones, ending inside a tile and inside a reduction step.
+@pytest.mark.parametrize("M,N,R", [(2044, 2040, 36), (1999, 2001, 33),    # 128 x 128
+                                   (1000, 1020, 100), (1001, 777, 101),   # 64 x 64
+                                   (1272, 1000, 68), (500, 1001, 69),     # 32 x 64
+                                   (300, 500, 132), (300, 301, 69),       # 32 x 32
+                                   (36, 68, 260), (17, 45, 257)])         # 16 x 16
+@pytest.mark.parametrize("op", [L.MATMUL_AB, L.MATMUL_ATB, L.MATMUL_ABT],
+                         ids=["ab", "at_b", "a_bt"])
+def test_matmul_tile_shapes(cuda, op, M, N, R):
+    # Against the 64-bit product within the a-priori bound of an R-term f32
+    # sum, (R + 1) 2^-24 sum_r |a||b|; the same from operands and into an
+    # output that start 4 bytes past a 16-byte boundary; nothing past the
+    # output is written.
+    say(f"case: op {op} M={M} N={N} R={R}")
+    rng = np.random.default_rng(M + N + R + op)
+    a = rng.standard_normal((M, R)).astype(np.float32)
+    b = rng.standard_normal((R, N)).astype(np.float32)
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    bound = (R + 1) * 2.0**-24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64))
+    a, b = (a.T if op == L.MATMUL_ATB else a), (b.T if op == L.MATMUL_ABT else b)
+
+    def shifted(x, by):
+        t = torch.empty(x.size + 8, device="cuda")[by:by + x.size].view(x.shape)
+        return t.copy_(torch.from_numpy(np.ascontiguousarray(x)))
+
+    for by in (0, 1):
+        buf = torch.full((M * N + 8,), 7.0, device="cuda")
+        out = buf[by:by + M * N].view(M, N)
+        ops.matmul_f32(op, shifted(a, by), shifted(b, by), out=out)
+        err = np.abs(out.cpu().numpy().astype(np.float64) - ref)
+        assert (err <= bound).all()
+        assert (buf[:by] == 7).all() and (buf[by + M * N:] == 7).all()
