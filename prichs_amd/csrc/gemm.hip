@@ -26,8 +26,8 @@
 // activations, or in the training forward the pre-activations, whose
 // activations then exchange halves between lane pairs and write 16 bytes per
 // lane).
-// f32 kernel: 128x128x16 tiles on v_mfma_f32_16x16x4_f32 (the fp32-checked
-// mode; accumulates in fp32 like the reference CPU path).
+// f32 kernel: the tiles of f32_tile.hpp on v_mfma_f32_16x16x4_f32 (the fp32-
+// checked mode; accumulates in fp32 like the reference CPU path).
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -35,6 +35,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "f32_tile.hpp"
 #include "router_quad.hpp"
 
 namespace prichs {
@@ -81,36 +82,10 @@ constexpr int kBf16KMultiple = 64;   // bf16 kernels need d and f to be multiple
 // ------------------------------------------------------------------------
 // Tile scheduler shared by the kernels.
 // ------------------------------------------------------------------------
-struct TileMap {
-  int prefix[kMaxGroups + 1];  // first global M-tile of each group
-  int offs[kMaxGroups + 1];    // offsets[] of the launch (row range of each group)
-};
-
-// offsets == nullptr is the dense case: one group of dense_m rows (G == 1).
-__device__ inline void build_tile_map(TileMap &tm, const int32_t *offsets, int G, int BM,
-                                      int dense_m) {
-  if (threadIdx.x == 0 && offsets == nullptr) {
-    tm.prefix[0] = 0;
-    tm.offs[0] = 0;
-    tm.prefix[1] = (dense_m + BM - 1) / BM;
-    tm.offs[1] = dense_m;
-  } else if (threadIdx.x == 0) {
-    int run = 0;
-    for (int g = 0; g < G; ++g) {
-      tm.prefix[g] = run;
-      tm.offs[g] = offsets[g];
-      const int mg = offsets[g + 1] - offsets[g];
-      run += mg > 0 ? (mg + BM - 1) / BM : 0;
-    }
-    tm.prefix[G] = run;
-    tm.offs[G] = offsets[G];
-  }
-  __syncthreads();
-}
-
-// The same table held in registers by every wave of a launch (the bf16
-// kernels' LDS is all ring): entry e <= G -- the first global M-tile (prefix)
-// and first row (offs) of group e -- sits in lane e % 64 of word e / 64.
+// The groups' tiles, held in registers by every wave of a launch: entry e <= G
+// -- the first global M-tile (prefix) and first row (offs) of group e -- sits
+// in lane e % 64 of word e / 64.  offsets == nullptr is the dense case: one
+// group of dense_m rows (G == 1).
 struct WaveTileMap {
   int prefix[2], offs[2];
   int G, m_tiles;
@@ -159,13 +134,6 @@ __device__ __forceinline__ int wave_find_group(const WaveTileMap &tm, int mt) {
   const unsigned long long b0 = __ballot(lane >= 1 && lane < tm.G && tm.prefix[0] <= mt);
   const unsigned long long b1 = __ballot(64 + lane < tm.G && tm.prefix[1] <= mt);
   return __builtin_amdgcn_readfirstlane(__popcll(b0) + __popcll(b1));
-}
-
-// Group of global M-tile mt (empty groups own no tiles and are skipped).
-__device__ inline int find_group(const TileMap &tm, int G, int mt) {
-  int g = 0;
-  while (g + 1 < G && tm.prefix[g + 1] <= mt) ++g;
-  return g;
 }
 
 // Linear tile id -> (M-tile, N-tile): bands of PRICHS_BAND_M M-tiles with the
@@ -818,162 +786,138 @@ __global__ __launch_bounds__(kBf16Threads) void bf16_gemm_kernel(
 // f32 kernel (fp32-checked mode)
 // ------------------------------------------------------------------------
 namespace fp {
-constexpr int BM = 128, BN = 128, BK = 16;
-constexpr int kThreads = 256;
-constexpr int WM = 64, WN = 64;
-constexpr int MI = WM / 16, NJ = WN / 16;
+constexpr int kPadN = 128;     // packed gate/up rows: padded to this
+constexpr int kKMultiple = 16;  // d and f must be multiples of this
 constexpr int kIl = 32;
-constexpr int kLd = BK + 1;  // padded LDS row (floats)
-constexpr int kStage = (BM + BN) * kLd;
-constexpr size_t kLdsBytes = 2 * kStage * sizeof(float);
-static_assert(WN == 2 * kIl, "a wave's N sub-tile must hold one gate/up block");
-static_assert(BN == 4 * kIl, "packed gate/up rows are padded to a multiple of 4 * il");
 
-template <bool GATEUP>
-__global__ __launch_bounds__(kThreads) void grouped_gemm_kernel(
+// A tile of f32_tile.hpp per (group, M-tile, N-tile).  A wave's N sub-tile is
+// one whole [32 gate | 32 up] block, so the SwiGLU stays in its registers.
+// A, B and the C tile's rows are K-contiguous; K a multiple of 16.
+template <class T, bool GATEUP>
+__global__ __launch_bounds__(T::kThreads) void grouped_gemm_kernel(
     const float *__restrict__ A, const int32_t *__restrict__ a_rows, int lda,
     const float *__restrict__ B, long long b_group_stride, int Np, int K,
     float *__restrict__ C, int ldc, int n_store, const int32_t *__restrict__ offsets, int G,
-    int dense_m, float *__restrict__ P) {
-  extern __shared__ float ldsf[];
-  __shared__ TileMap tm;
-  build_tile_map(tm, offsets, G, BM, dense_m);
+    int dense_m, float *__restrict__ P, int vec_c) {
+  static_assert(T::WN == 2 * kIl, "a wave's N sub-tile holds one gate/up block");
+  __shared__ __attribute__((aligned(16))) float lds[T::kLdsFloats];
+  WaveTileMap tm;
+  build_wave_tile_map(tm, offsets, G, T::BM, dense_m);
+  const int t = threadIdx.x;
+  const int n_tiles = Np / T::BN;
+  const unsigned total = (unsigned)(tm.m_tiles * n_tiles);
+  T tile(t);
+  const int fr = tile.lane & 15, fc = 4 * (tile.lane >> 4);
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int n_tiles = Np / BN;
-  const int total = tm.prefix[G] * n_tiles;
-  const int KT = K / BK;
-  const int ld_row = tid >> 2;  // + 64*i
-  const int ld_c4 = (tid & 3) * 4;
-
-  for (int tile = blockIdx.x; tile < total; tile += gridDim.x) {
-    const int mt = tile / n_tiles;
-    const int nt = tile - mt * n_tiles;
-    const int g = find_group(tm, G, mt);
-    const int row0 = tm.offs[g];
-    const int mg = tm.offs[g + 1] - row0;
-    const int m0 = (mt - tm.prefix[g]) * BM;
-    const int n0 = nt * BN;
+  for (unsigned b = blockIdx.x; b < total; b += gridDim.x) {
+    if (b != blockIdx.x) f32t::lds_barrier();  // the tile before is out of the LDS
+    int mt, nt;
+    tile_coords((int)f32t::xcd_run(b, total), tm.m_tiles, n_tiles, mt, nt);
+    const int g = wave_find_group(tm, mt);
+    const int row0 = wave_entry(tm.offs, g);
+    const int mg = wave_entry(tm.offs, g + 1) - row0;
+    const int m0 = (mt - wave_entry(tm.prefix, g)) * T::BM;
+    const int n0 = nt * T::BN;
     const float *Bg = B + (long long)g * b_group_stride;
-    const float *a_ptr[2];
-    const float *b_ptr[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      int lr = m0 + ld_row + 64 * i;
-      lr = lr < mg ? lr : mg - 1;
-      const int vr = row0 + lr;
-      const int src = a_rows ? a_rows[vr] : vr;
-      a_ptr[i] = A + (long long)src * lda + ld_c4;
-      b_ptr[i] = Bg + (long long)(n0 + ld_row + 64 * i) * K + ld_c4;
-    }
-    f32x4 acc[MI][NJ];
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    typename T::OpA oa;
+    typename T::OpB ob;
+    // Rows past the group read its last row; their outputs are dropped.
+    oa.init_rc(
+        [&](int r) {
+          const int vr = row0 + min(m0 + r, mg - 1);
+          return A + (long long)(a_rows ? a_rows[vr] : vr) * lda;
+        },
+        A, t);
+    ob.init_rc([&](int r) { return Bg + (long long)(n0 + r) * K; }, Bg, t);
+    if (!tile.run(lds, oa, ob, K, T::BK, T::BK, t)) continue;
 
-    float4 ra[2], rb[2];
-    auto gload = [&](int k0) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        ra[i] = *reinterpret_cast<const float4 *>(a_ptr[i] + k0);
-        rb[i] = *reinterpret_cast<const float4 *>(b_ptr[i] + k0);
+    for (int i = 0; i < T::MI; ++i) {
+      const int lr = m0 + tile.wm * T::WM + 16 * i + fr;
+      if (lr >= mg) continue;
+      const long long row = row0 + lr;
+      if (GATEUP && P != nullptr) {
+        // Training forward: the pre-activations, [rows][Np] in packed order.
+        float *prow = P + row * Np + n0 + tile.wn * T::WN + fc;
+#pragma unroll
+        for (int j = 0; j < T::NJ; ++j) *reinterpret_cast<f32x4 *>(prow + 16 * j) = tile.acc[i][j];
       }
-    };
-    auto lstore = [&](int buf) {
-      float *as = ldsf + buf * kStage;
-      float *bs = as + BM * kLd;
+      constexpr int kCols = GATEUP ? T::NJ / 2 : T::NJ;
+      const int c0 = (GATEUP ? (n0 + tile.wn * T::WN) / 2 : n0 + tile.wn * T::WN) + fc;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        float *pa = as + (ld_row + 64 * i) * kLd + ld_c4;
-        float *pb = bs + (ld_row + 64 * i) * kLd + ld_c4;
-        pa[0] = ra[i].x; pa[1] = ra[i].y; pa[2] = ra[i].z; pa[3] = ra[i].w;
-        pb[0] = rb[i].x; pb[1] = rb[i].y; pb[2] = rb[i].z; pb[3] = rb[i].w;
+      for (int j = 0; j < kCols; ++j) {
+        const int col = c0 + 16 * j;
+        if (col >= n_store) continue;
+        f32x4 v = tile.acc[i][j];
+        if (GATEUP) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = silu_ref(v[e]) * tile.acc[i][(j + kCols) % T::NJ][e];
+        }
+        float *dst = C + row * ldc + col;
+        if (vec_c) {
+          *reinterpret_cast<f32x4 *>(dst) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (col + e < n_store) dst[e] = v[e];
+        }
       }
-    };
-    auto compute = [&](int buf) {
-      const float *as = ldsf + buf * kStage;
-      const float *bs = as + BM * kLd;
-#pragma unroll
-      for (int ks = 0; ks < BK / 4; ++ks) {
-        const int kk = ks * 4 + (lane >> 4);
-        float af[MI], bfr[NJ];
-#pragma unroll
-        for (int i = 0; i < MI; ++i) af[i] = as[(wm * WM + i * 16 + (lane & 15)) * kLd + kk];
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) bfr[j] = bs[(wn * WN + j * 16 + (lane & 15)) * kLd + kk];
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int j = 0; j < NJ; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i], bfr[j], acc[i][j], 0, 0, 0);
-      }
-    };
-
-    gload(0);
-    lstore(0);
-    __syncthreads();
-    for (int kt = 0; kt < KT; ++kt) {
-      const bool more = kt + 1 < KT;
-      if (more) gload((kt + 1) * BK);
-      compute(kt & 1);
-      if (more) lstore((kt + 1) & 1);
-      __syncthreads();
-    }
-
-    const int rbase = m0 + wm * WM + 4 * (lane >> 4);
-    if (GATEUP && P != nullptr) {
-      // Training forward: the pre-activations, [rows][Np] in packed order.
-      const int pbase = n0 + wn * WN + (lane & 15);
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int lr = rbase + i * 16 + r;
-          if (lr < mg) {
-            float *prow = P + (long long)(row0 + lr) * Np + pbase;
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) prow[j * 16] = acc[i][j][r];
-          }
-        }
-    }
-    if (GATEUP) {
-      const int cbase = (n0 / (2 * kIl) + wn) * kIl + (lane & 15);
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int lr = rbase + i * 16 + r;
-          if (lr < mg) {
-            float *crow = C + (long long)(row0 + lr) * ldc;
-#pragma unroll
-            for (int j = 0; j < NJ / 2; ++j) {
-              const int col = cbase + j * 16;
-              if (col < n_store) crow[col] = silu_ref(acc[i][j][r]) * acc[i][j + NJ / 2][r];
-            }
-          }
-        }
-    } else {
-      const int cbase = n0 + wn * WN + (lane & 15);
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int lr = rbase + i * 16 + r;
-          if (lr < mg) {
-            float *crow = C + (long long)(row0 + lr) * ldc;
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-              const int col = cbase + j * 16;
-              if (col < n_store) crow[col] = acc[i][j][r];
-            }
-          }
-        }
     }
   }
+}
+
+// Tile shapes, and nanoseconds per K element of one tile on a CU: alone, and
+// each of several on it (measured on MI355X, dense: 6144 x 512 x 512 takes
+// 37.7 / 29.5 / 33.5 us in the three shapes, 1536 x 256 x 256 20.8 / 7.6 /
+// 6.1, 4096 x 4096 x 1024 252 / 269 / 305).
+struct TileCost {
+  int bm, bn;
+  double alone, shared;
+};
+constexpr TileCost kTileCost[3] = {{128, 128, 63.0, 63.0}, {64, 64, 18.0, 16.4}, {32, 64, 12.2, 9.4}};
+typedef f32t::Tile<128, 128, 32, 2, 2, 1, true, true> Large;
+typedef f32t::Tile<64, 64, 32, 4, 1, 1, true, true> Medium;
+typedef f32t::Tile<32, 64, 64, 2, 1, 2, true, true> Small;
+
+// The shape with the least whole rounds of the chip x time.  The groups' last
+// M-tiles are half full on average (their row counts are on the device).
+int tile_choice(size_t max_rows, int G, int Np, int cus) {
+  int best = 0;
+  double best_t = 0;
+  for (int c = 0; c < 3; ++c) {
+    const TileCost &k = kTileCost[c];
+    const double mt = (double)max_rows / k.bm + (G > 1 ? 0.5 * G : 0.0);
+    const double rounds = std::ceil(std::ceil(mt) * (Np / k.bn) / cus);
+    const double t = std::max(k.alone, rounds * k.shared);
+    if (c == 0 || t < best_t) best = c, best_t = t;
+  }
+  return best;
+}
+
+template <class T, bool GATEUP>
+int launch(const float *A, const int32_t *a_rows, int lda, const float *B, long long b_stride,
+           int Np, int K, float *C, int ldc, int n_store, const int32_t *offsets, int G,
+           int dense_m, size_t max_rows, hipStream_t s, float *pre) {
+  const size_t ub = (max_rows / T::BM + G) * (size_t)(Np / T::BN);
+  // More tiles than that are walked by the same workgroups.
+  const unsigned grid = (unsigned)std::min<size_t>(ub, (size_t)1 << 20);
+  const int vec_c = reinterpret_cast<uintptr_t>(C) % 16 == 0 && ldc % 4 == 0 && n_store % 4 == 0;
+  hipLaunchKernelGGL((grouped_gemm_kernel<T, GATEUP>), dim3(grid), dim3(T::kThreads), 0, s, A,
+                     a_rows, lda, B, b_stride, Np, K, C, ldc, n_store, offsets, G, dense_m, pre,
+                     vec_c);
+  PRICHS_LAUNCH_CHECK("grouped gemm launch");
+  return PRICHS_OK;
+}
+
+template <bool GATEUP>
+int launch_choice(int shape, const float *A, const int32_t *a_rows, int lda, const float *B,
+                  long long b_stride, int Np, int K, float *C, int ldc, int n_store,
+                  const int32_t *offsets, int G, int dense_m, size_t max_rows, hipStream_t s,
+                  float *pre) {
+  auto fn = shape == 0 ? &launch<Large, GATEUP>
+                       : shape == 1 ? &launch<Medium, GATEUP> : &launch<Small, GATEUP>;
+  return fn(A, a_rows, lda, B, b_stride, Np, K, C, ldc, n_store, offsets, G, dense_m, max_rows, s,
+            pre);
 }
 }  // namespace fp
 
@@ -1248,11 +1192,11 @@ __global__ __launch_bounds__(kThreads) void decode_gate_up_router_kernel(SkinnyA
 }  // namespace skinny
 
 size_t il_of(int dtype) { return dtype == PRICHS_DTYPE_BF16 ? (size_t)Bf16::kIl : (size_t)fp::kIl; }
-size_t bn_of(int dtype) { return dtype == PRICHS_DTYPE_BF16 ? (size_t)Bf16::BN : (size_t)fp::BN; }
+size_t bn_of(int dtype) { return dtype == PRICHS_DTYPE_BF16 ? (size_t)Bf16::BN : (size_t)fp::kPadN; }
 
 int check_gemm_shape(size_t d, size_t f, int dtype, const char *who) {
   if (!dtype_ok(dtype)) return fail(PRICHS_ERR_INVALID_ARGUMENT, "%s: bad dtype %d", who, dtype);
-  const size_t q = dtype == PRICHS_DTYPE_BF16 ? (size_t)kBf16KMultiple : (size_t)fp::BK;
+  const size_t q = dtype == PRICHS_DTYPE_BF16 ? (size_t)kBf16KMultiple : (size_t)fp::kKMultiple;
   if (d == 0 || f == 0 || d % q || f % q)
     return fail(PRICHS_ERR_UNSUPPORTED, "%s: d=%zu and f=%zu must be positive multiples of %zu",
                 who, d, f, q);
@@ -1498,17 +1442,12 @@ int launch_grouped(bool gateup, const void *A, const int32_t *a_rows, int lda, c
     return launch_bf16<Bf16Down, false>(A, a_rows, lda, B, b_stride, Np, K, Cp, ldc, n_store,
                                         offsets, G, dense_m, max_rows, cus, s, nullptr);
   } else {
-    const size_t ub = (max_rows / fp::BM + G) * (size_t)(Np / fp::BN);
-    const int grid = (int)std::max<size_t>(1, std::min<size_t>(ub, (size_t)cus * 4));
-    auto kern = gateup ? fp::grouped_gemm_kernel<true> : fp::grouped_gemm_kernel<false>;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(fp::kThreads), fp::kLdsBytes, s,
-                       static_cast<const float *>(A), a_rows, lda,
-                       static_cast<const float *>(B), b_stride, Np, K,
-                       static_cast<float *>(Cp), ldc, n_store, offsets, G, dense_m,
-                       gateup ? static_cast<float *>(pre) : nullptr);
+    auto run = gateup ? &fp::launch_choice<true> : &fp::launch_choice<false>;
+    return run(fp::tile_choice(max_rows, G, Np, cus), static_cast<const float *>(A), a_rows, lda,
+               static_cast<const float *>(B), b_stride, Np, K, static_cast<float *>(Cp), ldc,
+               n_store, offsets, G, dense_m, max_rows, s,
+               gateup ? static_cast<float *>(pre) : nullptr);
   }
-  PRICHS_LAUNCH_CHECK("grouped gemm launch");
-  return PRICHS_OK;
 }
 
 }  // namespace

@@ -204,6 +204,48 @@ def test_gate_up_unaligned_output_bit_identical(cuda):
     assert int(flat[:4].view(torch.int16).abs().sum()) == 0  # nothing written before it
 
 
+# The f32 grouped GEMMs' tile shapes (gate/up | down): 128 x 128 | 32 x 64,
+# 32 x 64 | 128 x 128, 64 x 64 | 32 x 64, and 32 x 64 twice with empty groups
+# and one-row groups; rows and columns ending inside tiles, K inside a step.
+@pytest.mark.parametrize("d,f,counts", [(48, 1008, [1190, 510]), (2000, 48, [1190, 510]),
+                                        (80, 496, [600, 250]), (112, 80, [0, 33, 1, 0, 64, 7])])
+@pytest.mark.parametrize("aligned", [True, False])
+def test_f32_grouped_gemm_tiles(cuda, d, f, counts, aligned):
+    # Against 64-bit products within the a-priori bounds of K-term f32 sums:
+    # eps_K sum |a||b|, eps_K = (K + 1) 2^-24; through silu(g) u (|silu'| <=
+    # 1.1, and 16 ulp for its exponential, division and products).
+    rng = np.random.default_rng(d + f + len(counts))
+    G, rows, Tx = len(counts), sum(counts), 100
+    x = rng.standard_normal((Tx, d)).astype(np.float32)
+    gate, up = (0.1 * rng.standard_normal((2, G, d, f))).astype(np.float32)
+    down = (0.1 * rng.standard_normal((G, f, d))).astype(np.float32)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    row_token = rng.integers(0, Tx, rows).astype(np.int32)
+    gu = ops.to_device_packed([ops.pack_gate_up(gate[g], up[g], "f32") for g in range(G)], "f32")
+    dn = ops.to_device_packed([ops.pack_down(down[g], "f32") for g in range(G)], "f32")
+    off_d, rt_d = dev(offsets).int(), torch.from_numpy(row_token).to("cuda")
+    say("f32 tiles", d, f, counts, aligned)
+    buf = torch.full((rows * f + 8,), 7.0, device="cuda")
+    by = 0 if aligned else 1
+    act = buf[by:by + rows * f].view(rows, f)
+    ops.grouped_gate_up_swiglu(dev(x), rt_d, off_d, G, rows, gu, d, f, out=act)
+    assert (buf[:by] == 7).all() and (buf[by + rows * f:] == 7).all()
+    y = ops.grouped_down(act.clone(), off_d, G, rows, dn, d, f)
+    h_act, h_y = host(act).astype(np.float64), host(y)
+    u = 2.0**-24
+    for g in range(G):
+        r = slice(offsets[g], offsets[g + 1])
+        xr = x[row_token[r]].astype(np.float64)
+        wg, wu, wd = (w[g].astype(np.float64) for w in (gate, up, down))
+        pg, pu = xr @ wg, xr @ wu
+        eg, eu = ((d + 1) * u * (np.abs(xr) @ np.abs(w)) for w in (wg, wu))
+        silu = pg / (1 + np.exp(-pg))
+        bound = 1.1 * eg * (np.abs(pu) + eu) + np.abs(silu) * eu + 16 * u * np.abs(silu * pu)
+        assert (np.abs(h_act[r] - silu * pu) <= bound + 1e-30).all(), ("act", g)
+        bound = (f + 1) * u * (np.abs(h_act[r]) @ np.abs(wd))
+        assert (np.abs(h_y[r] - h_act[r] @ wd) <= bound).all(), ("y", g)
+
+
 # Decode-sized groups (every group <= 64 rows) take the skinny weight-streaming
 # kernel: empty groups, one 16-row MFMA tile, two tiles, two 32-row M-tiles;
 # K with 8, 4 and 2 K-steps per chunk (K % 256, % 128, % 64).
