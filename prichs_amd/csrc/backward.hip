@@ -24,6 +24,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "f32_tile.hpp"
 
 namespace prichs {
 namespace {
@@ -222,28 +223,7 @@ __global__ __launch_bounds__(256) void swiglu_bwd_kernel(T *__restrict__ gu,
 //   gateup: B's columns are packed gate/up (block q = [32 gate | 32 up]); column
 //           p goes to out0 (gate) or out1 (up) at column 32 (p / 64) + p % 32
 //           when that is < f.
-// Workgroups: one per (group, 128 x 128 output tile), the shared group's
-// tiles first (it has the most rows).  Workgroups are dealt round-robin to
-// the 8 XCDs, so block b runs on XCD b % 8; each XCD takes a contiguous band
-// of every group's tiles (tiles in a band share A and B panels in that XCD's
-// L2), and every group's tiles spread over all XCDs.
-namespace wg {
-constexpr int BP = 128, BQ = 128;
-constexpr int kThreads = 256;
-}  // namespace wg
-
 __device__ __forceinline__ int slot_of(int g, int E) { return g < E ? g + 1 : 0; }
-
-// Block -> (group, tile), or false past the last tile (the grid is
-// 8 * band * G with band = ceil(tiles / 8)).
-__device__ __forceinline__ bool wgrad_item(int G, int tiles, int &g, int &tile) {
-  const int band = (tiles + 7) / 8;
-  const int xcd = (int)(blockIdx.x & 7), s = (int)(blockIdx.x >> 3);
-  const int gi = s / band;
-  tile = xcd * band + (s - gi * band);
-  g = (gi + G - 1) % G;  // the last group (shared) first
-  return gi < G && tile < tiles;
-}
 
 // Output element pointer of (i, j) or nullptr when outside the gradient.
 template <bool GATEUP>
@@ -685,15 +665,13 @@ __global__ __launch_bounds__(wgb::kThreads) void wgrad_bf16_kernel(
 
 // Finishes the groups the tile kernel does not write whole: a split group
 // gets its partials in chunk order, dW = beta dW + (((p0 + p1) + p2) + ...);
-// with beta = 0 a group without rows gets zeros.  (split = 0: the f32 kernel,
-// which splits nothing.)
+// with beta = 0 a group without rows gets zeros.
 template <bool GATEUP>
 __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float *__restrict__ part,
                                                            const int32_t *__restrict__ offsets,
                                                            int G, int E, int P, int Q, float *out0,
                                                            float *out1, int ldo,
-                                                           long long slot_stride, int f, int beta,
-                                                           int split) {
+                                                           long long slot_stride, int f, int beta) {
   __shared__ int sg[PRICHS_MAX_EXPERTS + 1], snc[PRICHS_MAX_EXPERTS + 1],
       sps[PRICHS_MAX_EXPERTS + 1];
   __shared__ int n_split;
@@ -714,7 +692,6 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float *__restri
         }
         continue;
       }
-      if (!split) continue;
       int L, nc;
       wg_split(m, L, nc);
       if (nc > 1) {
@@ -797,120 +774,91 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float *__restri
   }
 }
 
-// --- f32 (the fp32-checked mode): v_mfma_f32_16x16x4_f32, K-steps of 16 rows
-// through padded LDS tiles, register double buffering.  Lane l's operand is
-// element (row l / 16, column l % 16) of a 4-row slice: a plain LDS read.
-namespace wgf {
-constexpr int BK = 16;
-constexpr int kLd = 128 + 4;  // padded LDS row (floats)
-constexpr int kTile = BK * kLd;
-constexpr size_t kLdsBytes = 2 * 2 * (size_t)kTile * sizeof(float);  // A and B, two buffers
-}  // namespace wgf
-
-template <bool GATEUP>
-__global__ __launch_bounds__(wg::kThreads) void wgrad_f32_kernel(
+// --- f32 (the fp32-checked mode): the tiles of f32_tile.hpp, both operands
+// reduction-major (rows of P / Q consecutive elements).  One workgroup per
+// (group, tile), the shared group's tiles first: it has the most rows, and no
+// group is split, so a tile of the shared group is the longest item and the
+// others fill in beside it (several workgroups share a CU).  A group without
+// rows gets zeros (beta = 0) or is left alone.
+template <class T, bool GATEUP>
+__global__ __launch_bounds__(T::kThreads) void wgrad_f32_kernel(
     const float *__restrict__ A, int lda, const float *__restrict__ B, int ldb,
     const int32_t *__restrict__ offsets, int G, int E, int P, int Q, int tiles_q, int tiles,
     float *out0, float *out1, int ldo, long long slot_stride, int f, int beta) {
-  using namespace wgf;
-  extern __shared__ __attribute__((aligned(16))) float ldsw[];
-  int g, tile;
-  if (!wgrad_item(G, tiles, g, tile)) return;
+  __shared__ __attribute__((aligned(16))) float lds[T::kLdsFloats];
+  const int gi = (int)(blockIdx.x / (unsigned)tiles);
+  const int g = (gi + G - 1) % G;
+  const int id = (int)f32t::xcd_run(blockIdx.x - (unsigned)(gi * tiles), (unsigned)tiles);
   const int row_lo = offsets[g];
   const int mg = offsets[g + 1] - row_lo;
-  if (mg <= 0) return;
-  const int tp = tile / tiles_q;
-  const int i0 = tp * wg::BP, j0 = (tile - tp * tiles_q) * wg::BQ;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wp = wave >> 1, wq = wave & 1;
-  // Loads: thread t moves rows t / 32 and t / 32 + 8, columns 4 (t % 32)...
-  const int lrow = tid >> 5, lc4 = (tid & 31) * 4;
-  // Columns past P / Q read column 0 instead (their outputs are dropped).
-  const int ca = i0 + lc4 < P ? i0 + lc4 : 0;
-  const int cb = j0 + lc4 < Q ? j0 + lc4 : 0;
-  // Rows past the group's end read its last row and are replaced by zeros
-  // (a select of values: a select of pointers would read zeros from memory).
-  float4 ra0, ra1, rb0, rb1;
-#define PRICHS_WGF_SEL(v, ok) \
-  v = make_float4((ok) ? v.x : 0.f, (ok) ? v.y : 0.f, (ok) ? v.z : 0.f, (ok) ? v.w : 0.f)
-#define PRICHS_WGF_LOAD(k0)                                                         \
-  do {                                                                              \
-    const int r0_ = (k0) + lrow, r1_ = (k0) + lrow + 8;                             \
-    const size_t s0_ = (size_t)(row_lo + min(r0_, mg - 1));                         \
-    const size_t s1_ = (size_t)(row_lo + min(r1_, mg - 1));                         \
-    ra0 = *reinterpret_cast<const float4 *>(A + s0_ * lda + ca);                    \
-    rb0 = *reinterpret_cast<const float4 *>(B + s0_ * ldb + cb);                    \
-    ra1 = *reinterpret_cast<const float4 *>(A + s1_ * lda + ca);                    \
-    rb1 = *reinterpret_cast<const float4 *>(B + s1_ * ldb + cb);                    \
-    PRICHS_WGF_SEL(ra0, r0_ < mg);                                                  \
-    PRICHS_WGF_SEL(rb0, r0_ < mg);                                                  \
-    PRICHS_WGF_SEL(ra1, r1_ < mg);                                                  \
-    PRICHS_WGF_SEL(rb1, r1_ < mg);                                                  \
-  } while (0)
-#define PRICHS_WGF_STORE(buf)                                             \
-  do {                                                                    \
-    float *as_ = ldsw + (buf) * 2 * kTile;                                \
-    float *bs_ = as_ + kTile;                                             \
-    *reinterpret_cast<float4 *>(as_ + lrow * kLd + lc4) = ra0;            \
-    *reinterpret_cast<float4 *>(bs_ + lrow * kLd + lc4) = rb0;            \
-    *reinterpret_cast<float4 *>(as_ + (lrow + 8) * kLd + lc4) = ra1;      \
-    *reinterpret_cast<float4 *>(bs_ + (lrow + 8) * kLd + lc4) = rb1;      \
-  } while (0)
-  f32x4 acc[4][4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int KT = (mg + BK - 1) / BK;
-  PRICHS_WGF_LOAD(0);
-  PRICHS_WGF_STORE(0);
-  __syncthreads();
-  for (int kt = 0; kt < KT; ++kt) {
-    const bool more = kt + 1 < KT;
-    if (more) PRICHS_WGF_LOAD((kt + 1) * BK);
-    const float *as = ldsw + (kt & 1) * 2 * kTile;
-    const float *bs = as + kTile;
-#pragma unroll
-    for (int ks = 0; ks < BK / 4; ++ks) {
-      const int row = ks * 4 + (lane >> 4);
-      float av[4], bv[4];
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        av[b] = as[row * kLd + wp * 64 + b * 16 + (lane & 15)];
-        bv[b] = bs[row * kLd + wq * 64 + b * 16 + (lane & 15)];
-      }
-#pragma unroll
-      for (int jb = 0; jb < 4; ++jb)
-#pragma unroll
-        for (int ib = 0; ib < 4; ++ib)
-          acc[jb][ib] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[jb], av[ib], acc[jb][ib], 0, 0, 0);
-    }
-    if (more) PRICHS_WGF_STORE((kt + 1) & 1);
-    __syncthreads();
-  }
-#undef PRICHS_WGF_LOAD
-#undef PRICHS_WGF_SEL
-#undef PRICHS_WGF_STORE
+  if (mg <= 0 && beta != 0) return;
+  const int tp = id / tiles_q;
+  const int i0 = tp * T::BM, j0 = (id - tp * tiles_q) * T::BN;
+  const int t = threadIdx.x;
+  T tile(t);
+  typename T::OpA oa;
+  typename T::OpB ob;
+  oa.init_rm(A + (long long)row_lo * lda + i0, lda, P - i0, t);
+  ob.init_rm(B + (long long)row_lo * ldb + j0, ldb, Q - j0, t);
+  if (!tile.run(lds, oa, ob, mg > 0 ? mg : 0, (long long)T::BK * lda, (long long)T::BK * ldb, t))
+    return;
   const long long base = (long long)slot_of(g, E) * slot_stride;
 #pragma unroll
-  for (int jb = 0; jb < 4; ++jb)
+  for (int ib = 0; ib < T::MI; ++ib)
 #pragma unroll
-    for (int ib = 0; ib < 4; ++ib) {
-      const int i = i0 + wp * 64 + ib * 16 + (lane & 15);
-      const int j = j0 + wq * 64 + jb * 16 + 4 * (lane >> 4);
+    for (int jb = 0; jb < T::NJ; ++jb) {
+      const int i = i0 + tile.wm * T::WM + ib * 16 + (tile.lane & 15);
+      const int j = j0 + tile.wn * T::WN + jb * 16 + 4 * (tile.lane >> 4);
       float *dst = wgrad_dst<GATEUP>(out0, out1, ldo, base, i, j, P, Q, f);
-      if (dst) {
-        float4 v = make_float4(acc[jb][ib][0], acc[jb][ib][1], acc[jb][ib][2], acc[jb][ib][3]);
-        if (beta != 0) {
-          const float4 o = *reinterpret_cast<const float4 *>(dst);
-          v.x = o.x + v.x;
-          v.y = o.y + v.y;
-          v.z = o.z + v.z;
-          v.w = o.w + v.w;
-        }
-        *reinterpret_cast<float4 *>(dst) = v;
-      }
+      if (!dst) continue;
+      f32x4 v = tile.acc[ib][jb];
+      if (beta != 0) v = *reinterpret_cast<const f32x4 *>(dst) + v;
+      *reinterpret_cast<f32x4 *>(dst) = v;
     }
+}
+
+// Tile shapes, and nanoseconds per row of one tile on a CU: alone, and each of
+// several on it (as measured for the general A^T B product).  The launch takes
+// at least the longest group (T rows: the shared expert) alone and at least
+// every group's rows spread over the CUs: at T = 2048, 512 x 512 and 512 x
+// 1024 gradients, 212.6 and 232.7 us as 128 x 128 tiles with one LDS stage of
+// 16 rows in flight, 40 and 70 us in the shapes chosen here (32 x 64, 64 x 64).
+struct WgradTileCost {
+  int bp, bq;
+  double alone, shared;
+};
+constexpr WgradTileCost kWgradF32Cost[3] = {
+    {128, 128, 64.0, 64.0}, {64, 64, 20.0, 17.2}, {32, 64, 13.3, 9.9}};
+typedef f32t::Tile<128, 128, 32, 2, 2, 1, false, false> WgradLarge;
+typedef f32t::Tile<64, 64, 32, 2, 2, 1, false, false> WgradMedium;
+typedef f32t::Tile<32, 64, 64, 1, 2, 2, false, false> WgradSmall;
+
+int wgrad_f32_choice(size_t total_rows, size_t max_group_rows, size_t P, size_t Q, int cus) {
+  int best = 0;
+  double best_t = 0;
+  for (int c = 0; c < 3; ++c) {
+    const WgradTileCost &k = kWgradF32Cost[c];
+    const double tiles = (double)(cdiv(P, k.bp) * cdiv(Q, k.bq));
+    const double t = std::max(k.alone * (double)max_group_rows,
+                              k.shared * (double)total_rows * tiles / cus);
+    if (c == 0 || t < best_t) best = c, best_t = t;
+  }
+  return best;
+}
+
+template <class T>
+int launch_wgrad_f32(bool gateup, const float *A, int lda, const float *B, int ldb,
+                     const int32_t *offsets, int G, int E, int P, int Q, float *out0, float *out1,
+                     int ldo, long long slot_stride, int f, int beta, hipStream_t s) {
+  const size_t tiles_q = cdiv((size_t)Q, T::BN), tiles = cdiv((size_t)P, T::BM) * tiles_q;
+  if (tiles * (size_t)G > (size_t)INT32_MAX)
+    return fail(PRICHS_ERR_UNSUPPORTED, "moe backward: too many tiles");
+  auto kern = gateup ? wgrad_f32_kernel<T, true> : wgrad_f32_kernel<T, false>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * G)), dim3(T::kThreads), 0, s, A, lda, B, ldb,
+                     offsets, G, E, P, Q, (int)tiles_q, (int)tiles, out0, out1, ldo, slot_stride,
+                     f, beta);
+  PRICHS_LAUNCH_CHECK("moe backward: weight gradient");
+  return PRICHS_OK;
 }
 
 // ------------------------------------------------------------- combine --
@@ -1266,7 +1214,7 @@ size_t bwd_wgrad_part_elems(size_t max_rows, size_t P, size_t Q) {
 }
 
 int bwd_wgrad(bool gateup, const void *A, size_t lda, const void *B, size_t ldb, size_t total_rows,
-              const int32_t *offsets, size_t G, size_t E, size_t P, size_t Q, float *out0,
+              size_t max_group_rows, const int32_t *offsets, size_t G, size_t E, size_t P, size_t Q, float *out0,
               float *out1, size_t ldo, size_t slot_stride, size_t f, int dtype, float *part,
               int beta, hipStream_t s, const WgradAlt &alt) {
   if (total_rows == 0) return PRICHS_OK;
@@ -1313,29 +1261,20 @@ int bwd_wgrad(bool gateup, const void *A, size_t lda, const void *B, size_t ldb,
     if (total_rows > (size_t)wgb::kSplitRows || beta == 0) {
       auto rk = gateup ? wgrad_reduce_kernel<true> : wgrad_reduce_kernel<false>;
       hipLaunchKernelGGL(rk, dim3(rgrid), dim3(256), 0, s, part, offsets, (int)G, (int)E, (int)P,
-                         (int)Q, out0, out1, (int)ldo, (long long)slot_stride, (int)f, beta, 1);
+                         (int)Q, out0, out1, (int)ldo, (long long)slot_stride, (int)f, beta);
       PRICHS_LAUNCH_CHECK("moe backward: weight gradient partials");
     }
     return PRICHS_OK;
   }
   if (alt.A || alt.B)
     return fail(PRICHS_ERR_UNSUPPORTED, "moe backward: alternate row buffers need bf16");
-  const int tiles_q = (int)cdiv(Q, wg::BQ);
-  const int tiles = (int)cdiv(P, wg::BP) * tiles_q;
-  const unsigned grid = (unsigned)(8 * cdiv((size_t)tiles, 8) * G);
-  auto kern = gateup ? wgrad_f32_kernel<true> : wgrad_f32_kernel<false>;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(wg::kThreads), wgf::kLdsBytes, s,
-                     static_cast<const float *>(A), (int)lda, static_cast<const float *>(B),
-                     (int)ldb, offsets, (int)G, (int)E, (int)P, (int)Q, tiles_q, tiles, out0,
-                     out1, (int)ldo, (long long)slot_stride, (int)f, beta);
-  PRICHS_LAUNCH_CHECK("moe backward: weight gradient");
-  if (beta == 0) {  // zeros for groups without rows
-    auto rk = gateup ? wgrad_reduce_kernel<true> : wgrad_reduce_kernel<false>;
-    hipLaunchKernelGGL(rk, dim3(rgrid), dim3(256), 0, s, nullptr, offsets, (int)G, (int)E, (int)P,
-                       (int)Q, out0, out1, (int)ldo, (long long)slot_stride, (int)f, 0, 0);
-    PRICHS_LAUNCH_CHECK("moe backward: weight gradient zeros");
-  }
-  return PRICHS_OK;
+  const int shape = wgrad_f32_choice(total_rows, max_group_rows, P, Q, cus);
+  auto run = shape == 0 ? &launch_wgrad_f32<WgradLarge>
+                        : shape == 1 ? &launch_wgrad_f32<WgradMedium>
+                                     : &launch_wgrad_f32<WgradSmall>;
+  return run(gateup, static_cast<const float *>(A), (int)lda, static_cast<const float *>(B),
+             (int)ldb, offsets, (int)G, (int)E, (int)P, (int)Q, out0, out1, (int)ldo,
+             (long long)slot_stride, (int)f, beta, s);
 }
 
 int bwd_combine(const void *dX, const float *scal, const int32_t *topk_idx, const float *topk_w,

@@ -675,7 +675,7 @@ extern "C" int prichs_moe_engine_backward(prichs_moe_engine *eng, const void *x,
                 eng->xg, eng->scal, s);
   if (rc) return rc;
   PRICHS_BWD_MARK(2);
-  rc = bwd_wgrad(false, eng->act, f, eng->dy, d, rows, eng->offsets, G, E, f, d, grads->d_down,
+  rc = bwd_wgrad(false, eng->act, f, eng->dy, d, rows, T, eng->offsets, G, E, f, d, grads->d_down,
                  nullptr, d, grads->slot_stride, f, dt, eng->wpart, grads->beta, s, alt_dy);
   if (rc) return rc;
   PRICHS_BWD_MARK(3);
@@ -712,7 +712,7 @@ extern "C" int prichs_moe_engine_backward(prichs_moe_engine *eng, const void *x,
                    k, dx_weighting, dt, eng->dlr, d_x, d_x_dtype, s);
   if (rc) return rc;
   PRICHS_BWD_MARK(7);
-  rc = bwd_wgrad(true, eng->xg, d, eng->gu, np, rows, eng->offsets, G, E, d, np, grads->d_gate,
+  rc = bwd_wgrad(true, eng->xg, d, eng->gu, np, rows, T, eng->offsets, G, E, d, np, grads->d_gate,
                  grads->d_up, f, grads->slot_stride, f, dt, eng->wpart, grads->beta, s, alt_x);
   if (rc) return rc;
   PRICHS_BWD_MARK(8);
