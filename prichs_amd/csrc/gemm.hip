@@ -29,6 +29,7 @@
 // f32 kernel: the tiles of f32_tile.hpp on v_mfma_f32_16x16x4_f32 (the fp32-
 // checked mode; accumulates in fp32 like the reference CPU path).
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <type_traits>
 #include <cstring>
@@ -148,14 +149,6 @@ __device__ inline void tile_coords(int t, int m_tiles, int n_tiles, int &mt, int
   nt = r / rows;
 }
 
-// Workgroups are dealt round-robin to the 8 XCDs; renumbering them so each XCD
-// runs a contiguous run of the tile order keeps shared panels in its L2.
-__device__ inline int xcd_block_id() {
-  const int nblk = gridDim.x;
-  return (nblk % 8 == 0) ? (int)(blockIdx.x % 8) * (nblk / 8) + (int)(blockIdx.x / 8)
-                         : (int)blockIdx.x;
-}
-
 // ------------------------------------------------------------------------
 // bf16 kernel
 // ------------------------------------------------------------------------
@@ -243,7 +236,7 @@ template <int BM_, int BN_, int WGM_, int WGN_, int S_ = PRICHS_BF16_STAGES> str
   static constexpr int kStgStride = BN + 8;
   static constexpr size_t kStgBytes = (size_t)BM * kStgStride * sizeof(bf16_t);
   static constexpr size_t kLdsBytes = kRingBytes > kStgBytes ? kRingBytes : kStgBytes;
-  static_assert(MI % 2 == 0 && WN % 16 == 0, "two A halves and whole fragments per wave");
+  static_assert(WM % 16 == 0 && WN % 16 == 0, "whole fragments per wave");
   static_assert(kBlkA * kRowsPerInst == BM && kBlkB * kRowsPerInst == BN,
                 "the DMA instructions of one stage cover the A and B tiles exactly");
   static_assert(kInstPerStage >= 1, "every wave issues DMA in every stage");
@@ -274,6 +267,11 @@ using Bf16Wide = Bf16Cfg<128, 384, 2, 4>;
 // round of the CUs, where 256 x 256 tiles make 1.125 rounds and 128 x 384
 // tiles 1.5.
 using Bf16Tall = Bf16Cfg<256, 288, 4, 2>;
+
+// 128 x 256 tiles (and 128 x 128 halves) for launches with too few rows to
+// fill the CUs with 256 x 256 ones: a prompt's or a micro-batch's experts
+// (mid_tiles in the launch code).
+using Bf16Mid = Bf16Cfg<128, 256, 2, 4>;
 
 // C[m, n] = sum_k A[row(m), k] * B[n, k] for the rows of each group, with
 // B = packed weights [Np, K] of group g.  The MFMA takes the weight fragment
@@ -746,8 +744,8 @@ __global__ __launch_bounds__(kBf16Threads) void bf16_gemm_kernel(
     bf16_t *__restrict__ C, int ldc, int n_store, const int32_t *__restrict__ offsets,
     int G, int dense_m, int stage_c, bf16_t *__restrict__ P, A2Rows a2) {
   constexpr bool kSplit = !std::is_same<Cf, CfT>::value;
-  static_assert(!kSplit || (CfT::BM == Cf::BM && 2 * CfT::BN == Cf::BN && !GATEUP),
-                "tail tiles are the two column halves of a down / dense tile");
+  static_assert(!kSplit || (CfT::BM == Cf::BM && 2 * CfT::BN == Cf::BN),
+                "tail tiles are the two column halves of a tile");
   extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
   WaveTileMap tm;
   build_wave_tile_map(tm, offsets, G, Cf::BM, dense_m);
@@ -764,7 +762,13 @@ __global__ __launch_bounds__(kBf16Threads) void bf16_gemm_kernel(
       n_items = n_full + 2 * tail;
     }
   }
-  for (int t = xcd_block_id(); t < n_items; t += nblk) {
+  // Each XCD takes a contiguous run of every round's items.  A launch of at
+  // most one round deals its items evenly over the XCDs (333 tokens, gate/up
+  // in 128 x 256 tiles: 27.3 us, 34.6 with the last XCDs idle); a last
+  // partial round leaves them idle instead, which keeps longer runs together
+  // (8192 tokens, down: 97.6 us against 103.3 dealt evenly).
+  const int first = (int)f32t::xcd_run(blockIdx.x, min(nblk, n_items));
+  for (int t = (int)blockIdx.x < n_items ? first : n_items; t < n_items; t += nblk) {
     int mt, nt;
     if (t < n_full) {
       tile_coords(t, m_tiles, n_tiles, mt, nt);
@@ -1266,12 +1270,16 @@ int gemm_cu_limit(int cus) {
   return cap > 0 && cap < cus ? cap : cus;
 }
 
-// Half-width configuration of the last partial round (down / dense only,
-// and only where half a tile is still a whole number of B loads per wave).
+// Half-width configuration of the last partial round, where half a tile is
+// still a whole number of B loads per wave; 128-wide tiles keep 64 columns per
+// wave, one [gate | up] block.  Not for 256 x 256 gate/up tiles: their whole
+// tiles run 0.3% slower with the second path compiled in, and launches that
+// would gain mostly take 128 x 256 tiles (mid_tiles).
 template <class Cf, bool GATEUP>
 using TailCfg = typename std::conditional<
-    GATEUP || (Cf::BN / 2) % (Cf::kRowsPerInst * Cf::kWaves) != 0, Cf,
-    Bf16Cfg<Cf::BM, Cf::BN / 2, Cf::WGM, Cf::WGN, Cf::kStages>>::type;
+    (Cf::BN / 2) % (Cf::kRowsPerInst * Cf::kWaves) != 0 || (GATEUP && Cf::BM == 256), Cf,
+    Bf16Cfg<Cf::BM, Cf::BN / 2, Cf::BN == 256 ? 4 : Cf::WGM, Cf::BN == 256 ? 2 : Cf::WGN,
+            Cf::kStages>>::type;
 
 // Persistent grid of a bf16 launch: one workgroup per CU (the LDS ring allows
 // one), fewer when the launch has fewer tiles (twice the tiles when the last
@@ -1335,10 +1343,12 @@ double launch_tile_times(size_t tiles, size_t grid, bool split) {
 // 124.7 us as 1024 wide tiles, 120.2 us as 768 square ones).  A 256 x 288
 // tile is 1.125 square tiles of work at the square tile's rate per flop.
 constexpr double kWideWork = 0.75, kWideRate = 0.96, kTallWork = 1.125;
+constexpr double kMidWork = 0.64;  // of a 128 x 256 tile (mid_tiles, below)
 
 // Tile shape of a dense launch of M rows and Np packed columns: the one with
 // the fewest estimated square-tile-times on the grid launch_bf16 gives it
-// (0: 256 x 256 with half-width tails, 1: 128 x 384, 2: 256 x 288).
+// (0: 256 x 256 with half-width tails, 1: 128 x 384, 2: 256 x 288, 3: 128 x 256
+// with half-width tails).
 int dense_tile_choice(size_t M, size_t Np, int cus) {
   const size_t sq = ((M + Bf16Down::BM - 1) / Bf16Down::BM) * (Np / Bf16Down::BN);
   double best = launch_tile_times(sq, bf16_grid<Bf16Down, false>(M, 1, Np, cus), true);
@@ -1355,7 +1365,52 @@ int dense_tile_choice(size_t M, size_t Np, int cus) {
         launch_tile_times(tl, bf16_grid<Bf16Tall, false>(M, 1, Np, cus), false) * kTallWork;
     if (t < best) best = t, choice = 2;
   }
+  // 128 x 256 tiles where the rows are few (below, mid_tiles).
+  const size_t mid = ((M + Bf16Mid::BM - 1) / Bf16Mid::BM) * (Np / Bf16Mid::BN);
+  const double t =
+      launch_tile_times(mid, bf16_grid<Bf16Mid, false>(M, 1, Np, cus), true) * kMidWork;
+  if (t < best) choice = 3;
   return choice;
+}
+
+// Time of a grouped launch of `tiles` tiles in tile-times of its
+// configuration: whole rounds; then a last round of half-width tiles (halves:
+// the configuration has them), or a partial one (its tiles run a little
+// faster than a full round's: fewer CUs share the clock and the caches).
+double grouped_tile_times(double tiles, double grid, bool halves) {
+  const double full = std::floor(tiles / grid), tail = tiles - full * grid;
+  if (tail < 1) return full;
+  return full + (halves && 2 * tail <= grid ? 0.62 : 0.75 + 0.25 * tail / grid);
+}
+
+// M-tiles of BM rows of a grouped launch.  The groups' row counts are on the
+// device: the engine's launches have one group of max_group_rows rows (the
+// shared expert) and the others' rows spread evenly, give or take a tenth;
+// launches without a tighter bound per group spread all rows.
+double grouped_m_tiles(size_t BM, size_t max_rows, size_t max_group_rows, int G) {
+  const bool shared = max_group_rows < max_rows && G > 1;
+  const double n = shared ? G - 1 : G;
+  const double m = (double)(max_rows - (shared ? max_group_rows : 0)) / n;
+  const double dev = std::max(std::sqrt(m), 0.1 * m);
+  double per = 0;
+  for (int i = -1; i <= 1; ++i)
+    per += std::max(m > 0 ? 1.0 : 0.0, std::ceil((m + i * dev) / (double)BM)) / 3;
+  return n * per + (shared ? (double)cdiv(max_group_rows, BM) : 0.0);
+}
+
+// Whether a grouped launch takes 128 x 256 tiles: one costs 0.64 of a 256 x
+// 256 tile (half the work; fewer products per byte staged), so they pay where
+// the large tiles leave the last or only round mostly empty.  Measured on
+// MI355X (d = 1536, f = 1280, 8 + 1 experts, top-2; 256 x 256 against 128 x
+// 256, us): gate/up 333 tokens 29.0 / 22.9, 512 33.0 / 31.3, 1500 47.9 / 53.5,
+// 3000 78.8 / 86.7, 8192 172 / 194; down 333 21.4 / 15.0, 777 22.1 / 21.2,
+// 1500 31.6 / 26.3, 3000 42.6 / 48.5, 8192 101 / 111; dX 512 48.6 / 37.2, 1000
+// 56.5 / 50.0, 2048 73.2 / 73.5, 8192 181 / 202.
+bool mid_tiles(bool gateup, size_t max_rows, size_t max_group_rows, int G, int Np, int cus) {
+  const double grid = gemm_cu_limit(cus), nt = Np / Bf16Mid::BN;
+  const double big = grouped_m_tiles(Bf16::BM, max_rows, max_group_rows, G) * nt;
+  const double mid = grouped_m_tiles(Bf16Mid::BM, max_rows, max_group_rows, G) * nt;
+  return kMidWork * grouped_tile_times(mid, grid, true) < grouped_tile_times(big, grid, !gateup);
 }
 
 template <bool GATEUP, int U, int SK>
@@ -1429,16 +1484,23 @@ int launch_grouped(bool gateup, const void *A, const int32_t *a_rows, int lda, c
   const int cus = device_cu_count();
   if (cus <= 0) return fail(PRICHS_ERR_HIP, "grouped gemm: cannot query the device");
   if (dtype == PRICHS_DTYPE_BF16) {
-    if (gateup)
-      return launch_bf16<Bf16, true>(A, a_rows, lda, B, b_stride, Np, K, Cp, ldc, n_store,
-                                     offsets, G, dense_m, max_rows, cus, s, pre);
-    const int shape = offsets == nullptr ? dense_tile_choice((size_t)dense_m, (size_t)Np, cus) : 0;
+    const bool mid = offsets != nullptr && mid_tiles(gateup, max_rows, max_group_rows, G, Np, cus);
+    if (gateup) {
+      auto run = mid ? &launch_bf16<Bf16Mid, true> : &launch_bf16<Bf16, true>;
+      return run(A, a_rows, lda, B, b_stride, Np, K, Cp, ldc, n_store, offsets, G, dense_m,
+                 max_rows, cus, s, pre, A2Rows());
+    }
+    const int shape = offsets != nullptr ? (mid ? 3 : 0)
+                                         : dense_tile_choice((size_t)dense_m, (size_t)Np, cus);
     if (shape == 1)
       return launch_bf16<Bf16Wide, false>(A, a_rows, lda, B, b_stride, Np, K, Cp, ldc, n_store,
                                           offsets, G, dense_m, max_rows, cus, s, nullptr);
     if (shape == 2)
       return launch_bf16<Bf16Tall, false>(A, a_rows, lda, B, b_stride, Np, K, Cp, ldc, n_store,
                                           offsets, G, dense_m, max_rows, cus, s, nullptr);
+    if (shape == 3)
+      return launch_bf16<Bf16Mid, false>(A, a_rows, lda, B, b_stride, Np, K, Cp, ldc, n_store,
+                                         offsets, G, dense_m, max_rows, cus, s, nullptr);
     return launch_bf16<Bf16Down, false>(A, a_rows, lda, B, b_stride, Np, K, Cp, ldc, n_store,
                                         offsets, G, dense_m, max_rows, cus, s, nullptr);
   } else {
@@ -1645,10 +1707,11 @@ int grouped_dact_swiglu_bwd(const void *dy, size_t d, const void *w_down_t, size
     alt.row0 = (int)a2_row0;
   }
   *fused = true;
-  return launch_bf16<Bf16Down, false, true>(dy, nullptr, (int)d, w_down_t,
-                                            (long long)b_group_stride, (int)np_f, (int)d, nullptr,
-                                            (int)np, (int)f, offsets, (int)G, 0, max_rows, cus,
-                                            as_stream(stream), gu, alt);
+  auto run = mid_tiles(false, max_rows, std::min(max_rows, max_group_rows), (int)G, (int)np_f, cus)
+                 ? &launch_bf16<Bf16Mid, false, true>
+                 : &launch_bf16<Bf16Down, false, true>;
+  return run(dy, nullptr, (int)d, w_down_t, (long long)b_group_stride, (int)np_f, (int)d, nullptr,
+             (int)np, (int)f, offsets, (int)G, 0, max_rows, cus, as_stream(stream), gu, alt);
 }
 }  // namespace prichs
 

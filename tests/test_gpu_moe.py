@@ -204,6 +204,47 @@ def test_gate_up_unaligned_output_bit_identical(cuda):
     assert int(flat[:4].view(torch.int16).abs().sum()) == 0  # nothing written before it
 
 
+# Launches with few rows take 128 x 256 tiles (whole ones, or all as 128 x 128
+# halves where those fill at most half the CUs): ragged, empty, one-row and
+# exactly full groups.  The extra group of the second launch makes the same
+# rows take 256 x 256 tiles; every output element is one MFMA chain over K, so
+# the shared rows agree bit for bit.
+@pytest.mark.parametrize("d,f,counts", [(1536, 1280, [83, 0, 129, 300, 1]),      # halves
+                                        (1536, 1280, [256, 128, 700, 384, 513]),  # whole
+                                        (320, 192, [65, 255, 1000])])
+@pytest.mark.parametrize("aligned", [True, False])
+def test_mid_tiles_bit_identical(cuda, orc, d, f, counts, aligned):
+    rng = np.random.default_rng(d + f + len(counts))
+    G, rows, extra, Tx = len(counts), sum(counts), 9000, 400
+    x = dev(synth.round_bf16(rng.standard_normal((Tx, d))), "bf16")
+    w = [synth.round_bf16(0.03 * rng.standard_normal((d, f))) for _ in range(3)]
+    gu = ops.to_device_packed([ops.pack_gate_up(w[g % 2], w[(g + 1) % 3], "bf16")
+                               for g in range(G + 1)], "bf16")
+    dn = ops.to_device_packed([ops.pack_down(np.ascontiguousarray(w[g % 3].T), "bf16")
+                               for g in range(G + 1)], "bf16")
+    row_token = torch.from_numpy(rng.integers(0, Tx, rows + extra).astype(np.int32)).to("cuda")
+    off = torch.from_numpy(np.concatenate([[0], np.cumsum(counts), [rows + extra]])
+                           .astype(np.int32)).to("cuda")
+    say("mid tiles", d, f, counts, aligned)
+    got = []
+    for n, r in ((G, rows), (G + 1, rows + extra)):
+        buf = torch.full((r * f + 16,), 7.0, dtype=torch.bfloat16, device="cuda")
+        by = 0 if aligned else 4  # 8 bytes past a 16-byte boundary: direct stores
+        act = buf[by:by + r * f].view(r, f)
+        ops.grouped_gate_up_swiglu(x, row_token[:r], off[:n + 1], n, r, gu, d, f, out=act)
+        assert (buf[:by] == 7).all() and (buf[by + r * f:] == 7).all()
+        got.append((act[:rows], ops.grouped_down(act.contiguous(), off[:n + 1], n, r, dn, d, f)[:rows]))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    h_act, h_y = host(got[0][0]), host(got[0][1])
+    o = np.concatenate([[0], np.cumsum(counts)])
+    for g in (2, G - 1):  # against the oracle: two groups
+        r = slice(o[g], o[g + 1])
+        xr = host(x[row_token[r].long()])
+        a_ref = orc.swiglu(orc.matmul_2d(xr, w[g % 2]), orc.matmul_2d(xr, w[(g + 1) % 3]))
+        assert rel_err(h_act[r], a_ref) <= 2e-2, ("act", g)
+        assert rel_err(h_y[r], orc.matmul_2d(h_act[r], w[g % 3].T)) <= 2e-2, ("y", g)
+
+
 # The f32 grouped GEMMs' tile shapes (gate/up | down): 128 x 128 | 32 x 64,
 # 32 x 64 | 128 x 128, 64 x 64 | 32 x 64, and 32 x 64 twice with empty groups
 # and one-row groups; rows and columns ending inside tiles, K inside a step.
