@@ -137,27 +137,25 @@ int grouped_down_rows(const void *act, const int32_t *offsets, size_t G, size_t 
                       size_t max_group_rows, const void *w_packed, size_t d, size_t f, int dtype,
                       void *y, void *stream);
 
-// Decode path (gemm.hip).  When one router workgroup covers the batch, every
-// expert's weights are streamed whatever the routing, so one launch runs the
-// router (which also writes the permutation) in its first workgroup while the
-// others run the gate/up GEMM densely over all T tokens of every group:
-// act_dense [(E + 1) T][f], group g's rows g T .. g T + T - 1 (routed experts,
-// then the shared expert).  The router also writes dense_row [T k + T], the
-// dense row of every row-space row.  decode_down then runs the down GEMM over
-// the row space only, its A rows gathered as act_dense[dense_row[r]], and
-// copies those rows to act (the row-space activations) as it stages them.
-// Every row's values are bit-identical to the routed path's.
+// Decode path (gemm.hip), at most 32 tokens: every expert's weights are
+// streamed whatever the routing, so one launch runs the chain router in its
+// first workgroups (8 tokens each) while the others run the gate/up GEMM
+// densely over all T tokens of every group: act_dense [(E + 1) T][f], group
+// g's rows g T .. g T + T - 1 (routed experts, then the shared expert).
+// decode_down then runs the down GEMM over the row space: each workgroup finds
+// its group's rows from the selections, reads their dense rows and copies
+// them to act (the row-space activations); the permutation is written there
+// too.  Every row's values are bit-identical to the routed path's.
 bool decode_dense_applies(size_t T, size_t d, size_t f, size_t E, size_t k, size_t n_shared,
-                          int dtype, const void *x, const float *w_router);
+                          int dtype, const void *x, const float *w_lds);
 int decode_gate_up_router(const void *x, size_t T, size_t d, size_t f, size_t E, size_t k,
-                          const float *w_router, const float *w_lds, const float *router_bias,
+                          const float *w_lds, const float *router_bias,
                           const float *concept_bias, size_t n_concept, float *logits,
                           int32_t *topk_idx, float *topk_w, int32_t *block_counts,
-                          int32_t *offsets, int32_t *row_token, float *row_weight,
-                          int32_t *token_row, int32_t *dense_row, const void *w_gate_up,
-                          void *act_dense, void *stream);
-int decode_down(const void *act_dense, const int32_t *dense_row, const int32_t *offsets, size_t T,
-                size_t d, size_t f, size_t E, size_t k, const void *w_down, void *y, void *act,
+                          const void *w_gate_up, void *act_dense, void *stream);
+int decode_down(const void *act_dense, const int32_t *topk_idx, const float *topk_w, size_t T,
+                size_t d, size_t f, size_t E, size_t k, const void *w_down, int32_t *offsets,
+                int32_t *row_token, float *row_weight, int32_t *token_row, void *y, void *act,
                 void *stream);
 
 // Plain grouped GEMM over the engine's row space (no SwiGLU):
@@ -253,6 +251,22 @@ int router_topk_lds(const void *x, int x_dtype, const float *w_router, const flo
                     const float *router_bias, const float *concept_bias, size_t n_concept,
                     size_t T, size_t d, size_t E, size_t k, float *logits, int32_t *topk_idx,
                     float *topk_w, int32_t *block_counts, void *stream);
+// Router and permutation of a batch of at most kRouterChainMaxTokens tokens on
+// the chain router (router_quad.hpp), with the W^T copy above; block_counts
+// holds ceil(T / 8) * E int32.  Bit-identical to router_topk_permute.
+// routed_event (may be null) is recorded between the two launches.  2048: one
+// workgroup per CU.  MI355X, d = 1536, stage events, quad -> chain router us:
+// 333 tokens 17.0 -> 12.6, 2048 17.4 -> 13.2, 4096 17.6 -> 18.1 (two adding
+// waves and their products per CU), 8192 18.7 -> 27.4.
+constexpr size_t kRouterChainMaxTokens = 2048;
+bool router_chain_applies(size_t T, size_t d, size_t E, const void *x, const float *w_lds);
+int router_topk_permute_chain(const void *x, int x_dtype, const float *w_lds,
+                              const float *router_bias, const float *concept_bias,
+                              size_t n_concept, size_t T, size_t d, size_t E, size_t k,
+                              float *logits, int32_t *topk_idx, float *topk_w,
+                              int32_t *block_counts, int32_t *offsets, int32_t *row_token,
+                              float *row_weight, int32_t *token_row, void *stream,
+                              void *routed_event);
 // Elements of that copy (0 when the router kernel that reads it does not
 // apply to the shape), and the copy of host weights W [d][E] into host memory.
 size_t router_lds_layout_elems(size_t d, size_t E);

@@ -48,10 +48,9 @@ struct prichs_moe_engine {
   void *act = nullptr;
   void *y = nullptr;
   // Decode path (decode_gate_up_router / decode_down): the dense gate/up
-  // activations [(E + 1) dense_tokens][f] and the dense row of every row.
+  // activations [(E + 1) dense_tokens][f].
   size_t dense_tokens = 0;
   void *act_dense = nullptr;
-  int32_t *dense_row = nullptr;
   size_t gu_elems = 0, dn_elems = 0;  // packed elements per expert
   size_t last_T = 0;
   bool stash_valid = false;  // a forward's intermediates await a backward
@@ -142,7 +141,9 @@ extern "C" int prichs_moe_engine_create(size_t d, size_t f, size_t E, size_t k, 
   const size_t G = E + n_shared;
   const size_t Tm = max_tokens;
   const size_t rows = Tm * k + n_shared * Tm;
-  const size_t nb = prichs_router_num_blocks(Tm, E);
+  // Router workgroups: of prichs_router_topk, and of the chain router.
+  const size_t nb = std::max(prichs_router_num_blocks(Tm, E),
+                             cdiv(std::min(Tm, kRouterChainMaxTokens), 8));
 
   prichs_moe_engine *eng = new (std::nothrow) prichs_moe_engine();
   if (!eng) return fail(PRICHS_ERR_CAPACITY, "engine_create: out of host memory");
@@ -176,7 +177,6 @@ extern "C" int prichs_moe_engine_create(size_t d, size_t f, size_t E, size_t k, 
   // Decode buffers for batches one router workgroup covers (32 tokens).
   const size_t Td = (dtype == PRICHS_DTYPE_BF16 && n_shared == 1) ? std::min<size_t>(Tm, 32) : 0;
   const size_t o_actd = c.take(es * (E + 1) * Td * f + 1);
-  const size_t o_drow = c.take(sizeof(int32_t) * (Td * k + Td) + 1);
 
   int rc = PRICHS_OK;
   if (hipGetDevice(&eng->device) != hipSuccess) {
@@ -210,7 +210,6 @@ extern "C" int prichs_moe_engine_create(size_t d, size_t f, size_t E, size_t k, 
   eng->act = base + o_act;
   eng->dense_tokens = Td;
   eng->act_dense = Td > 0 ? base + o_actd : nullptr;
-  eng->dense_row = Td > 0 ? reinterpret_cast<int32_t *>(base + o_drow) : nullptr;
   eng->y = base + o_y;
   *out = eng;
   return PRICHS_OK;
@@ -429,26 +428,34 @@ static int moe_forward_impl(prichs_moe_engine *eng, const void *x, size_t T,
   if (tm) PRICHS_HIP_TRY(hipEventRecord(ev[0], s), "engine_forward: event");
   if (!eng->bwd && T <= eng->dense_tokens &&
       decode_dense_applies(T, eng->d, eng->f, eng->E, eng->k, eng->S, eng->dtype, x,
-                           eng->w_router)) {
-    // Decode: the router (and the permutation) runs in the first workgroup
-    // of the gate/up launch, which covers every token of every expert; the
-    // down GEMM gathers the routed rows.  Events [0]-[2] bracket no work.
+                           eng->w_router_lds)) {
+    // Decode: the router runs in the first workgroups of the gate/up launch,
+    // which covers every token of every expert; the down GEMM finds the
+    // routed rows and writes the permutation.  Events [0]-[2] bracket no work.
     if (tm) PRICHS_HIP_TRY(hipEventRecord(ev[1], s), "engine_forward: event");
     if (tm) PRICHS_HIP_TRY(hipEventRecord(ev[2], s), "engine_forward: event");
-    rc = decode_gate_up_router(x, T, eng->d, eng->f, eng->E, eng->k, eng->w_router,
-                               eng->w_router_lds, eng->router_bias, concept_bias, n_concept,
-                               eng->logits, eng->topk_idx, eng->topk_w, eng->block_counts,
-                               eng->offsets, eng->row_token, eng->row_weight, eng->token_row,
-                               eng->dense_row, eng->w_gate_up, eng->act_dense, stream);
+    rc = decode_gate_up_router(x, T, eng->d, eng->f, eng->E, eng->k, eng->w_router_lds,
+                               eng->router_bias, concept_bias, n_concept, eng->logits,
+                               eng->topk_idx, eng->topk_w, eng->block_counts, eng->w_gate_up,
+                               eng->act_dense, stream);
     if (rc) return rc;
     if (tm) PRICHS_HIP_TRY(hipEventRecord(ev[3], s), "engine_forward: event");
-    rc = decode_down(eng->act_dense, eng->dense_row, eng->offsets, T, eng->d, eng->f, eng->E,
-                     eng->k, eng->w_down, eng->y, eng->act, stream);
+    rc = decode_down(eng->act_dense, eng->topk_idx, eng->topk_w, T, eng->d, eng->f, eng->E,
+                     eng->k, eng->w_down, eng->offsets, eng->row_token, eng->row_weight,
+                     eng->token_row, eng->y, eng->act, stream);
     if (rc) return rc;
     if (tm) PRICHS_HIP_TRY(hipEventRecord(ev[4], s), "engine_forward: event");
     return moe_finish(eng, T, out, out_dtype, stream, residual, moe_out, tm, ev);
   }
-  if (prichs_router_num_blocks(T, eng->E) == 1) {
+  if (router_chain_applies(T, eng->d, eng->E, x, eng->w_router_lds) &&
+      (T <= 8 || prichs_router_num_blocks(T, eng->E) > 1)) {
+    rc = router_topk_permute_chain(x, eng->dtype, eng->w_router_lds, eng->router_bias,
+                                   concept_bias, n_concept, T, eng->d, eng->E, eng->k,
+                                   eng->logits, eng->topk_idx, eng->topk_w, eng->block_counts,
+                                   eng->offsets, eng->row_token, eng->row_weight, eng->token_row,
+                                   stream, tm ? ev[1] : nullptr);
+    if (rc) return rc;
+  } else if (prichs_router_num_blocks(T, eng->E) == 1) {
     // Decode-sized batch: the router's one workgroup also writes the
     // permutation (the permute stage then times as zero).
     rc = router_topk_permute(x, eng->dtype, eng->w_router, eng->router_bias, concept_bias,

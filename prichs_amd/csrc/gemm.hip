@@ -968,6 +968,18 @@ __device__ inline void load_w(const bf16_t *__restrict__ wp, int s0, bf16x8 (&w)
 // row r of the row space is A[a_rows[r]] when a_rows is set.  a_copy (may be
 // null): the workgroups of N-slab 0 also write the A rows they stage to
 // a_copy [row][lda] at their row-space rows.
+// SELF (the decode path's down GEMM): each workgroup finds its group's rows
+// itself from the selections (perm), A being the dense [group][token]
+// activations; the workgroups of N-slab 0 also write the permutation.
+struct SelfPerm {
+  const int32_t *topk_idx;
+  const float *topk_w;
+  int T, E, k;  // T * k <= 64 * kSelfWindows
+  int32_t *offsets, *row_token;
+  float *row_weight;
+  int32_t *token_row;
+};
+constexpr int kSelfWindows = PRICHS_MAX_TOPK * BM / 64;
 struct SkinnyArgs {
   const bf16_t *A;
   const int32_t *a_rows;
@@ -982,10 +994,59 @@ struct SkinnyArgs {
   bf16_t *P;
   int ldp;
   bf16_t *a_copy;
+  SelfPerm perm;
 };
 
+// Group g's first row and row count from the selections, and the tokens of
+// its rows (tok_s, visible after the caller's barrier): rows are ordered by
+// (expert, token) and the shared expert's (g = E) follow, as prichs_permute
+// orders them.  At most kSelfWindows waves of (token, slot) entries, counted
+// by ballots; every wave computes the same.  write: the workgroup also writes
+// the group's part of the permutation.
+__device__ __forceinline__ void self_permute(const SelfPerm &p, int g, bool write, int *tok_s,
+                                             int &off, int &cnt) {
+  const int lane = threadIdx.x & 63, n = p.T * p.k;
+  const bool w0 = threadIdx.x < 64;
+  off = cnt = 0;
+  int e[kSelfWindows];
+#pragma unroll
+  for (int i = 0; i < kSelfWindows; ++i)
+    e[i] = 64 * i + lane < n ? p.topk_idx[64 * i + lane] : p.E;  // past the end: no routed group
+#pragma unroll
+  for (int i = 0; i < kSelfWindows; ++i)
+    if (64 * i < n) off += __popcll(__ballot(e[i] < g));
+  if (g == p.E) {
+    off = n;
+    cnt = p.T;
+    if (w0 && lane < p.T) {
+      tok_s[lane] = lane;
+      if (write) p.row_token[n + lane] = lane;
+    }
+    if (write && threadIdx.x == 0) p.offsets[p.E + 1] = n + p.T;
+  } else {
+#pragma unroll
+    for (int i = 0; i < kSelfWindows; ++i) {
+      if (64 * i >= n) continue;
+      const bool mine = e[i] == g;
+      const uint64_t m = __ballot(mine);
+      const int r = cnt + __popcll(m & (lane == 0 ? 0ull : ~0ull >> (64 - lane)));
+      cnt += __popcll(m);
+      if (w0 && mine) {
+        const int ts = 64 * i + lane, t = ts / p.k;
+        tok_s[r] = t;
+        if (write) {
+          p.row_token[off + r] = t;
+          p.row_weight[off + r] = p.topk_w[ts];
+          p.token_row[ts] = off + r;
+        }
+      }
+    }
+  }
+  if (write && threadIdx.x == 0) p.offsets[g] = off;
+}
+
 // The workgroup (N-slab bx, group g, M-tile bz) of a skinny launch.
-template <bool GATEUP, int U, int SK>
+template <bool GATEUP, int U, int SK, bool SELF = false>
 __device__ __forceinline__ void skinny_body(const SkinnyArgs &sa, int bx, int g, int bz) {
   const bf16_t *__restrict__ A = sa.A;
   const int32_t *__restrict__ a_rows = sa.a_rows;
@@ -1001,9 +1062,17 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs &sa, int bx, int g,
   __shared__ __attribute__((aligned(16))) bf16_t a_s[SK][2][BM * kRow];
   __shared__ f32x4 red_s[SK > 1 ? SK - 1 : 1][4][2][64];  // [slice-1][N-wave][tile][lane]
   __shared__ f32x4 gate_s[2][2][64];                      // [gate wave][tile][lane]
+  __shared__ int tok_s[SELF ? BM : 1];
   const bool dense = sa.dense_T > 0;
-  const int g0 = dense ? g * sa.dense_T : sa.offsets[g];
-  const int r1 = dense ? g0 + sa.dense_T : sa.offsets[g + 1];
+  int g0, r1;
+  if constexpr (SELF) {
+    self_permute(sa.perm, g, bx == 0, tok_s, g0, r1);
+    r1 += g0;
+    __syncthreads();
+  } else {
+    g0 = dense ? g * sa.dense_T : sa.offsets[g];
+    r1 = dense ? g0 + sa.dense_T : sa.offsets[g + 1];
+  }
   const int m0 = g0 + bz * BM;
   if (m0 >= r1) return;  // uniform: this M-tile of the group is empty
   const int mrows = min(BM, r1 - m0);
@@ -1029,7 +1098,9 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs &sa, int bx, int g,
     const int i = st + kThreads * j;
     const int r = i / (4 * U), sc = i % (4 * U);
     int src = min(m0 + r, r1 - 1);
-    if (a_rows != nullptr)
+    if constexpr (SELF)
+      src = g * sa.perm.T + tok_s[src - g0];
+    else if (a_rows != nullptr)
       src = a_rows[src];
     else if (dense)
       src -= g0;
@@ -1155,42 +1226,41 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs &sa, int bx, int g,
     }
   }
 }
-template <bool GATEUP, int U, int SK>
+template <bool GATEUP, int U, int SK, bool SELF = false>
 __global__ __launch_bounds__(kThreads * SK) void skinny_gemm_kernel(SkinnyArgs sa) {
-  skinny_body<GATEUP, U, SK>(sa, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z);
+  skinny_body<GATEUP, U, SK, SELF>(sa, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z);
 }
 
-// The router workgroup's arguments in the decode launch (router_quad_body).
+// The router workgroups' arguments in the decode launch (router_chain_body).
 struct RouterArgs {
   const bf16_t *x;
-  const float *w, *bias, *concept;
+  const float *w_lds, *bias, *concept;
   int n_concept, T, d, E, k;
   float *logits;
   int32_t *topk_idx;
   float *topk_w;
   int32_t *block_counts;
-  rq::FusedPerm perm;
-  const float *w_lds;
 };
 
-// Decode launch: workgroup 0 routes the batch (one router workgroup covers
-// it) and writes its permutation; workgroups 1.. are the dense gate/up GEMM
-// (N-slab, group, M-tile) = the workgroups of skinny_gemm_kernel<true, U, 1>
-// over nx x ny x .. blocks, dispatched after the router's so it starts first.
+// Decode launch: workgroups 0 .. routers - 1 route 8 tokens each; the others
+// are the dense gate/up GEMM (N-slab, group, M-tile) = the workgroups of
+// skinny_gemm_kernel<true, U, 1> over nx x ny x .. blocks, dispatched after
+// the routers', which therefore start first.
 template <int U>
 __global__ __launch_bounds__(kThreads) void decode_gate_up_router_kernel(SkinnyArgs sa,
-                                                                        RouterArgs ra, int nx,
-                                                                        int ny) {
+                                                                        RouterArgs ra, int routers,
+                                                                        int nx, int ny) {
   static_assert(kThreads == rq::kRouterThreads, "one workgroup size for both roles");
-  extern __shared__ __attribute__((aligned(16))) float router_wt_s[];  // W^T [8][d + 4]
+  extern __shared__ __attribute__((aligned(16))) float router_s[];  // the chain router's products
   const int b = (int)blockIdx.x;
-  if (b == 0) {
-    rq::router_quad_body<bf16_t>(ra.x, ra.w, ra.bias, ra.concept, ra.n_concept, ra.T, ra.d, ra.E,
-                                 ra.k, ra.logits, ra.topk_idx, ra.topk_w, ra.block_counts,
-                                 ra.perm, ra.w_lds, 0, router_wt_s);
+  if (b < routers) {
+    rq::router_chain_body<bf16_t>(ra.x, ra.w_lds, ra.bias, ra.concept, ra.n_concept, ra.T, ra.d,
+                                  ra.E, ra.k, ra.logits, ra.topk_idx, ra.topk_w, ra.block_counts,
+                                  rq::FusedPerm{nullptr, nullptr, nullptr, nullptr}, b,
+                                  reinterpret_cast<rq::f32x4 *>(router_s));
     return;
   }
-  const int i = b - 1;
+  const int i = b - routers;
   skinny_body<true, U, 1>(sa, i % nx, (i / nx) % ny, i / (nx * ny));
 }
 }  // namespace skinny
@@ -1416,13 +1486,13 @@ bool mid_tiles(bool gateup, size_t max_rows, size_t max_group_rows, int G, int N
 template <bool GATEUP, int U, int SK>
 int launch_skinny_u(const void *A, const int32_t *a_rows, int lda, const void *B,
                     long long b_stride, int Np, int K, void *Cp, int ldc, int n_store,
-                    const int32_t *offsets, int G, int mtiles, hipStream_t s, void *pre,
-                    void *a_copy = nullptr) {
+                    const int32_t *offsets, int G, int mtiles, hipStream_t s, void *pre) {
   static_assert(Bf16::kIl == skinny::BN / 2, "a skinny slab is one [gate | up] block");
   const skinny::SkinnyArgs sa{static_cast<const bf16_t *>(A), a_rows, lda,
                               static_cast<const bf16_t *>(B), b_stride, K,
                               static_cast<bf16_t *>(Cp), ldc, n_store, offsets, 0,
-                              static_cast<bf16_t *>(pre), Np, static_cast<bf16_t *>(a_copy)};
+                              static_cast<bf16_t *>(pre), Np, nullptr,
+                              skinny::SelfPerm()};
   hipLaunchKernelGGL((skinny::skinny_gemm_kernel<GATEUP, U, SK>),
                      dim3(Np / skinny::BN, G, mtiles), dim3(skinny::kThreads * SK), 0, s, sa);
   PRICHS_LAUNCH_CHECK("skinny grouped gemm launch");
@@ -1444,7 +1514,7 @@ int launch_skinny_u(const void *A, const int32_t *a_rows, int lda, const void *B
 template <bool GATEUP>
 int launch_skinny(const void *A, const int32_t *a_rows, int lda, const void *B, long long b_stride,
                   int Np, int K, void *Cp, int ldc, int n_store, const int32_t *offsets, int G,
-                  size_t max_group_rows, hipStream_t s, void *pre, void *a_copy = nullptr) {
+                  size_t max_group_rows, hipStream_t s, void *pre) {
   const int mtiles = (int)std::max<size_t>(1, (max_group_rows + skinny::BM - 1) / skinny::BM);
   int sk = PRICHS_SKINNY_SK;
   while (sk > 1 && K % (sk * 64) != 0) sk /= 2;
@@ -1454,7 +1524,7 @@ int launch_skinny(const void *A, const int32_t *a_rows, int lda, const void *B, 
 #define PRICHS_SKINNY(U_, SK_)                                                                   \
   if (u == U_ && sk == SK_)                                                                     \
   return launch_skinny_u<GATEUP, U_, SK_>(A, a_rows, lda, B, b_stride, Np, K, Cp, ldc, n_store, \
-                                          offsets, G, mtiles, s, pre, a_copy)
+                                          offsets, G, mtiles, s, pre)
   PRICHS_SKINNY(2, 1);
   PRICHS_SKINNY(4, 1);
   PRICHS_SKINNY(8, 1);
@@ -1583,27 +1653,22 @@ int grouped_down_rows(const void *act, const int32_t *offsets, size_t G, size_t 
                         as_stream(stream), std::min(max_rows, max_group_rows));
 }
 bool decode_dense_applies(size_t T, size_t d, size_t f, size_t E, size_t k, size_t n_shared,
-                          int dtype, const void *x, const float *w_router) {
-  constexpr size_t kTokens = rq::kRouterThreads / 8;  // one quad-router workgroup
+                          int dtype, const void *x, const float *w_lds) {
   return dtype == PRICHS_DTYPE_BF16 && n_shared == 1 && E > 4 && E <= 8 && k >= 1 && k <= E &&
-         T >= 1 && T <= kTokens && d % 128 == 0 && (size_t)8 * (d + 4) * 4 <= 150 * 1024 &&
-         f % kBf16KMultiple == 0 && d <= (1u << 20) && f <= (1u << 20) &&
-         reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w_router) % 16 == 0;
+         T >= 1 && T <= (size_t)skinny::BM && d % 128 == 0 && f % kBf16KMultiple == 0 &&
+         d <= (1u << 20) && f <= (1u << 20) && router_chain_applies(T, d, E, x, w_lds);
 }
 
 int decode_gate_up_router(const void *x, size_t T, size_t d, size_t f, size_t E, size_t k,
-                          const float *w_router, const float *w_lds, const float *router_bias,
+                          const float *w_lds, const float *router_bias,
                           const float *concept_bias, size_t n_concept, float *logits,
                           int32_t *topk_idx, float *topk_w, int32_t *block_counts,
-                          int32_t *offsets, int32_t *row_token, float *row_weight,
-                          int32_t *token_row, int32_t *dense_row, const void *w_gate_up,
-                          void *act_dense, void *stream) {
-  PRICHS_REQUIRE(decode_dense_applies(T, d, f, E, k, 1, PRICHS_DTYPE_BF16, x, w_router),
+                          const void *w_gate_up, void *act_dense, void *stream) {
+  PRICHS_REQUIRE(decode_dense_applies(T, d, f, E, k, 1, PRICHS_DTYPE_BF16, x, w_lds),
                  "decode_gate_up_router: T=%zu, d=%zu, f=%zu, E=%zu, k=%zu not a decode shape",
                  T, d, f, E, k);
-  PRICHS_REQUIRE(x && w_router && router_bias && logits && topk_idx && topk_w && block_counts &&
-                     offsets && row_token && row_weight && token_row && dense_row && w_gate_up &&
-                     act_dense,
+  PRICHS_REQUIRE(x && w_lds && router_bias && logits && topk_idx && topk_w && block_counts &&
+                     w_gate_up && act_dense,
                  "decode_gate_up_router: null pointer argument");
   PRICHS_REQUIRE(concept_bias != nullptr || n_concept == 0,
                  "decode_gate_up_router: concept_bias is NULL but n_concept=%zu", n_concept);
@@ -1612,44 +1677,50 @@ int decode_gate_up_router(const void *x, size_t T, size_t d, size_t f, size_t E,
   const int G = (int)E + 1;
   const int nx = (int)(np / skinny::BN);
   const int mtiles = (int)((T + skinny::BM - 1) / skinny::BM);
-  const size_t lds = (size_t)8 * (d + 4) * sizeof(float);
-  static int attr_bytes = 0;
-  if ((int)lds > attr_bytes) {
-    PRICHS_HIP_TRY(hipFuncSetAttribute(
-                       reinterpret_cast<const void *>(&skinny::decode_gate_up_router_kernel<U>),
-                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
-                   "decode_gate_up_router: set LDS size");
-    attr_bytes = (int)lds;
-  }
+  const int routers = (int)cdiv(T, (size_t)rq::kChainTokens);
+  static_assert(rq::kChainLdsBytes <= 64 * 1024, "needs no raised LDS limit");
   const skinny::SkinnyArgs sa{static_cast<const bf16_t *>(x), nullptr, (int)d,
                               static_cast<const bf16_t *>(w_gate_up), (long long)(np * d), (int)d,
                               static_cast<bf16_t *>(act_dense), (int)f, (int)f, nullptr, (int)T,
-                              nullptr, (int)np, nullptr};
+                              nullptr, (int)np, nullptr, skinny::SelfPerm()};
   const int nc = (int)(n_concept < E ? n_concept : E);
-  const skinny::RouterArgs ra{static_cast<const bf16_t *>(x), w_router, router_bias, concept_bias,
+  const skinny::RouterArgs ra{static_cast<const bf16_t *>(x), w_lds, router_bias, concept_bias,
                               nc, (int)T, (int)d, (int)E, (int)k, logits, topk_idx, topk_w,
-                              block_counts,
-                              rq::FusedPerm{offsets, row_token, row_weight, token_row, dense_row},
-                              w_lds};
-  const unsigned grid = 1u + (unsigned)(nx * G * mtiles);
+                              block_counts};
+  const unsigned grid = (unsigned)(routers + nx * G * mtiles);
   hipLaunchKernelGGL((skinny::decode_gate_up_router_kernel<U>), dim3(grid), dim3(skinny::kThreads),
-                     lds, as_stream(stream), sa, ra, nx, G);
+                     rq::kChainLdsBytes, as_stream(stream), sa, ra, routers, nx, G);
   PRICHS_LAUNCH_CHECK("decode gate/up + router launch");
   return PRICHS_OK;
 }
 
-int decode_down(const void *act_dense, const int32_t *dense_row, const int32_t *offsets, size_t T,
-                size_t d, size_t f, size_t E, size_t k, const void *w_down, void *y, void *act,
+int decode_down(const void *act_dense, const int32_t *topk_idx, const float *topk_w, size_t T,
+                size_t d, size_t f, size_t E, size_t k, const void *w_down, int32_t *offsets,
+                int32_t *row_token, float *row_weight, int32_t *token_row, void *y, void *act,
                 void *stream) {
   if (int rc = check_gemm_shape(d, f, PRICHS_DTYPE_BF16, "decode_down")) return rc;
-  PRICHS_REQUIRE(act_dense && dense_row && offsets && w_down && y && act,
+  PRICHS_REQUIRE(act_dense && topk_idx && topk_w && offsets && row_token && row_weight &&
+                     token_row && w_down && y && act,
                  "decode_down: null pointer argument");
-  PRICHS_REQUIRE(T >= 1 && T <= (size_t)skinny::kSkinnyRows && k <= E,
+  PRICHS_REQUIRE(T >= 1 && T <= (size_t)skinny::BM && k <= E && k <= PRICHS_MAX_TOPK,
                  "decode_down: T=%zu, k=%zu, E=%zu not a decode shape", T, k, E);
   const size_t np = roundup(d, kPadRowsDown);
-  return launch_skinny<false>(act_dense, dense_row, (int)f, w_down, (long long)(np * f), (int)np,
-                              (int)f, y, (int)d, (int)d, offsets, (int)E + 1, T,
-                              as_stream(stream), nullptr, act);
+  const skinny::SkinnyArgs sa{static_cast<const bf16_t *>(act_dense), nullptr, (int)f,
+                              static_cast<const bf16_t *>(w_down), (long long)(np * f), (int)f,
+                              static_cast<bf16_t *>(y), (int)d, (int)d, nullptr, 0, nullptr,
+                              (int)np, static_cast<bf16_t *>(act),
+                              skinny::SelfPerm{topk_idx, topk_w, (int)T, (int)E, (int)k, offsets,
+                                               row_token, row_weight, token_row}};
+  // K-steps per chunk: the most that divide f evenly (a multiple of 64).
+  const dim3 grid((unsigned)(np / skinny::BN), (unsigned)(E + 1), 1), block(skinny::kThreads);
+  if (f % 128 == 0)
+    hipLaunchKernelGGL((skinny::skinny_gemm_kernel<false, 4, 1, true>), grid, block, 0,
+                       as_stream(stream), sa);
+  else
+    hipLaunchKernelGGL((skinny::skinny_gemm_kernel<false, 2, 1, true>), grid, block, 0,
+                       as_stream(stream), sa);
+  PRICHS_LAUNCH_CHECK("decode down launch");
+  return PRICHS_OK;
 }
 
 int grouped_gemm_rows(const void *A, const int32_t *a_rows, size_t lda, const void *B,

@@ -296,6 +296,18 @@ __global__ __launch_bounds__(kRouterThreads) void router_topk_quad_kernel(
                        block_counts, perm, w_lds, (int)blockIdx.x, wt_s);
 }
 
+// The chain router (router_quad.hpp): one workgroup per 8 tokens.
+template <typename XT>
+__global__ __launch_bounds__(kRouterThreads) void router_topk_chain_kernel(
+    const XT *__restrict__ x, const float *__restrict__ w_lds, const float *__restrict__ bias,
+    const float *__restrict__ concept, int n_concept, int T, int d, int E, int k,
+    float *__restrict__ logits, int32_t *__restrict__ topk_idx, float *__restrict__ topk_w,
+    int32_t *__restrict__ block_counts, FusedPerm perm) {
+  __shared__ f32x4 ring_s[kChainLdsF4];
+  router_chain_body<XT>(x, w_lds, bias, concept, n_concept, T, d, E, k, logits, topk_idx, topk_w,
+                        block_counts, perm, (int)blockIdx.x, ring_s);
+}
+
 template <typename XT>
 int launch_quad_t(const XT *x, const float *w, const float *bias, const float *concept, int nc,
                   int T, int d, int E, int k, float *logits, int32_t *idx, float *wt, int32_t *bc,
@@ -618,6 +630,52 @@ int router_topk_lds(const void *x, int x_dtype, const float *w_router, const flo
   return router_topk_impl(x, x_dtype, w_router, router_bias, concept_bias, n_concept, T, d, E, k,
                           logits, topk_idx, topk_w, block_counts, stream,
                           FusedPerm{nullptr, nullptr, nullptr, nullptr}, &fused, w_lds);
+}
+
+int router_topk_permute_chain(const void *x, int x_dtype, const float *w_lds,
+                              const float *router_bias, const float *concept_bias,
+                              size_t n_concept, size_t T, size_t d, size_t E, size_t k,
+                              float *logits, int32_t *topk_idx, float *topk_w,
+                              int32_t *block_counts, int32_t *offsets, int32_t *row_token,
+                              float *row_weight, int32_t *token_row, void *stream,
+                              void *routed_event) {
+  PRICHS_REQUIRE(router_chain_applies(T, d, E, x, w_lds) && k >= 1 && k <= E &&
+                     k <= PRICHS_MAX_TOPK && T <= (size_t)INT32_MAX / (k + 1),
+                 "router: T=%zu, d=%zu, E=%zu, k=%zu not a chain router shape", T, d, E, k);
+  PRICHS_REQUIRE(router_bias && topk_idx && topk_w && block_counts && offsets && row_token &&
+                     row_weight && token_row,
+                 "router: null pointer argument");
+  PRICHS_REQUIRE(concept_bias != nullptr || n_concept == 0,
+                 "router: concept_bias is NULL but n_concept=%zu", n_concept);
+  const int nb = (int)cdiv(T, (size_t)kChainTokens);
+  const int nc = (int)(n_concept < E ? n_concept : E);
+  hipStream_t s = as_stream(stream);
+  const FusedPerm perm = nb == 1 ? FusedPerm{offsets, row_token, row_weight, token_row}
+                                 : FusedPerm{nullptr, nullptr, nullptr, nullptr};
+  if (x_dtype == PRICHS_DTYPE_BF16)
+    hipLaunchKernelGGL(router_topk_chain_kernel<bf16_t>, dim3(nb), dim3(kRouterThreads), 0, s,
+                       static_cast<const bf16_t *>(x), w_lds, router_bias, concept_bias, nc,
+                       (int)T, (int)d, (int)E, (int)k, logits, topk_idx, topk_w, block_counts,
+                       perm);
+  else
+    hipLaunchKernelGGL(router_topk_chain_kernel<float>, dim3(nb), dim3(kRouterThreads), 0, s,
+                       static_cast<const float *>(x), w_lds, router_bias, concept_bias, nc,
+                       (int)T, (int)d, (int)E, (int)k, logits, topk_idx, topk_w, block_counts,
+                       perm);
+  PRICHS_LAUNCH_CHECK("router chain launch");
+  if (routed_event != nullptr)
+    PRICHS_HIP_TRY(hipEventRecord(static_cast<hipEvent_t>(routed_event), s), "router: event");
+  if (nb == 1) return PRICHS_OK;
+  hipLaunchKernelGGL(permute_kernel, dim3(nb), dim3(256), 0, s, topk_idx, topk_w, block_counts,
+                     (int)T, (int)E, (int)k, kChainTokens, nb, offsets, row_token, row_weight,
+                     token_row);
+  PRICHS_LAUNCH_CHECK("permute launch");
+  return PRICHS_OK;
+}
+
+bool router_chain_applies(size_t T, size_t d, size_t E, const void *x, const float *w_lds) {
+  return T >= 1 && T <= kRouterChainMaxTokens && w_lds != nullptr && E >= 1 && E <= 8 &&
+         d % kChainK == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
 }
 
 int router_topk_permute(const void *x, int x_dtype, const float *w_router,

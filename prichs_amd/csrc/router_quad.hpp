@@ -1,8 +1,8 @@
 // router_quad.hpp -- router device code shared by router.hip (the router and
-// permutation kernels) and gemm.hip (the decode launch that runs one router
-// workgroup beside the gate/up GEMM): top-k gating of one token, the
-// permutation of a batch that one workgroup covers, and the body of the
-// quad-broadcast router workgroup.  Restates crates/prichs-model/src/
+// permutation kernels) and gemm.hip (the decode launch that runs router
+// workgroups beside the gate/up GEMM): top-k gating of one token, the
+// permutation of a batch that one workgroup covers, and the bodies of the
+// quad-broadcast and chain router workgroups.  Restates crates/prichs-model/src/
 // moe.rs:113-142 and crates/prichs-core/src/ops.rs:219-248 (see router.hip).
 #pragma once
 
@@ -146,16 +146,11 @@ __device__ inline void topk_epilogue(float acc, float adj, bool valid, int e, in
 // per expert).  The 64-lane windows are taken in order by wave 0 alone,
 // which keeps the running bases sequential.  All threads then write the
 // shared-expert rows, which follow the routed rows in token order.
-// dense_row (may be null): for each row r of the row space, the row of the
-// dense [group][token] layout holding the same (expert, token) pair --
-// expert e's row of token t is e * T + t, the shared row of token t is
-// E * T + t (the decode path runs the gate/up GEMM densely over all tokens).
 __device__ inline void place_entries(const int32_t *__restrict__ topk_idx,
                                      const float *__restrict__ topk_w, int t0, int t1, int T,
                                      int E, int k, const int *base_s, int32_t *__restrict__ row_token,
                                      float *__restrict__ row_weight,
-                                     int32_t *__restrict__ token_row,
-                                     int32_t *__restrict__ dense_row = nullptr) {
+                                     int32_t *__restrict__ token_row) {
   const int tid = threadIdx.x;
   if (tid < 64) {
     const int lane = tid;
@@ -178,14 +173,10 @@ __device__ inline void place_entries(const int32_t *__restrict__ topk_idx,
         row_token[r] = (int32_t)(ts / k);
         row_weight[r] = wt;
         token_row[ts] = r;
-        if (dense_row != nullptr) dense_row[r] = e_me * T + (int32_t)(ts / k);
       }
     }
   }
-  for (int t = t0 + tid; t < t1; t += blockDim.x) {
-    row_token[(size_t)T * k + t] = t;
-    if (dense_row != nullptr) dense_row[(size_t)T * k + t] = E * T + t;
-  }
+  for (int t = t0 + tid; t < t1; t += blockDim.x) row_token[(size_t)T * k + t] = t;
 }
 
 // Outputs of the permutation, filled by the router's own workgroup when one
@@ -195,8 +186,41 @@ struct FusedPerm {
   int32_t *offsets, *row_token;
   float *row_weight;
   int32_t *token_row;
-  int32_t *dense_row;  // optional (see place_entries)
 };
+
+// The end of a router workgroup: its expert histogram, and with a fused
+// permutation (the only workgroup) the placement of its entries, which are in
+// idx_s / wsel_s.
+__device__ inline void finish_block(const int *cnt_s, const int32_t *idx_s, const float *wsel_s,
+                                    int T, int E, int k, int32_t *__restrict__ block_counts,
+                                    const FusedPerm &perm, int bid) {
+  const int tid = threadIdx.x;
+  __syncthreads();
+  if (tid < E) block_counts[(size_t)bid * E + tid] = cnt_s[tid];
+  if (perm.offsets == nullptr) return;
+  // The histogram is the expert totals, the exclusive scan gives the bases
+  // (as permute_kernel's block 0 computes them).
+  __shared__ int base_s[PRICHS_MAX_EXPERTS];
+  if (tid == 0) {
+    int run = 0;
+    for (int ee = 0; ee < E; ++ee) {
+      base_s[ee] = run;
+      perm.offsets[ee] = run;
+      run += cnt_s[ee];
+    }
+    perm.offsets[E] = run;  // == T * k
+    perm.offsets[E + 1] = run + T;
+  }
+  __syncthreads();
+  place_entries(idx_s, wsel_s, 0, T, T, E, k, base_s, perm.row_token, perm.row_weight,
+                perm.token_row);
+}
+
+// LDS writes done, then the workgroup barrier; unlike __syncthreads it leaves
+// global loads in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
 
 // ---------------------------------------------------------------------------
 // Quad-broadcast router (E <= 8, eight lanes per token, d % 128 == 0).  The
@@ -378,28 +402,147 @@ __device__ inline void router_quad_body(
   const bool fused = perm.offsets != nullptr;
   topk_epilogue(acc, adj, valid, e, t, T, E, k, 8, logits, topk_idx, topk_w, cnt_s,
                 fused ? idx_s : nullptr, fused ? wsel_s : nullptr);
-  __syncthreads();
-  if (tid < E) block_counts[(size_t)bid * E + tid] = cnt_s[tid];
-  if (fused) {
-    // The only workgroup: the histogram is the expert totals, the exclusive
-    // scan gives the bases (as permute_kernel's block 0 computes them), and
-    // the block's entries (in LDS, visible after the barrier) are placed
-    // here.
-    __shared__ int base_s[PRICHS_MAX_EXPERTS];
-    if (tid == 0) {
-      int run = 0;
-      for (int ee = 0; ee < E; ++ee) {
-        base_s[ee] = run;
-        perm.offsets[ee] = run;
-        run += cnt_s[ee];
+  finish_block(cnt_s, idx_s, wsel_s, T, E, k, block_counts, perm, bid);
+}
+
+// ---------------------------------------------------------------------------
+// Chain router (E <= 8, d % 32 == 0): 8 tokens per workgroup, for batches that
+// leave most CUs without a quad workgroup.  Each logit is a chain of d rounded
+// sums (k ascending), and one wave per SIMD takes 9 cycles per dependent add;
+// the quad kernel's multiplies, conversions and weight reads in the same wave
+// bring that to 12.5.  Here wave 0 only adds: lane 8 t + e holds the chain of
+// (token t, expert e).  Waves 1-3 form the rounded products, each for every
+// third chunk of 32 k: lane (e, q) holds W[e][4q .. 4q + 3], reads x of each
+// token from a wave-private LDS row and writes the products at [q][8 t + e],
+// as float4 (slot XOR q: conflict-free for the writes, whose lanes run over q,
+// and for the reads).  Products are double-buffered by rounds of three chunks,
+// one barrier per round; the adder keeps a round's last chunk in registers and
+// adds it behind the next round's first reads.  Weights and x are loaded
+// straight from global memory, kAhead rounds ahead, so nothing waits for a
+// staged W^T first.
+// ---------------------------------------------------------------------------
+constexpr int kChainTokens = 8;                    // tokens per workgroup
+constexpr int kChainK = 32, kChainProd = 3;        // k per chunk, producer waves
+constexpr int kChainChunk = kChainK / 4 * 64;      // float4 of one chunk's products
+constexpr int kChainLdsF4 = 2 * kChainProd * kChainChunk + kChainProd * 64;
+constexpr size_t kChainLdsBytes = sizeof(float) * 4 * (size_t)kChainLdsF4;
+
+template <typename XT>
+__device__ inline void router_chain_body(
+    const XT *__restrict__ x, const float *__restrict__ w_lds, const float *__restrict__ bias,
+    const float *__restrict__ concept, int n_concept, int T, int d, int E, int k,
+    float *__restrict__ logits, int32_t *__restrict__ topk_idx, float *__restrict__ topk_w,
+    int32_t *__restrict__ block_counts, FusedPerm perm, int bid, f32x4 *__restrict__ ring_s) {
+#pragma clang fp contract(off)
+  __shared__ int cnt_s[PRICHS_MAX_EXPERTS];
+  __shared__ int32_t idx_s[kChainTokens * PRICHS_MAX_TOPK];
+  __shared__ float wsel_s[kChainTokens * PRICHS_MAX_TOPK];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nch = d / kChainK;
+  const int rounds = (nch + kChainProd - 1) / kChainProd;
+  const bool fused = perm.offsets != nullptr;
+  if (tid < E) cnt_s[tid] = 0;
+
+  if (wave > 0) {
+    const int j = wave - 1;
+    const int hi = lane >> 3, q = lane & 7;
+    const float *wp = w_lds + (size_t)(hi < E ? hi : 0) * (d + 4) + 4 * q;  // expert hi
+    const XT *xp = x + (size_t)min(bid * kChainTokens + hi, T - 1) * d + 4 * q;  // token hi
+    f32x4 *const xs = ring_s + 2 * kChainProd * kChainChunk + j * 64;
+    constexpr int kAhead = 8;
+    f32x4 wr[kAhead];
+    uint32_t xr[kAhead][sizeof(XT)];  // 4 values: 2 words of bf16, 4 of f32
+    auto fetch = [&](int r, int i) {
+      const int c = min(kChainProd * r + j, nch - 1) * kChainK;
+      wr[i] = *reinterpret_cast<const f32x4 *>(wp + c);
+      if constexpr (sizeof(XT) == 2) {
+        const uint2 u = *reinterpret_cast<const uint2 *>(xp + c);
+        xr[i][0] = u.x, xr[i][1] = u.y;
+      } else {
+        const uint4 u = *reinterpret_cast<const uint4 *>(xp + c);
+        xr[i][0] = u.x, xr[i][1] = u.y, xr[i][2] = u.z, xr[i][3] = u.w;
       }
-      perm.offsets[E] = run;  // == T * k
-      perm.offsets[E + 1] = run + T;
+    };
+    auto produce = [&](int r, int i) {
+      f32x4 xv;
+      if constexpr (sizeof(XT) == 2) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          xv[2 * h] = __uint_as_float(xr[i][h] << 16);
+          xv[2 * h + 1] = __uint_as_float(xr[i][h] & 0xffff0000u);
+        }
+      } else {
+#pragma unroll
+        for (int h = 0; h < 4; ++h) xv[h] = __uint_as_float(xr[i][h]);
+      }
+      const f32x4 wv = wr[i];
+      fetch(r + kAhead, i);
+      xs[lane] = xv;  // [token][q]; the wave's own LDS operations stay in order
+      f32x4 *const out = ring_s + ((r & 1) * kChainProd + j) * kChainChunk + q * 64;
+      f32x4 p[kChainTokens];
+#pragma unroll
+      for (int t = 0; t < kChainTokens; ++t) p[t] = xs[8 * t + q];
+#pragma unroll
+      for (int t = 0; t < kChainTokens; ++t) {
+#pragma unroll
+        for (int h = 0; h < 4; ++h) p[t][h] = p[t][h] * wv[h];
+        out[(8 * t + hi) ^ q] = p[t];
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) fetch(i, i);
+    for (int r0 = 0; r0 < rounds; r0 += kAhead) {
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        if (r0 + i < rounds) {
+          produce(r0 + i, i);
+          lds_barrier();
+        }
+      }
     }
-    __syncthreads();
-    place_entries(idx_s, wsel_s, 0, T, T, E, k, base_s, perm.row_token, perm.row_weight,
-                  perm.token_row, perm.dense_row);
+    lds_barrier();
+  } else {
+    float acc = 0.0f;
+    f32x4 held[kChainK / 4];
+    auto read = [&](int r, int j, f32x4(&v)[kChainK / 4]) {
+      const f32x4 *src = ring_s + ((r & 1) * kChainProd + j) * kChainChunk;
+#pragma unroll
+      for (int q = 0; q < kChainK / 4; ++q) v[q] = src[q * 64 + (lane ^ q)];
+    };
+    auto add = [&](const f32x4(&v)[kChainK / 4]) {
+#pragma unroll
+      for (int q = 0; q < kChainK / 4; ++q)
+#pragma unroll
+        for (int h = 0; h < 4; ++h) acc = acc + v[q][h];
+    };
+    // Round r's products are complete after barrier r; its buffer is written
+    // again only after barrier r + 1, which this wave reaches with its reads
+    // of round r done.
+    for (int r = 0; r < rounds; ++r) {
+      lds_barrier();
+      f32x4 v0[kChainK / 4], v1[kChainK / 4];
+      read(r, 0, v0);
+      if (r > 0) add(held);  // always a whole round before
+      read(r, 1, v1);
+      read(r, 2, held);
+      add(v0);
+      if (kChainProd * r + 1 < nch) add(v1);
+    }
+    lds_barrier();
+    if (kChainProd * (rounds - 1) + 2 < nch) add(held);
+
+    const int e = lane & 7, t = bid * kChainTokens + (lane >> 3);
+    const bool valid = t < T && e < E;
+    float adj = 0.0f;
+    if (valid) {
+      adj = acc + bias[e];
+      if (concept != nullptr && e < n_concept) adj = adj + concept[e];
+    }
+    topk_epilogue(acc, adj, valid, e, t, T, E, k, 8, logits, topk_idx, topk_w, cnt_s,
+                  fused ? idx_s : nullptr, fused ? wsel_s : nullptr);
   }
+  finish_block(cnt_s, idx_s, wsel_s, T, E, k, block_counts, perm, bid);
 }
 
 }  // namespace rq
