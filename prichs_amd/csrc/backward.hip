@@ -268,6 +268,7 @@ constexpr size_t kLdsBytes = (size_t)kStages * kStageBytes;  // 128 KiB
 constexpr uint32_t kHiOff = 16 * kRowBytes;           // rows 16.. of a tile
 constexpr uint32_t kOutOfRange = 0x80000000u;         // buffer offset that loads zeros
 constexpr int kSplitRows = 2560;
+constexpr size_t kShortLdsBytes = 3 * (size_t)(kTileBytes / 2 + kTileBytes);  // 72 KiB
 static_assert(BQ == 4 * 64 && BP == 2 * 128, "wave grid 2 x 4 of 128 x 64");
 static_assert(kThreads == 8 * 64, "ping-pong K loop: two groups of 4 waves, one of each per SIMD");
 }  // namespace wgb
@@ -306,12 +307,19 @@ __device__ __forceinline__ void wg_wait_tied(u32x2 (&a)[8]) {
                :
                : "memory");
 }
+__device__ __forceinline__ void wg_wait_tied(u32x2 (&a)[4]) {
+  asm volatile("s_waitcnt lgkmcnt(0)"
+               : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3])
+               :
+               : "memory");
+}
 // s_waitcnt with only vmcnt constrained (gfx9 encoding, vmcnt < 16 here).
 #define PRICHS_WG_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (7 << 4) | (15 << 8))
 
 // One work item: P rows [i0, i0 + BPT) x Q columns [j0, j0 + 256) of group g's
-// dW over the item's rows (BPT = 256: a whole tile; 128: half of one).
-template <bool GATEUP, int BPT>
+// dW over the item's rows (BPT = 256: a whole tile; 128: half of one).  S
+// stages of LDS; S = 3 leaves room for two workgroups of 128-row items per CU.
+template <bool GATEUP, int BPT, int S = wgb::kStages>
 __device__ __forceinline__ void wgrad_item(
     const bf16_t *__restrict__ A, int lda, uint32_t a_bytes, const bf16_t *__restrict__ B,
     int ldb, uint32_t b_bytes, int E, int P, int Q, float *out0, float *out1, int ldo,
@@ -319,6 +327,8 @@ __device__ __forceinline__ void wgrad_item(
     int a_row_lo, int b_row_lo, int mg, int pslot, int i0, int j0) {
   using namespace wgb;
   static_assert(BPT == 256 || BPT == 128, "whole or half tiles");
+  static_assert(S == 4 || (S == 3 && BPT == 128), "rings of 4, or 3 for short items");
+  auto slot = [](int kt) { return S == 4 ? kt & 3 : kt % 3; };
   // A tile: [BK][BPT] bf16 (rows of kRowA bytes); B tile: [BK][256].
   constexpr int kRowA = 2 * BPT;
   constexpr uint32_t kTileA = BK * kRowA;
@@ -355,7 +365,7 @@ __device__ __forceinline__ void wgrad_item(
     a_col[i] = 2u * (uint32_t)(i0 + lc * 8);
   }
   auto issue = [&](int kt) {
-    bf16_t *sa = lds + (size_t)(kt & (kStages - 1)) * (kStage / 2);
+    bf16_t *sa = lds + (size_t)slot(kt) * (kStage / 2);
     bf16_t *sb = sa + kTileA / 2;
 #pragma unroll
     for (int i = 0; i < kInstA; ++i) {
@@ -405,7 +415,7 @@ __device__ __forceinline__ void wgrad_item(
   // Ping-pong K loop (as the forward GEMM's): waves 0-3 (group 0) and 4-7
   // (group 1) sit one per SIMD each.  Every wave runs, per K-step kt, a
   // memory phase (the transposing reads of stage kt, its share of stage
-  // kt + 3, a wait for its share of stage kt + 1 and for its reads), a
+  // kt + S - 1 (here S = 4), a wait for its share of stage kt + 1 and for its reads), a
   // barrier, an MFMA phase, a barrier; group 1 runs one barrier behind, so on
   // each SIMD one wave multiplies while the other reads and loads.
   //  - Stage s is first read after b(2s-1); both groups waited for their
@@ -426,9 +436,9 @@ __device__ __forceinline__ void wgrad_item(
   };
   issue(0);
   if (KT > 1) issue(1);
-  if (KT > 2) issue(2);
+  if (S == 4 && KT > 2) issue(2);
   // Own share of stage 0 (kInst instructions per stage and wave).
-  if (KT > 2)
+  if (S == 4 && KT > 2)
     PRICHS_WG_VMCNT(2 * kInst);
   else if (KT > 1)
     PRICHS_WG_VMCNT(kInst);
@@ -437,26 +447,22 @@ __device__ __forceinline__ void wgrad_item(
   pp_barrier();
   if (grp == 1) pp_barrier();  // group 1 runs one phase behind
   // One K-step; kAhead = this wave's stages still allowed in flight after the
-  // wait (stages kt + 2 .. min(kt + 3, KT - 1)), a compile-time count.
+  // wait (stages kt + 2 .. min(kt + S - 1, KT - 1)), a compile-time count.
   auto kstep = [&](int kt, auto ahead_c) {
     constexpr int kAhead = decltype(ahead_c)::value;
-    const uint32_t st = (uint32_t)(kt & (kStages - 1)) * kStage;
-    u32x2 alo[8], ahi[8], bt[8];  // bt: B lo (0..3) and hi (4..7); A: kIB used
+    const uint32_t st = (uint32_t)slot(kt) * kStage;
+    u32x2 alo[kIB], ahi[kIB], bt[8];  // bt: B lo (0..3) and hi (4..7)
 #pragma unroll
     for (int blk = 0; blk < 4; ++blk) {
       bt[blk] = wg_read_tr<0>(b_rd[blk] + st);
       bt[4 + blk] = wg_read_tr<(int)kHiOff>(b_rd[blk] + st);
     }
 #pragma unroll
-    for (int blk = 0; blk < 8; ++blk) {
-      if (blk < kIB) {
-        alo[blk] = wg_read_tr<0>(a_rd[blk] + st);
-        ahi[blk] = wg_read_tr<(int)kHiA>(a_rd[blk] + st);
-      } else {
-        alo[blk] = ahi[blk] = u32x2{0u, 0u};
-      }
+    for (int blk = 0; blk < kIB; ++blk) {
+      alo[blk] = wg_read_tr<0>(a_rd[blk] + st);
+      ahi[blk] = wg_read_tr<(int)kHiA>(a_rd[blk] + st);
     }
-    if constexpr (kAhead == 2) issue(kt + 3);
+    if constexpr (kAhead == S - 2) issue(kt + S - 1);
     PRICHS_WG_VMCNT(kInst * kAhead);
     wg_wait_tied(bt);
     wg_wait_tied(alo);
@@ -475,10 +481,11 @@ __device__ __forceinline__ void wgrad_item(
     }
     pp_barrier();
   };
-  // Steps that issue stage kt + 3, then the last (up to three).
+  // Steps that issue stage kt + S - 1, then the last (up to S - 1).
   int kt = 0;
-  for (; kt + 3 < KT; ++kt) kstep(kt, std::integral_constant<int, 2>{});
-  if (kt + 2 < KT) kstep(kt++, std::integral_constant<int, 1>{});
+  for (; kt + S - 1 < KT; ++kt) kstep(kt, std::integral_constant<int, S - 2>{});
+  if constexpr (S == 4)
+    if (kt + 2 < KT) kstep(kt++, std::integral_constant<int, 1>{});
   if (kt + 1 < KT) kstep(kt++, std::integral_constant<int, 0>{});
   if (kt < KT) kstep(kt++, std::integral_constant<int, 0>{});
   if (grp == 0) pp_barrier();  // both groups leave after the same barrier count
@@ -487,7 +494,7 @@ __device__ __forceinline__ void wgrad_item(
   // of the wave's (BPT / 2) x 64 block.
   //
   // The tile leaves through the stage ring (idle after the last K-step), 128
-  // rows of 1 KiB at a time: the waves holding them write their fragments to
+  // (S = 3: 64) rows of 1 KiB at a time: the waves holding them write their fragments to
   // LDS (float4 chunk c of row r at c ^ (r & 15), no bank conflicts either
   // way), then each wave stores 16 whole rows, one 1 KiB row per
   // instruction, instead of 16 rows x 64 bytes per instruction.
@@ -495,7 +502,8 @@ __device__ __forceinline__ void wgrad_item(
   float *const pbase = pslot >= 0 ? part + (long long)pslot * P * Q : nullptr;
   const bool rmw = pslot < 0 && beta != 0;  // dW += tile (beta = 1, an unsplit group)
   f32x4 *const st = reinterpret_cast<f32x4 *>(lds);
-  constexpr int kPasses = BPT / 128;
+  constexpr int kPassRows = S == 4 ? 128 : 64;
+  constexpr int kPasses = BPT / kPassRows;
 #pragma unroll
   for (int h = 0; h < kPasses; ++h) {
     if (kPasses == 1 || wp == h) {
@@ -509,27 +517,28 @@ __device__ __forceinline__ void wgrad_item(
         }
     }
     __syncthreads();
-    // Rows in batches of 8: all loads of a batch (LDS, and the old values
-    // for a read-modify-write) are issued before its stores.
+    // Rows in batches of 8 (S = 3: 4): all loads of a batch (LDS, and the old
+    // values for a read-modify-write) are issued before its stores.
+    constexpr int kRows = S == 4 ? 8 : 4;
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      f32x4 v[8];
-      float *dst[8];
+    for (int b = 0; b < kPassRows / 8 / kRows; ++b) {
+      f32x4 v[kRows];
+      float *dst[kRows];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int r = wave * 16 + b * 8 + e;
-        const int i = i0 + h * 128 + r, j = j0 + 4 * lane;
+      for (int e = 0; e < kRows; ++e) {
+        const int r = wave * (kPassRows / 8) + b * kRows + e;
+        const int i = i0 + h * kPassRows + r, j = j0 + 4 * lane;
         v[e] = st[r * 64 + (lane ^ (r & 15))];
         dst[e] = pbase != nullptr ? (i < P && j < Q ? pbase + (long long)i * Q + j : nullptr)
                                   : wgrad_dst<GATEUP>(out0, out1, ldo, base, i, j, P, Q, f);
       }
       if (rmw) {
-        float4 old[8];
+        float4 old[kRows];
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
+        for (int e = 0; e < kRows; ++e)
           old[e] = dst[e] ? *reinterpret_cast<const float4 *>(dst[e]) : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
+        for (int e = 0; e < kRows; ++e) {
           v[e][0] = old[e].x + v[e][0];
           v[e][1] = old[e].y + v[e][1];
           v[e][2] = old[e].z + v[e][2];
@@ -537,7 +546,7 @@ __device__ __forceinline__ void wgrad_item(
         }
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
+      for (int e = 0; e < kRows; ++e)
         if (dst[e]) {
           // The gradients go back to the caller and nothing in the step reads
           // them again: non-temporal stores keep their 211 MB (config 2) out
@@ -661,6 +670,35 @@ __global__ __launch_bounds__(wgb::kThreads) void wgrad_bf16_kernel(
                             part, beta, lds, g, a_row_lo, b_row_lo, mg, pslot, i0 + 128 * half,
                             j0);
   }
+}
+
+// Short items (wgrad_short): most of an item's time is then its epilogue, whose 256 KiB of f32 per 256 x 256 tile leave every CU at
+// the same time.  One workgroup per (group, 128 x 256 tile), the shared group
+// first, three stages of LDS and at most 128 registers, so two share a CU and
+// one's stores run behind the other's products; no group is split, and a
+// group without rows writes its zeros (beta = 0) here, so there is no reduce
+// pass.  The same MFMA chain per element as the items above.
+template <bool GATEUP>
+__global__ __launch_bounds__(wgb::kThreads, 4) void wgrad_bf16_short_kernel(
+    const bf16_t *__restrict__ A, int lda, uint32_t a_bytes, const bf16_t *__restrict__ B,
+    int ldb, uint32_t b_bytes, const int32_t *__restrict__ offsets, int G, int E, int P, int Q,
+    int tiles_q, int tiles, float *out0, float *out1, int ldo, long long slot_stride, int f,
+    int beta, const bf16_t *__restrict__ A2, uint32_t a2_bytes, const bf16_t *__restrict__ B2,
+    uint32_t b2_bytes, int alt_g, int alt_row0) {
+  extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
+  const int gi = (int)(blockIdx.x / (unsigned)tiles);
+  const int g = (gi + G - 1) % G;
+  const int id = (int)f32t::xcd_run(blockIdx.x - (unsigned)(gi * tiles), (unsigned)tiles);
+  const int row_lo = offsets[g];
+  const int mg = max(offsets[g + 1] - row_lo, 0);
+  if (mg == 0 && beta != 0) return;
+  const int tp = id / tiles_q;
+  const bool alt_a = g == alt_g && A2 != nullptr, alt_b = g == alt_g && B2 != nullptr;
+  wgrad_item<GATEUP, 128, 3>(alt_a ? A2 : A, lda, alt_a ? a2_bytes : a_bytes, alt_b ? B2 : B, ldb,
+                             alt_b ? b2_bytes : b_bytes, E, P, Q, out0, out1, ldo, slot_stride, f,
+                             nullptr, beta, lds, g, alt_a ? row_lo - alt_row0 : row_lo,
+                             alt_b ? row_lo - alt_row0 : row_lo, mg, -1, tp * 128,
+                             (id - tp * tiles_q) * wgb::BQ);
 }
 
 // Finishes the groups the tile kernel does not write whole: a split group
@@ -1213,18 +1251,28 @@ size_t bwd_wgrad_part_elems(size_t max_rows, size_t P, size_t Q) {
   return 2 * (max_rows / wgb::kSplitRows) * P * Q;
 }
 
+// Whether the bf16 weight gradients take wgrad_bf16_short_kernel: where the
+// other kernel would not split a group either, and up to 4096 rows per group
+// where the items fill the CUs' two places at least twice, so that the longest
+// group's do not run alone.  Measured on MI355X (d = 1536, f = 1280, 8 + 1
+// experts, top-2, beta = 0; other -> short kernel, us with the reduce pass):
+// dW_gate/up 300 tokens 55.9 -> 33.3, 1000 78.6 -> 47.2, 2500 131 -> 88.3, 4096
+// 160 -> 126, 8192 222 -> 225; dW_down (half as many items) 300 37.7 -> 23.4,
+// 1000 54.9 -> 32.7, 2500 89.6 -> 63.3, 4096 99.4 -> 97.5, 8192 133 -> 189.
+bool wgrad_short(size_t max_group_rows, size_t items, int cus) {
+  return max_group_rows <= (size_t)wgb::kSplitRows ||
+         (max_group_rows <= 4096 && items >= 4 * (size_t)cus);
+}
+
 int bwd_wgrad(bool gateup, const void *A, size_t lda, const void *B, size_t ldb, size_t total_rows,
-              size_t max_group_rows, const int32_t *offsets, size_t G, size_t E, size_t P, size_t Q, float *out0,
-              float *out1, size_t ldo, size_t slot_stride, size_t f, int dtype, float *part,
+              size_t max_group_rows, const int32_t *offsets, size_t G, size_t E, size_t P, size_t Q,
+              float *out0, float *out1, size_t ldo, size_t slot_stride, size_t f, int dtype, float *part,
               int beta, hipStream_t s, const WgradAlt &alt) {
   if (total_rows == 0) return PRICHS_OK;
   const int cus = device_cu_count();
   const unsigned rgrid = (unsigned)std::max(1, 4 * cus);
   if (dtype == PRICHS_DTYPE_BF16) {
     const int tiles_q = (int)cdiv(Q, wgb::BQ);
-    const int tiles = (int)cdiv(P, wgb::BP) * tiles_q;
-    // Every group's chunks: at most G + total_rows / kSplitRows per tile.
-    const size_t items = (G + total_rows / wgb::kSplitRows) * (size_t)tiles;
     const size_t ab = total_rows * lda * 2, bb = total_rows * ldb * 2;
     const size_t ab2 = alt.A ? alt.rows * lda * 2 : 0, bb2 = alt.B ? alt.rows * ldb * 2 : 0;
     if (ab >= wgb::kOutOfRange || bb >= wgb::kOutOfRange || ab2 >= wgb::kOutOfRange ||
@@ -1232,6 +1280,32 @@ int bwd_wgrad(bool gateup, const void *A, size_t lda, const void *B, size_t ldb,
       return fail(PRICHS_ERR_UNSUPPORTED,
                   "moe backward: operands of %zu and %zu bytes or a %zu x %zu gradient exceed 2 GiB",
                   ab, bb, P, Q);
+    const size_t n = cdiv(P, 128) * (size_t)tiles_q;  // 128 x 256 tiles
+    if (wgrad_short(max_group_rows, n * G, cus)) {
+      if (n * G > (size_t)INT32_MAX)
+        return fail(PRICHS_ERR_UNSUPPORTED, "moe backward: too many tiles");
+      auto sk = gateup ? wgrad_bf16_short_kernel<true> : wgrad_bf16_short_kernel<false>;
+      static bool short_attr_set[2] = {false, false};
+      if (!short_attr_set[gateup]) {
+        PRICHS_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(sk),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           (int)wgb::kShortLdsBytes),
+                       "moe backward: set LDS size");
+        short_attr_set[gateup] = true;
+      }
+      hipLaunchKernelGGL(sk, dim3((unsigned)(n * G)), dim3(wgb::kThreads), wgb::kShortLdsBytes, s,
+                         static_cast<const bf16_t *>(A), (int)lda, (uint32_t)ab,
+                         static_cast<const bf16_t *>(B), (int)ldb, (uint32_t)bb, offsets, (int)G,
+                         (int)E, (int)P, (int)Q, tiles_q, (int)n, out0, out1, (int)ldo,
+                         (long long)slot_stride, (int)f, beta, static_cast<const bf16_t *>(alt.A),
+                         (uint32_t)ab2, static_cast<const bf16_t *>(alt.B), (uint32_t)bb2,
+                         alt.A || alt.B ? (int)alt.g : -1, (int)alt.row0);
+      PRICHS_LAUNCH_CHECK("moe backward: weight gradient");
+      return PRICHS_OK;
+    }
+    const int tiles = (int)cdiv(P, wgb::BP) * tiles_q;
+    // Every group's chunks: at most G + total_rows / kSplitRows per tile.
+    const size_t items = (G + total_rows / wgb::kSplitRows) * (size_t)tiles;
     if (items + (size_t)cus > (size_t)INT32_MAX)
       return fail(PRICHS_ERR_UNSUPPORTED, "moe backward: too many tiles");
     auto kern = gateup ? wgrad_bf16_kernel<true, false> : wgrad_bf16_kernel<false, true>;

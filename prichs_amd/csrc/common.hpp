@@ -197,9 +197,9 @@ struct WgradAlt {
   size_t g = 0, row0 = 0, rows = 0;
 };
 int bwd_wgrad(bool gateup, const void *A, size_t lda, const void *B, size_t ldb, size_t total_rows,
-              size_t max_group_rows, const int32_t *offsets, size_t G, size_t E, size_t P, size_t Q, float *out0,
-              float *out1, size_t ldo, size_t slot_stride, size_t f, int dtype, float *part,
-              int beta, hipStream_t s, const WgradAlt &alt = WgradAlt());
+              size_t max_group_rows, const int32_t *offsets, size_t G, size_t E, size_t P, size_t Q,
+              float *out0, float *out1, size_t ldo, size_t slot_stride, size_t f, int dtype,
+              float *part, int beta, hipStream_t s, const WgradAlt &alt = WgradAlt());
 int bwd_combine(const void *dX, const float *scal, const int32_t *topk_idx, const float *topk_w,
                 const int32_t *token_row, const float *wrt, size_t T, size_t d, size_t k,
                 int weighting, int dtype, float *dlr, void *d_x, int dx_dtype, hipStream_t s);

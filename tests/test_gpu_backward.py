@@ -123,6 +123,28 @@ def test_backward_bf16_matches_oracle(cuda, orc, T, d, f, E, k, weighting):
     check_against_oracle(orc, inp, d_out, weighting, d_x, grads, TOL["bf16"])
 
 
+# The short-item weight gradients (128 x 256 tiles, 3 LDS stages): gradients
+# ending inside a tile, groups of one row, of one to four 32-row K-steps and
+# without rows, and (2600 tokens at the large size) groups longer than the
+# other kernel's split, which dW_down then takes.
+@pytest.mark.parametrize("T,d,f,E,k", [(5, 192, 64, 8, 2), (40, 64, 192, 5, 1),
+                                       (70, 320, 320, 4, 2), (130, 448, 128, 2, 1),
+                                       (2600, 1536, 1280, 8, 2)])
+@pytest.mark.parametrize("beta", [0, 1])
+def test_backward_short_items(cuda, orc, T, d, f, E, k, beta):
+    say("short items", T, d, f, E, k, "beta", beta)
+    inp, d_out = inputs(T, d, f, E, k, "bf16", seed=T + d, w_std=0.05)
+    eng = make_engine(inp)
+    x = dev(inp.x, "bf16")
+    eng.forward(x)
+    grads = zero_grads(inp)
+    if beta == 0:  # every element is written, experts without rows included
+        for t in grads.values():
+            t.fill_(float("nan"))
+    d_x = eng.backward(x, dev(d_out, "bf16"), grads, d_x_dtype=torch.float32, beta=beta)
+    check_against_oracle(orc, inp, d_out, 2, d_x, grads, TOL["bf16"])
+
+
 @pytest.mark.parametrize("T", [400, 6000])
 def test_backward_skewed_routing(cuda, orc, T):
     # Config-3 style bias: experts 0-1 take most rows, some experts may get none.
