@@ -204,6 +204,14 @@ __device__ inline void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// The same between LDS writes and other waves' reads of them: the bare barrier
+// does not wait for the writes (the LDS queues of the SIMDs drain on their
+// own), so the wave waits for its own first.
+__device__ inline void lds_write_barrier() {
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+  lds_barrier();
+}
+
 #ifndef PRICHS_BF16_STAGES
 #define PRICHS_BF16_STAGES 4
 #endif
@@ -507,7 +515,7 @@ __device__ __forceinline__ void bf16_tile(
             u32x2{pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3])};
       }
     }
-    lds_barrier();
+    lds_write_barrier();
     constexpr int kChunksRow = BN / 8;  // 16-byte chunks per tile row
     if constexpr (DSW) {
       // SwiGLU backward on the staged (bf16-rounded) dA: chunk ch of row r
@@ -628,7 +636,7 @@ __device__ __forceinline__ void bf16_tile(
               u32x2{pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3])};
         }
       }
-      lds_barrier();
+      lds_write_barrier();
       constexpr int kChunksRow = BN / 8;  // 16-byte chunks per tile row
 #pragma unroll 4
       for (int c = tid; c < BM * kChunksRow; c += Cf::kThreads) {
@@ -677,7 +685,7 @@ __device__ __forceinline__ void bf16_tile(
           }
         }
       }
-      lds_barrier();
+      lds_write_barrier();
       constexpr int kChunksRow = BN / 16;  // 16-byte chunks per activation row
 #pragma unroll 4
       for (int c = tid; c < BM * kChunksRow; c += Cf::kThreads) {
