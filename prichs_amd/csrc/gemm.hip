@@ -219,6 +219,8 @@ template <int BM_, int BN_, int WGM_, int WGN_, int S_ = PRICHS_BF16_STAGES> str
   static constexpr int BM = BM_, BN = BN_, BK = kBK, kStages = S_;
   static constexpr int WGM = WGM_, WGN = WGN_;
   static constexpr int kWaves = WGM * WGN;
+  // Four waves: the pipelined K loop of small tiles; eight: the ping-pong loop.
+  static constexpr bool kPipe = kWaves == 4;
   static constexpr int kThreads = 64 * kWaves;
   static constexpr int WM = BM / WGM, WN = BN / WGN;
   static constexpr int MI = WM / 16, NJ = WN / 16;
@@ -244,6 +246,7 @@ template <int BM_, int BN_, int WGM_, int WGN_, int S_ = PRICHS_BF16_STAGES> str
   static constexpr int kStgStride = BN + 8;
   static constexpr size_t kStgBytes = (size_t)BM * kStgStride * sizeof(bf16_t);
   static constexpr size_t kLdsBytes = kRingBytes > kStgBytes ? kRingBytes : kStgBytes;
+  static constexpr int kPerCu = kPipe && 2 * kLdsBytes <= 160 * 1024 ? 2 : 1;  // workgroups
   static_assert(WM % 16 == 0 && WN % 16 == 0, "whole fragments per wave");
   static_assert(kBlkA * kRowsPerInst == BM && kBlkB * kRowsPerInst == BN,
                 "the DMA instructions of one stage cover the A and B tiles exactly");
@@ -278,8 +281,11 @@ using Bf16Tall = Bf16Cfg<256, 288, 4, 2>;
 
 // 128 x 256 tiles (and 128 x 128 halves) for launches with too few rows to
 // fill the CUs with 256 x 256 ones: a prompt's or a micro-batch's experts
-// (mid_tiles in the launch code).
+// (grouped_tile_choice).
 using Bf16Mid = Bf16Cfg<128, 256, 2, 4>;
+// 64 x 128 tiles of 4 waves of 32 x 64 on the pipelined K loop, for launches
+// that even 128 x 128 tiles would not spread over the CUs.
+using Bf16Small = Bf16Cfg<64, 128, 2, 2, 6>;
 
 // C[m, n] = sum_k A[row(m), k] * B[n, k] for the rows of each group, with
 // B = packed weights [Np, K] of group g.  The MFMA takes the weight fragment
@@ -299,6 +305,18 @@ struct A2Rows {
   int g = -1, row0 = 0;
 };
 
+// One fragment read in front of each share of the MFMAs of a K-step.
+template <int READS, int MFMAS> __device__ __forceinline__ void interleave_mma() {
+#ifdef __HIP_DEVICE_COMPILE__
+  constexpr int kShare = MFMAS / READS > 0 ? MFMAS / READS : 1;
+#pragma unroll
+  for (int i = 0; i < READS; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
+    __builtin_amdgcn_sched_group_barrier(0x008, kShare, 0);
+  }
+#endif
+}
+
 // One output tile of the grouped GEMM: M-tile mt (global over the groups of
 // tm) and N-tile nt of width Cf::BN, computed by the whole workgroup.
 // DSW (down configurations only): the tile is dA of the MoE backward and its
@@ -316,8 +334,9 @@ __device__ __forceinline__ void bf16_tile(
   constexpr int WGN = Cf::WGN, WM = Cf::WM, WN = Cf::WN, MI = Cf::MI, NJ = Cf::NJ;
   constexpr int kRowsPerInst = Cf::kRowsPerInst, kInstA = Cf::kInstA, kInstB = Cf::kInstB;
   constexpr int kInstPerStage = Cf::kInstPerStage, kStageElems = Cf::kStageElems;
-  static_assert(Cf::kThreads == kBf16Threads, "launch bound of the bf16 kernels");
-  static_assert(Cf::kWaves == 8, "ping-pong K loop: two groups of 4 waves, one of each per SIMD");
+  static_assert(Cf::kThreads <= kBf16Threads, "launch bound of the bf16 kernels");
+  static_assert(Cf::kWaves == 8 || Cf::kPipe,
+                "ping-pong K loop: two groups of 4 waves, one of each per SIMD");
   static_assert(!(GATEUP && DSW), "the SwiGLU-backward epilogue is a down / dense mode");
   static_assert(!GATEUP || (WN % (2 * Cf::kIl) == 0 && BN % (2 * Cf::kIl) == 0),
                 "whole [gate | up] blocks per wave; packed gate/up rows padded to BN");
@@ -403,6 +422,82 @@ __device__ __forceinline__ void bf16_tile(
     for (int w = 0; w < kInstA + kInstB; ++w) issue_one(kt_, w);
   };
 
+  struct Frags {
+    bf16x8 w[NJ], a[MI];
+  };
+  auto read_frags = [&](Frags &F, int st) {
+    const bf16_t *as = lds + (st % kStages) * kStageElems;
+    const bf16_t *bs = as + BM * BK;
+#pragma unroll
+    for (int jj = 0; jj < NJ; ++jj)
+      F.w[jj] = *reinterpret_cast<const bf16x8 *>(bs + b_rd + jj * 16 * BK);
+#pragma unroll
+    for (int ii = 0; ii < MI; ++ii)
+      F.a[ii] = *reinterpret_cast<const bf16x8 *>(as + a_rd + ii * 16 * BK);
+  };
+  if constexpr (Cf::kPipe) {
+    // Pipelined K loop of the small tiles: a step is two K-steps of 32, the
+    // ring holds R = kStages / 2 steps, and each wave multiplies one K-step
+    // while its fragments of the next are read.  Per step one barrier, in
+    // front of the second half: there every wave has read all of step s (its
+    // slots take step s + R) and waited for its share of step s + 1.  A small
+    // ping-pong tile's phases would be as long as their LDS reads, which here
+    // run behind the products (down GEMM, 128 tokens: 14.4 us in 128 x 128
+    // ping-pong tiles, 10.4 in 64 x 128 pipelined ones).
+    constexpr int R = kStages / 2, kInst2 = 2 * kInstPerStage;
+    static_assert(kStages == 6 && Cf::kEvenA && Cf::kEvenB, "a ring of three steps");
+    const int NS = KT / 2;
+    Frags f0, f1;
+    for (int s_ = 0; s_ < R && s_ < NS; ++s_) {
+      issue_stage(2 * s_);
+      issue_stage(2 * s_ + 1);
+    }
+    if (NS >= 3)
+      PRICHS_WAIT_VMCNT(2 * kInst2);
+    else if (NS == 2)
+      PRICHS_WAIT_VMCNT(kInst2);
+    else
+      PRICHS_WAIT_VMCNT(0);
+    lds_barrier();
+    read_frags(f0, 0);
+    auto mma = [&](const Frags &F) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = mfma_bf16(F.w[j], F.a[i], acc[i][j]);
+    };
+    // Step s < NS - 1; FULL: steps s + 2 and s + R exist.
+    auto step = [&](int s_, auto full_c) {
+      constexpr bool kFull = decltype(full_c)::value;
+      read_frags(f1, 2 * s_ + 1);
+      mma(f0);
+      interleave_mma<MI + NJ, MI * NJ>();
+      __builtin_amdgcn_sched_barrier(0);
+      if (kFull || s_ + 2 < NS)
+        PRICHS_WAIT_VMCNT(kInst2);  // step s + 1 is here; s + 2 may be in flight
+      else
+        PRICHS_WAIT_VMCNT(0);
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): own reads of step s done
+      lds_barrier();
+      if (kFull || s_ + R < NS) {
+        issue_stage(2 * (s_ + R));
+        issue_stage(2 * (s_ + R) + 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      read_frags(f0, 2 * s_ + 2);
+      mma(f1);
+      interleave_mma<MI + NJ, MI * NJ>();
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    int s_ = 0;
+    for (; s_ + R < NS; ++s_) step(s_, bool_c<true>{});
+    for (; s_ + 1 < NS; ++s_) step(s_, bool_c<false>{});
+    read_frags(f1, 2 * s_ + 1);
+    mma(f0);
+    mma(f1);
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    lds_barrier();  // every wave is done reading the ring
+  } else {
   // Ping-pong K loop over a ring of S = kStages LDS stages, S - 1 of them in
   // flight.  Waves 0-3 (group 0) and 4-7 (group 1) sit one per SIMD each, so
   // every SIMD hosts one wave of each group.  Every wave runs the same
@@ -432,19 +527,7 @@ __device__ __forceinline__ void bf16_tile(
     lds_barrier();
     __builtin_amdgcn_sched_barrier(0);
   };
-  struct Frags {
-    bf16x8 w[NJ], a[MI];
-  } F;
-  auto read_frags = [&](int st) {
-    const bf16_t *as = lds + (st % kStages) * kStageElems;
-    const bf16_t *bs = as + BM * BK;
-#pragma unroll
-    for (int jj = 0; jj < NJ; ++jj)
-      F.w[jj] = *reinterpret_cast<const bf16x8 *>(bs + b_rd + jj * 16 * BK);
-#pragma unroll
-    for (int ii = 0; ii < MI; ++ii)
-      F.a[ii] = *reinterpret_cast<const bf16x8 *>(as + a_rd + ii * 16 * BK);
-  };
+  Frags F;
   constexpr int kMaxAhead = kStages - 2;  // own stages in flight after a step's wait
   for (int s_ = 0; s_ <= kMaxAhead && s_ < KT; ++s_) issue_stage(s_);
   wait_vmcnt(min(kMaxAhead, KT - 1) * kInstPerStage);  // own share of stage 0
@@ -458,7 +541,7 @@ __device__ __forceinline__ void bf16_tile(
   auto kstep = [&](int kt, auto ahead_c, auto first_c) {
     constexpr int kAhead = decltype(ahead_c)::value;
     constexpr bool kFirst = decltype(first_c)::value;
-    read_frags(kt);
+    read_frags(F, kt);
     if constexpr (kAhead == kMaxAhead) issue_stage(kt + kStages - 1);
     PRICHS_WAIT_VMCNT(kAhead * kInstPerStage);
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): own LDS reads done
@@ -491,6 +574,8 @@ __device__ __forceinline__ void bf16_tile(
   });
   if (kt < KT) kstep(kt++, A0{}, bool_c<false>{});
   if (grp == 0) pp_barrier();  // both groups leave after the same barrier count
+
+  }
 
   // Epilogue: acc[i][j][r] = C[row m0 + wm*WM + 16i + (lane & 15)]
   //                           [packed col n0 + wn*WN + 16j + 4*(lane >> 4) + r].
@@ -1352,10 +1437,10 @@ int gemm_cu_limit(int cus) {
 // still a whole number of B loads per wave; 128-wide tiles keep 64 columns per
 // wave, one [gate | up] block.  Not for 256 x 256 gate/up tiles: their whole
 // tiles run 0.3% slower with the second path compiled in, and launches that
-// would gain mostly take 128 x 256 tiles (mid_tiles).
+// would gain mostly take smaller tiles (grouped_tile_choice).
 template <class Cf, bool GATEUP>
 using TailCfg = typename std::conditional<
-    (Cf::BN / 2) % (Cf::kRowsPerInst * Cf::kWaves) != 0 || (GATEUP && Cf::BM == 256), Cf,
+    Cf::kPipe || (Cf::BN / 2) % (Cf::kRowsPerInst * Cf::kWaves) != 0 || (GATEUP && Cf::BM == 256), Cf,
     Bf16Cfg<Cf::BM, Cf::BN / 2, Cf::BN == 256 ? 4 : Cf::WGM, Cf::BN == 256 ? 2 : Cf::WGN,
             Cf::kStages>>::type;
 
@@ -1366,7 +1451,7 @@ template <class Cf, bool GATEUP>
 size_t bf16_grid(size_t max_rows, int G, int Np, int cus) {
   const bool halves = !std::is_same<Cf, TailCfg<Cf, GATEUP>>::value;
   const size_t ub = (max_rows / Cf::BM + G) * (size_t)(Np / Cf::BN) * (halves ? 2 : 1);
-  return std::max<size_t>(1, std::min<size_t>(ub, (size_t)gemm_cu_limit(cus)));
+  return std::max<size_t>(1, std::min<size_t>(ub, (size_t)gemm_cu_limit(cus) * Cf::kPerCu));
 }
 
 template <class Cf, bool GATEUP, bool DSW = false>
@@ -1421,12 +1506,13 @@ double launch_tile_times(size_t tiles, size_t grid, bool split) {
 // 124.7 us as 1024 wide tiles, 120.2 us as 768 square ones).  A 256 x 288
 // tile is 1.125 square tiles of work at the square tile's rate per flop.
 constexpr double kWideWork = 0.75, kWideRate = 0.96, kTallWork = 1.125;
-constexpr double kMidWork = 0.64;  // of a 128 x 256 tile (mid_tiles, below)
+// Of a 128 x 256 and a 64 x 128 tile (grouped_tile_choice, below).
+constexpr double kMidWork = 0.64, kSmallWork = 0.26;
 
 // Tile shape of a dense launch of M rows and Np packed columns: the one with
 // the fewest estimated square-tile-times on the grid launch_bf16 gives it
 // (0: 256 x 256 with half-width tails, 1: 128 x 384, 2: 256 x 288, 3: 128 x 256
-// with half-width tails).
+// with half-width tails, 4: 64 x 128).
 int dense_tile_choice(size_t M, size_t Np, int cus) {
   const size_t sq = ((M + Bf16Down::BM - 1) / Bf16Down::BM) * (Np / Bf16Down::BN);
   double best = launch_tile_times(sq, bf16_grid<Bf16Down, false>(M, 1, Np, cus), true);
@@ -1443,11 +1529,13 @@ int dense_tile_choice(size_t M, size_t Np, int cus) {
         launch_tile_times(tl, bf16_grid<Bf16Tall, false>(M, 1, Np, cus), false) * kTallWork;
     if (t < best) best = t, choice = 2;
   }
-  // 128 x 256 tiles where the rows are few (below, mid_tiles).
+  // 128 x 256 and 64 x 128 tiles where the rows are few (grouped_tile_choice).
   const size_t mid = ((M + Bf16Mid::BM - 1) / Bf16Mid::BM) * (Np / Bf16Mid::BN);
   const double t =
       launch_tile_times(mid, bf16_grid<Bf16Mid, false>(M, 1, Np, cus), true) * kMidWork;
-  if (t < best) choice = 3;
+  if (t < best) best = t, choice = 3;
+  const size_t small = ((M + Bf16Small::BM - 1) / Bf16Small::BM) * (Np / Bf16Small::BN);
+  if (kSmallWork * std::ceil((double)small / gemm_cu_limit(cus)) < best) choice = 4;
   return choice;
 }
 
@@ -1476,19 +1564,26 @@ double grouped_m_tiles(size_t BM, size_t max_rows, size_t max_group_rows, int G)
   return n * per + (shared ? (double)cdiv(max_group_rows, BM) : 0.0);
 }
 
-// Whether a grouped launch takes 128 x 256 tiles: one costs 0.64 of a 256 x
-// 256 tile (half the work; fewer products per byte staged), so they pay where
-// the large tiles leave the last or only round mostly empty.  Measured on
-// MI355X (d = 1536, f = 1280, 8 + 1 experts, top-2; 256 x 256 against 128 x
-// 256, us): gate/up 333 tokens 29.0 / 22.9, 512 33.0 / 31.3, 1500 47.9 / 53.5,
-// 3000 78.8 / 86.7, 8192 172 / 194; down 333 21.4 / 15.0, 777 22.1 / 21.2,
-// 1500 31.6 / 26.3, 3000 42.6 / 48.5, 8192 101 / 111; dX 512 48.6 / 37.2, 1000
-// 56.5 / 50.0, 2048 73.2 / 73.5, 8192 181 / 202.
-bool mid_tiles(bool gateup, size_t max_rows, size_t max_group_rows, int G, int Np, int cus) {
-  const double grid = gemm_cu_limit(cus), nt = Np / Bf16Mid::BN;
-  const double big = grouped_m_tiles(Bf16::BM, max_rows, max_group_rows, G) * nt;
-  const double mid = grouped_m_tiles(Bf16Mid::BM, max_rows, max_group_rows, G) * nt;
-  return kMidWork * grouped_tile_times(mid, grid, true) < grouped_tile_times(big, grid, !gateup);
+// Tile shape of a grouped launch: 0 = 256 x 256, 1 = 128 x 256, 2 = 64 x 128.
+// A 128 x 256 tile costs 0.64 of a 256 x 256 one (half the work; fewer products
+// per byte staged), a 64 x 128 tile 0.26 (an eighth), so they pay where the
+// larger tiles leave the last or only round mostly empty.  Measured on MI355X
+// (d = 1536, f = 1280, 8 + 1 experts, top-2; 256 x 256 / 128 x 256 / 64 x 128,
+// us): gate/up 128 tokens 33.8 / 22.1 / 17.1, 333 31.5 / 22.3 / 23.0, 512 39.4
+// / 31.3 / 33.8, 1500 47.7 / 53.1 / 65.8, 8192 172 / 194; down 128 tokens 16.9 /
+// 14.4 / 10.4, 333 21.1 / 14.8 / 16.6, 777 21.6 / 21.4 / 20.4, 1500 31.2 / 23.9
+// / 35.7, 3000 42.6 / 48.5, 8192 101 / 111; dX 777 51.1 / 45.2 / 40.9, 1000
+// 55.8 / 50.0 / 64.2, 2048 72.2 / 68.4 / 96.9.
+int grouped_tile_choice(bool gateup, size_t max_rows, size_t max_group_rows, int G, int Np,
+                        int cus) {
+  const double grid = gemm_cu_limit(cus);
+  auto tiles = [&](size_t bm, size_t bn) {
+    return grouped_m_tiles(bm, max_rows, max_group_rows, G) * (double)(Np / bn);
+  };
+  const double big = grouped_tile_times(tiles(Bf16::BM, Bf16::BN), grid, !gateup);
+  const double mid = kMidWork * grouped_tile_times(tiles(Bf16Mid::BM, Bf16Mid::BN), grid, true);
+  const double small = kSmallWork * std::ceil(tiles(Bf16Small::BM, Bf16Small::BN) / grid);
+  return small < mid && small < big ? 2 : mid < big ? 1 : 0;
 }
 
 template <bool GATEUP, int U, int SK>
@@ -1562,13 +1657,17 @@ int launch_grouped(bool gateup, const void *A, const int32_t *a_rows, int lda, c
   const int cus = device_cu_count();
   if (cus <= 0) return fail(PRICHS_ERR_HIP, "grouped gemm: cannot query the device");
   if (dtype == PRICHS_DTYPE_BF16) {
-    const bool mid = offsets != nullptr && mid_tiles(gateup, max_rows, max_group_rows, G, Np, cus);
+    const int few = offsets == nullptr
+                        ? 0
+                        : grouped_tile_choice(gateup, max_rows, max_group_rows, G, Np, cus);
     if (gateup) {
-      auto run = mid ? &launch_bf16<Bf16Mid, true> : &launch_bf16<Bf16, true>;
+      auto run = few == 2   ? &launch_bf16<Bf16Small, true>
+                 : few == 1 ? &launch_bf16<Bf16Mid, true>
+                            : &launch_bf16<Bf16, true>;
       return run(A, a_rows, lda, B, b_stride, Np, K, Cp, ldc, n_store, offsets, G, dense_m,
                  max_rows, cus, s, pre, A2Rows());
     }
-    const int shape = offsets != nullptr ? (mid ? 3 : 0)
+    const int shape = offsets != nullptr ? (few > 0 ? 2 + few : 0)
                                          : dense_tile_choice((size_t)dense_m, (size_t)Np, cus);
     if (shape == 1)
       return launch_bf16<Bf16Wide, false>(A, a_rows, lda, B, b_stride, Np, K, Cp, ldc, n_store,
@@ -1579,6 +1678,9 @@ int launch_grouped(bool gateup, const void *A, const int32_t *a_rows, int lda, c
     if (shape == 3)
       return launch_bf16<Bf16Mid, false>(A, a_rows, lda, B, b_stride, Np, K, Cp, ldc, n_store,
                                          offsets, G, dense_m, max_rows, cus, s, nullptr);
+    if (shape == 4)
+      return launch_bf16<Bf16Small, false>(A, a_rows, lda, B, b_stride, Np, K, Cp, ldc, n_store,
+                                           offsets, G, dense_m, max_rows, cus, s, nullptr);
     return launch_bf16<Bf16Down, false>(A, a_rows, lda, B, b_stride, Np, K, Cp, ldc, n_store,
                                         offsets, G, dense_m, max_rows, cus, s, nullptr);
   } else {
@@ -1791,9 +1893,11 @@ int grouped_dact_swiglu_bwd(const void *dy, size_t d, const void *w_down_t, size
     alt.row0 = (int)a2_row0;
   }
   *fused = true;
-  auto run = mid_tiles(false, max_rows, std::min(max_rows, max_group_rows), (int)G, (int)np_f, cus)
-                 ? &launch_bf16<Bf16Mid, false, true>
-                 : &launch_bf16<Bf16Down, false, true>;
+  const int few = grouped_tile_choice(false, max_rows, std::min(max_rows, max_group_rows), (int)G,
+                                      (int)np_f, cus);
+  auto run = few == 2   ? &launch_bf16<Bf16Small, false, true>
+             : few == 1 ? &launch_bf16<Bf16Mid, false, true>
+                        : &launch_bf16<Bf16Down, false, true>;
   return run(dy, nullptr, (int)d, w_down_t, (long long)b_group_stride, (int)np_f, (int)d, nullptr,
              (int)np, (int)f, offsets, (int)G, 0, max_rows, cus, as_stream(stream), gu, alt);
 }

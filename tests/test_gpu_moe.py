@@ -205,11 +205,13 @@ def test_gate_up_unaligned_output_bit_identical(cuda):
 
 
 # Launches with few rows take 128 x 256 tiles (whole ones, or all as 128 x 128
-# halves where those fill at most half the CUs): ragged, empty, one-row and
+# halves where those fill at most half the CUs) or 64 x 128 ones: ragged, empty, one-row and
 # exactly full groups.  The extra group of the second launch makes the same
 # rows take 256 x 256 tiles; every output element is one MFMA chain over K, so
 # the shared rows agree bit for bit.
 @pytest.mark.parametrize("d,f,counts", [(1536, 1280, [83, 0, 129, 300, 1]),      # halves
+                                        (1536, 1280, [64, 0, 65, 1, 63, 70]),     # 64 x 128
+                                        (64, 192, [100, 33]),      # 64 x 128, 1 and 3 K-steps
                                         (1536, 1280, [256, 128, 700, 384, 513]),  # whole
                                         (320, 192, [65, 255, 1000])])
 @pytest.mark.parametrize("aligned", [True, False])
@@ -237,7 +239,7 @@ def test_mid_tiles_bit_identical(cuda, orc, d, f, counts, aligned):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
     h_act, h_y = host(got[0][0]), host(got[0][1])
     o = np.concatenate([[0], np.cumsum(counts)])
-    for g in (2, G - 1):  # against the oracle: two groups
+    for g in (G // 2, G - 1):  # against the oracle: two groups
         r = slice(o[g], o[g + 1])
         xr = host(x[row_token[r].long()])
         a_ref = orc.swiglu(orc.matmul_2d(xr, w[g % 2]), orc.matmul_2d(xr, w[(g + 1) % 3]))
