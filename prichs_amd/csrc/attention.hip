@@ -36,6 +36,7 @@
 // lane i that column's 4 consecutive kv values.
 #include "common.hpp"
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -155,14 +156,15 @@ __device__ __forceinline__ bf16x8 rope_frag(bf16x8 f, float4 c4, float4 s4) {
   return __builtin_bit_cast(bf16x8, u);
 }
 
-template <int HPW>
+// NB: 16-row query blocks per wave.
+template <int HPW, int NB>
 __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(
     const bf16_t *__restrict__ q, int ldq, const bf16_t *__restrict__ k, int ldk,
     const bf16_t *__restrict__ v, int ldv, bf16_t *__restrict__ o, int ldo, int S, int Hq,
     int group, float scale_log2, const float *__restrict__ rcos, const float *__restrict__ rsin,
     int pos_offset) {
   static_assert(kWaves % HPW == 0, "whole row blocks per head");
-  constexpr int kRowsWg = 32 * kWaves / HPW;  // query rows per workgroup
+  constexpr int kRowsWg = 16 * NB * kWaves / HPW;  // query rows per workgroup
   extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
 
   // Grid (head set, sequence, query block): blocks are dispatched x-fastest,
@@ -183,13 +185,13 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(
   const bf16_t *kbase = k + seq0 * ldk + (size_t)kvh * kHd;
   const bf16_t *vbase = v + seq0 * ldv + (size_t)kvh * kHd;
 
-  // Query rows of this wave: q0 + 16*nb + l16 (nb = 0, 1).
-  const int q0 = qb * kRowsWg + (wave / HPW) * 32;
+  // Query rows of this wave: q0 + 16*nb + l16 (nb < NB).
+  const int q0 = qb * kRowsWg + (wave / HPW) * 16 * NB;
 
   // Q fragments (B operand of S^T = K Q^T): lane holds Q[q][32kk + 8g .. +8].
-  bf16x8 qf[2][4];
+  bf16x8 qf[NB][4];
 #pragma unroll
-  for (int nb = 0; nb < 2; ++nb) {
+  for (int nb = 0; nb < NB; ++nb) {
     int qr = q0 + 16 * nb + l16;
     qr = qr < S ? qr : S - 1;
     const bf16_t *qrow = q + (seq0 + qr) * ldq + (size_t)h * kHd + 8 * g;
@@ -205,18 +207,23 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(
     }
   }
 
-  f32x4 oacc[8][2];  // O^T blocks: d block jd, query block nb
+  f32x4 oacc[8][NB];  // O^T blocks: d block jd, query block nb
 #pragma unroll
   for (int jd = 0; jd < 8; ++jd)
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) oacc[jd][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int nb = 0; nb < NB; ++nb) oacc[jd][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
   // Reference max (log2 units) of row q: p = exp2(s - m_ref).  It is only
   // raised when a block's max exceeds it by more than kLazy, so p <= 2^kLazy
   // and the output rows are rescaled a few times per row, not per block.
-  float m_ref[2] = {-INFINITY, -INFINITY};
+  float m_ref[NB];
   // Row sums of P, accumulated by MFMA against a ones fragment (every element
   // of lsum[nb] holds the sum of query row q0 + 16 nb + lane % 16).
-  f32x4 lsum[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+  f32x4 lsum[NB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) {
+    m_ref[nb] = -INFINITY;
+    lsum[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
   const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u,
                                                         0x3f803f80u});
 
@@ -277,13 +284,13 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(
     __syncthreads();
   };
 
-  // S^T = K Q^T of block kb: 4 kv blocks x 2 query blocks; sacc[c][nb][r] =
+  // S^T = K Q^T of block kb: 4 kv blocks x NB query blocks; sacc[c][nb][r] =
   // raw score of (query q0 + 16nb + l16, kv 64 kb + 16c + 4g + r).
-  auto compute_s = [&](int kb, f32x4 (&sacc)[4][2]) {
+  auto compute_s = [&](int kb, f32x4 (&sacc)[4][NB]) {
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb) sacc[c][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int nb = 0; nb < NB; ++nb) sacc[c][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
     const char *kbytes = reinterpret_cast<const char *>(lds) + (uint32_t)(kb & 1) * kStageBytes;
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
@@ -294,7 +301,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(
 #pragma unroll
       for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) sacc[c][nb] = mfma_bf16(kf[c], qf[nb][kk], sacc[c][nb]);
+        for (int nb = 0; nb < NB; ++nb) sacc[c][nb] = mfma_bf16(kf[c], qf[nb][kk], sacc[c][nb]);
     }
   };
 
@@ -302,7 +309,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(
   // stale tile it reads gives a result nobody uses), then the softmax and
   // P.V of block kb from scur.  MASKED applies the causal / length mask
   // (blocks reaching past this wave's first query row or the sequence end).
-  auto run_iter = [&](int kb, auto masked_c, f32x4 (&scur)[4][2], f32x4 (&snext)[4][2]) {
+  auto run_iter = [&](int kb, auto masked_c, f32x4 (&scur)[4][NB], f32x4 (&snext)[4][NB]) {
     constexpr bool kMasked = decltype(masked_c)::value;
     const int kv0 = kb * kBKV;
     // K of block kb + 1 and V of block kb have landed; the buffers of K kb
@@ -316,11 +323,11 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(
     // Online softmax.  The block max is taken on raw scores (the scale is
     // positive, and rounding is monotone, so max(fl(s * c)) = fl(max(s) * c))
     // and p = exp2(s * scale_log2 - m_ref) is one fma per score.
-    u32x4 pf[2][2];  // P fragments: [nb][32-row kv step]
-    float alpha[2];
-    bool raise[2];
+    u32x4 pf[NB][2];  // P fragments: [nb][32-row kv step]
+    float alpha[NB];
+    bool raise[NB];
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) {
+    for (int nb = 0; nb < NB; ++nb) {
       if constexpr (kMasked) {
         // Valid iff kv <= query row and kv < S, i.e. 16c + r <= lim.
         const int lim = min(q0 + 16 * nb + l16, S - 1) - kv0 - 4 * g;
@@ -362,11 +369,12 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(
     }
     // Pin the P fragments here: otherwise the compiler sinks the exp work
     // past the branch below, out of reach of the S MFMAs it should overlap.
-    asm volatile("" ::"v"(pf[0][0]), "v"(pf[0][1]), "v"(pf[1][0]), "v"(pf[1][1]));
-    // Rescale the output rows where the reference max was raised (rare).
-    if (__any(raise[0] || raise[1])) {
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb) {
+    for (int nb = 0; nb < NB; ++nb) asm volatile("" ::"v"(pf[nb][0]), "v"(pf[nb][1]));
+    // Rescale the output rows where the reference max was raised (rare).
+    if (__any(raise[0] || raise[NB - 1])) {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
         for (int jd = 0; jd < 8; ++jd) oacc[jd][nb] = oacc[jd][nb] * alpha[nb];
         lsum[nb] = lsum[nb] * alpha[nb];
@@ -396,13 +404,13 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(
         for (int t = 0; t < 4; ++t) {
           const bf16x8 vf = __builtin_bit_cast(bf16x8, u32x4{lo[t][0], lo[t][1], hi[t][0], hi[t][1]});
 #pragma unroll
-          for (int nb = 0; nb < 2; ++nb)
+          for (int nb = 0; nb < NB; ++nb)
             oacc[j0 + t][nb] =
                 mfma_bf16(vf, __builtin_bit_cast(bf16x8, pf[nb][ks2]), oacc[j0 + t][nb]);
         }
       }
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb)
+      for (int nb = 0; nb < NB; ++nb)
         lsum[nb] = mfma_bf16(ones, __builtin_bit_cast(bf16x8, pf[nb][ks2]), lsum[nb]);
     });
   };
@@ -412,7 +420,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(
   // registers swap roles without copies); the rest (the diagonal and the
   // ragged tail) run masked.
   const int n_full = min(min(q0 + 1, S) / kBKV, n_kvb);
-  f32x4 sa[4][2], sb[4][2];
+  f32x4 sa[4][NB], sb[4][NB];
   issue_k(0);
   sync_tiles();
   issue_v(0);
@@ -427,7 +435,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb) sa[c][nb] = sb[c][nb];
+      for (int nb = 0; nb < NB; ++nb) sa[c][nb] = sb[c][nb];
   };
   if (kb < n_full) {
     run_iter(kb, bool_c<false>{}, sa, sb);
@@ -441,7 +449,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(
 
   // Normalise by the row sum and store: lane holds O[q][16 jd + 4g + r].
 #pragma unroll
-  for (int nb = 0; nb < 2; ++nb) {
+  for (int nb = 0; nb < NB; ++nb) {
     const float inv = 1.0f / fmaxf(lsum[nb][0], 1e-30f);
     const int qrow = q0 + 16 * nb + l16;
     if (qrow < S) {
@@ -497,12 +505,27 @@ int attention_forward_impl(const void *q, size_t ldq, const void *k, size_t ldk,
   const int group = (int)(n_heads / n_kv_heads);
   // Heads per workgroup: the largest of 4, 2, 1 dividing the GQA group.
   const int hpw = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
-  const int rows_wg = 32 * kWaves / hpw;
-  const int n_qb = (int)cdiv(seq_len, (size_t)rows_wg);
+  int n_qb = (int)cdiv(seq_len, (size_t)(32 * kWaves / hpw));
   const float scale_log2 = (1.0f / sqrtf((float)head_dim)) * 1.4426950408889634f;
   PRICHS_REQUIRE(n_qb <= 65535, "attention: seq_len too large");
+  // 16 query rows per wave instead of 32 where the workgroups would all be
+  // resident with room to spare (two fit a CU): each walks its causal K / V
+  // blocks one after the other, and half the products and exponentials per
+  // block shorten that chain; beyond, they only read every K / V tile twice as
+  // often.  The same operations per row, so the same bits.  MI355X, 12 + 3
+  // heads, 32 -> 16 rows, us: 1 x 333 11.2 -> 9.1, 1 x 777 19.1 -> 13.5, 1 x
+  // 2048 41.2 -> 31.0, 4 x 1024 (384 workgroups) 26.6 -> 24.1, 4 x 2048 (768)
+  // 60.3 -> 69.8.
+  const int cus = device_cu_count();
+  const bool few = 2 * (n_heads / hpw) * batch * (size_t)n_qb <= 3 * (size_t)std::max(cus, 0);
+  if (few) n_qb = (int)cdiv(seq_len, (size_t)(16 * kWaves / hpw));
   const dim3 grid((unsigned)(n_heads / hpw), (unsigned)batch, (unsigned)n_qb);
-  auto kern = hpw == 4 ? attn_fwd_kernel<4> : hpw == 2 ? attn_fwd_kernel<2> : attn_fwd_kernel<1>;
+  auto kern = few ? (hpw == 4   ? attn_fwd_kernel<4, 1>
+                     : hpw == 2 ? attn_fwd_kernel<2, 1>
+                                : attn_fwd_kernel<1, 1>)
+                  : (hpw == 4   ? attn_fwd_kernel<4, 2>
+                     : hpw == 2 ? attn_fwd_kernel<2, 2>
+                                : attn_fwd_kernel<1, 2>);
   hipLaunchKernelGGL(kern, grid, dim3(kThreads), kLdsBytes, as_stream(stream),
                      static_cast<const bf16_t *>(q), (int)ldq, static_cast<const bf16_t *>(k),
                      (int)ldk, static_cast<const bf16_t *>(v), (int)ldv,

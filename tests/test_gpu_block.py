@@ -189,6 +189,26 @@ def test_attention_kernel(cuda, B, S, Hq, Hkv):
         assert rel_err(got, r) <= 2e-2, (b, h)
 
 
+# Few workgroups take 16 query rows per wave, many 32 (1, 2 or 4 heads per
+# workgroup; query rows ending inside a wave's block, one row, K / V ending
+# inside a block): the same operations per row, so a sequence alone gives the
+# bits it gives in a large batch.
+@pytest.mark.parametrize("S,Hq,Hkv", [(1, 4, 1), (33, 4, 1), (257, 8, 2), (100, 2, 1),
+                                      (145, 4, 2), (64, 1, 1), (81, 3, 3)])
+def test_attention_rows_per_wave_bit_identical(cuda, S, Hq, Hkv):
+    n, many = (Hq + 2 * Hkv) * 128, 800  # 800 sequences are at least 400 workgroups
+    rng = np.random.default_rng(S + Hq)
+    one = dev(synth.round_bf16(rng.standard_normal((S, n)) * 0.7))
+    say("attention rows per wave", S, Hq, Hkv)
+    outs = []
+    for b in (1, many):
+        x = one.repeat(b, 1)
+        q, k, v = x[:, :Hq * 128], x[:, Hq * 128:(Hq + Hkv) * 128], x[:, (Hq + Hkv) * 128:]
+        outs.append(ops.attention(q, k, v, b, S, Hq, Hkv))
+    assert torch.equal(outs[0], outs[1][:S])
+    assert torch.equal(outs[0], outs[1][-S:])
+
+
 def test_attention_kernel_config5_shape(cuda):
     # 4 sequences x 2048, 12 query heads on 3 kv heads; sampled (b, h) checked.
     B, S, Hq, Hkv, hd = 4, 2048, 12, 3, 128
