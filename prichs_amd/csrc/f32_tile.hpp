@@ -28,7 +28,7 @@
 // with one of them in front of each share of the MFMAs (no branch in a whole
 // stage, sched_group_barrier) 253-260 us, 134 of the 154 TFLOP/s that MFMAs
 // alone reach.  2048 x 1280 x 1536: 196 us (64 x 64 tiles, 4-byte checked
-// loads, one LDS buffer) -> 75 us.
+// loads, one LDS buffer) -> 71 us.
 //
 // WGK > 1: that many waves share an output block and split each stage's
 // 16-element slices; their sums are added in wave order through LDS at the

@@ -16,6 +16,7 @@
 #include <cmath>
 #include <mutex>
 #include <new>
+#include <type_traits>
 
 #include "common.hpp"
 #include "f32_tile.hpp"
@@ -37,20 +38,16 @@ using f32t::f32x4;
 //   OP 0 (A B):    opA(i, r) = A[i R + r],  opB(r, j) = B[r N + j]
 //   OP 1 (A^T B):  opA(i, r) = A[r M + i],  opB(r, j) = B[r N + j]
 //   OP 2 (A B^T):  opA(i, r) = A[i R + r],  opB(r, j) = B[j R + r]
-// One workgroup per tile; tiles in bands of 4 tile rows, column by column in
-// a band, each XCD taking a contiguous run of them.  Rows and columns past
-// the matrix read its last ones and are not stored.
+// Tiles in bands of 4 tile rows, column by column in a band, each XCD taking a
+// contiguous run of them.  Rows and columns past the matrix read its last ones
+// and are not stored.
 template <class T, int OP>
-__global__ __launch_bounds__(T::kThreads) void f32_matmul_kernel(
-    const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, long long M,
-    long long N, long long R, unsigned m_tiles, unsigned n_tiles, int vec_c) {
-  __shared__ __attribute__((aligned(16))) float lds[T::kLdsFloats];
+__device__ __forceinline__ void f32_matmul_tile(float *lds, const float *__restrict__ A,
+                                                const float *__restrict__ B,
+                                                float *__restrict__ C, long long M, long long N,
+                                                long long R, long long m0, long long n0,
+                                                int vec_c) {
   const int t = threadIdx.x;
-  const unsigned id = f32t::xcd_run(blockIdx.x, gridDim.x);
-  const unsigned band = id / n_tiles / 4, in = id - band * 4 * n_tiles;
-  const unsigned rows = min(4u, m_tiles - band * 4);
-  const long long m0 = (long long)(band * 4 + in % rows) * T::BM;
-  const long long n0 = (long long)(in / rows) * T::BN;
   T tile(t);
   typename T::OpA oa;
   typename T::OpB ob;
@@ -82,12 +79,41 @@ __global__ __launch_bounds__(T::kThreads) void f32_matmul_kernel(
     }
 }
 
+// One workgroup per tile.  Tiles n_full .. are computed as two half-height
+// tiles (TH) each, on two workgroups: the last partial round of a launch.
+// TH = T: no halves (n_full is the number of tiles).
+template <class T, class TH, int OP>
+__global__ __launch_bounds__(T::kThreads) void f32_matmul_kernel(
+    const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, long long M,
+    long long N, long long R, unsigned m_tiles, unsigned n_tiles, unsigned n_full, int vec_c) {
+  static_assert(T::kThreads == TH::kThreads && T::BN == TH::BN, "one launch for both");
+  __shared__ __attribute__((aligned(16))) float
+      lds[T::kLdsFloats > TH::kLdsFloats ? T::kLdsFloats : TH::kLdsFloats];
+  const bool half = blockIdx.x >= n_full;
+  const unsigned run = half ? n_full + f32t::xcd_run(blockIdx.x - n_full, gridDim.x - n_full) / 2
+                            : f32t::xcd_run(blockIdx.x, n_full);
+  const unsigned band = run / n_tiles / 4, in = run - band * 4 * n_tiles;
+  const unsigned rows = min(4u, m_tiles - band * 4);
+  const long long m0 = (long long)(band * 4 + in % rows) * T::BM;
+  const long long n0 = (long long)(in / rows) * T::BN;
+  if constexpr (!std::is_same<T, TH>::value) {
+    if (half) {
+      const unsigned u = f32t::xcd_run(blockIdx.x - n_full, gridDim.x - n_full);
+      const long long mh = m0 + (u & 1) * TH::BM;
+      if (mh < M) f32_matmul_tile<TH, OP>(lds, A, B, C, M, N, R, mh, n0, vec_c);
+      return;
+    }
+  }
+  f32_matmul_tile<T, OP>(lds, A, B, C, M, N, R, m0, n0, vec_c);
+}
+
 // The tile shapes, from large outputs to outputs of a few tiles with a long
 // reduction (waves m x n x k: the last split the reduction).
 template <int CFG, int OP, int W> struct MatmulCfg;
 #define PRICHS_MATMUL_CFG(I, BM, BN, BK, WM, WN, WK)                                      \
   template <int OP, int W> struct MatmulCfg<I, OP, W> {                                   \
     typedef f32t::Tile<BM, BN, BK, WM, WN, WK, OP != 1, OP == 2, W> T;                    \
+    typedef T TH;                                                                         \
   };
 PRICHS_MATMUL_CFG(0, 128, 128, 32, 2, 2, 1)
 PRICHS_MATMUL_CFG(1, 64, 64, 64, 2, 2, 2)
@@ -95,6 +121,11 @@ PRICHS_MATMUL_CFG(2, 32, 64, 64, 1, 2, 2)
 PRICHS_MATMUL_CFG(3, 32, 32, 64, 2, 2, 2)
 PRICHS_MATMUL_CFG(4, 16, 16, 256, 1, 1, 8)
 #undef PRICHS_MATMUL_CFG
+// 64 x 64 tiles with the last partial round as 32 x 64 halves.
+template <int OP, int W> struct MatmulCfg<5, OP, W> {
+  typedef f32t::Tile<64, 64, 32, 2, 2, 1, OP != 1, OP == 2, W> T;
+  typedef f32t::Tile<32, 64, 64, 1, 2, 2, OP != 1, OP == 2, W> TH;
+};
 constexpr int kMatmulCfgs = 5;
 
 // Nanoseconds per reduction element of one tile on a CU: alone, and each of
@@ -115,6 +146,16 @@ constexpr MatmulTileCost kMatmulCost[kMatmulCfgs] = {
     {16, 16, 256, {2.5, 5.7}, {2.6, 10.0}},
 };
 
+// Configuration 5: a last partial round of at most half the CUs in half tiles
+// (2048 x 1280 x 1536: 640 tiles are 2.5 rounds, 71.0 us against 75.0 in 32
+// x 64 tiles and 83 in whole 64 x 64 ones).
+constexpr double kMatmulWhole = 17.6, kMatmulHalf = 9.8;
+bool matmul_halves(size_t M, size_t N, int cus, size_t &full) {
+  const size_t tiles = cdiv(M, 64) * cdiv(N, 64), tail = tiles % (size_t)cus;
+  full = tiles - tail;
+  return full > 0 && tail > 0 && 2 * tail <= (size_t)cus;
+}
+
 int matmul_cfg(size_t M, size_t N, size_t R, bool vec, int cus) {
   int best = 0;
   double best_t = 0;
@@ -126,6 +167,10 @@ int matmul_cfg(size_t M, size_t N, size_t R, bool vec, int cus) {
     const double t = (double)roundup(R, k.bk) * std::max(k.alone[!vec], rounds * k.shared[!vec]);
     if (c == 0 || t < best_t) best = c, best_t = t;
   }
+  size_t full = 0;
+  if (vec && matmul_halves(M, N, cus, full) &&
+      (double)roundup(R, 32) * ((double)(full / cus) * kMatmulWhole + kMatmulHalf) < best_t)
+    best = 5;
   return best;
 }
 
@@ -163,9 +208,14 @@ template <int CFG, int OP, int W>
 void launch_matmul_kernel(const float *a, const float *b, float *c, const MatmulDims &d, int vec_c,
                           hipStream_t s) {
   typedef typename MatmulCfg<CFG, OP, W>::T T;
+  typedef typename MatmulCfg<CFG, OP, W>::TH TH;
   const unsigned mt = (unsigned)cdiv(d.M, T::BM), nt = (unsigned)cdiv(d.N, T::BN);
-  hipLaunchKernelGGL((f32_matmul_kernel<T, OP>), dim3(mt * nt), dim3(T::kThreads), 0, s, a, b, c,
-                     (long long)d.M, (long long)d.N, (long long)d.R, mt, nt, vec_c);
+  size_t full = (size_t)mt * nt;
+  if (!std::is_same<T, TH>::value) matmul_halves(d.M, d.N, device_cu_count(), full);
+  const unsigned grid = (unsigned)(full + 2 * ((size_t)mt * nt - full));
+  hipLaunchKernelGGL((f32_matmul_kernel<T, TH, OP>), dim3(grid), dim3(T::kThreads), 0, s, a, b, c,
+                     (long long)d.M, (long long)d.N, (long long)d.R, mt, nt, (unsigned)full,
+                     vec_c);
 }
 
 template <int OP, int W>
@@ -176,6 +226,7 @@ void launch_matmul_cfg(int cfg, const float *a, const float *b, float *c, const 
     case 1: return launch_matmul_kernel<1, OP, W>(a, b, c, d, vec_c, s);
     case 2: return launch_matmul_kernel<2, OP, W>(a, b, c, d, vec_c, s);
     case 3: return launch_matmul_kernel<3, OP, W>(a, b, c, d, vec_c, s);
+    case 5: return launch_matmul_kernel<W == 4 ? 5 : 4, OP, W>(a, b, c, d, vec_c, s);
     default: return launch_matmul_kernel<4, OP, W>(a, b, c, d, vec_c, s);
   }
 }

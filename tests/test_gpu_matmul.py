@@ -199,6 +199,7 @@ def test_matmul_device_entry_on_stream_and_big_reduction(cuda, orc):
 @pytest.mark.parametrize("M,N,R", [(2044, 2040, 36), (1999, 2001, 33),    # 128 x 128
                                    (1000, 1020, 100), (1001, 777, 101),   # 64 x 64
                                    (1272, 1000, 68), (500, 1001, 69),     # 32 x 64
+                                   (1156, 1152, 100), (1220, 1084, 36),   # 64 x 64, tail in halves
                                    (300, 500, 132), (300, 301, 69),       # 32 x 32
                                    (36, 68, 260), (17, 45, 257)])         # 16 x 16
 @pytest.mark.parametrize("op", [L.MATMUL_AB, L.MATMUL_ATB, L.MATMUL_ABT],
