@@ -1013,21 +1013,27 @@ __global__ __launch_bounds__(256) void combine_kernel(
 // engine.rs:2705-2789).  d_logits[t][e] is zero unless t selected e, so
 // column e is a weighted sum over expert e's rows of the row space:
 // dW[:, e] += sum over rows r of group e of dlr[r] * xg[r] (xg = x gathered
-// by row, written by the rows pass).  Pass 1: one workgroup per chunk of
-// kRouterChunk rows of one group (chunks numbered group by group) writes
-// part[chunk][c]; pass 2 adds each group's chunks in ascending order.
-constexpr int kRouterChunk = 64;
+// by row, written by the rows pass).  Pass 1: one workgroup per chunk of rows
+// of one group (chunks numbered group by group) writes part[chunk][c]; pass 2
+// adds each group's chunks in ascending order.
+// Rows per chunk for `rows` routed rows: short enough that the first pass has
+// workgroups for the CUs (a chunk is a chain of load batches), long enough that
+// the second pass adds few chunks.  Both passes, MI355X, d = 1536, 64-row
+// chunks -> these: 2000 rows 14.5 -> 10.8 us, 4096 14.6 -> 13.1, 8192 15.7 ->
+// 15.0; 16384 rows take 17.8 with 64-row chunks and 20.4 with 32.
+size_t router_chunk_rows(size_t rows) { return rows <= 4096 ? 16 : rows <= 8192 ? 32 : 64; }
 constexpr int kRouterUnroll = 8;  // rows whose loads are in flight together
 
 // Group and row range of chunk `ch` (-1 past the last chunk); offsets in LDS.
-__device__ inline int router_chunk(const int *offsets, int E, int ch, int &r0, int &r1) {
+__device__ inline int router_chunk(const int *offsets, int E, int chunk, int ch, int &r0,
+                                   int &r1) {
   int first = 0;
   for (int e = 0; e < E; ++e) {
     const int lo = offsets[e], hi = offsets[e + 1];
-    const int n = (hi - lo + kRouterChunk - 1) / kRouterChunk;
+    const int n = (hi - lo + chunk - 1) / chunk;
     if (ch < first + n) {
-      r0 = lo + (ch - first) * kRouterChunk;
-      r1 = min(r0 + kRouterChunk, hi);
+      r0 = lo + (ch - first) * chunk;
+      r1 = min(r0 + chunk, hi);
       return e;
     }
     first += n;
@@ -1039,14 +1045,14 @@ template <typename T>
 __global__ __launch_bounds__(256) void router_wgrad_part_kernel(const T *__restrict__ xg,
                                                                 const float *__restrict__ dlr,
                                                                 const int32_t *__restrict__ offsets,
-                                                                int E, int d,
+                                                                int E, int d, int chunk,
                                                                 float *__restrict__ part) {
 #pragma clang fp contract(off)
   __shared__ int offs_s[PRICHS_MAX_EXPERTS + 1];
   if ((int)threadIdx.x <= E) offs_s[threadIdx.x] = offsets[threadIdx.x];
   __syncthreads();
   int r0 = 0, r1 = 0;
-  if (router_chunk(offs_s, E, blockIdx.x, r0, r1) < 0) return;
+  if (router_chunk(offs_s, E, chunk, blockIdx.x, r0, r1) < 0) return;
   for (int c = threadIdx.x * 8; c < d; c += 256 * 8) {
     float acc[8];
 #pragma unroll
@@ -1073,7 +1079,8 @@ __global__ __launch_bounds__(256) void router_wgrad_part_kernel(const T *__restr
 
 __global__ __launch_bounds__(256) void router_wgrad_reduce_kernel(const float *__restrict__ part,
                                                                   const int32_t *__restrict__ offsets,
-                                                                  int E, int d, int beta,
+                                                                  int E, int d, int chunk,
+                                                                  int beta,
                                                                   float *__restrict__ dw) {
 #pragma clang fp contract(off)
   __shared__ int offs_s[PRICHS_MAX_EXPERTS + 1];
@@ -1086,8 +1093,8 @@ __global__ __launch_bounds__(256) void router_wgrad_reduce_kernel(const float *_
   const int e = i / d, c = i - e * d;
   int first = 0;
   for (int g = 0; g < e; ++g)
-    first += (offs_s[g + 1] - offs_s[g] + kRouterChunk - 1) / kRouterChunk;
-  const int n = (offs_s[e + 1] - offs_s[e] + kRouterChunk - 1) / kRouterChunk;
+    first += (offs_s[g + 1] - offs_s[g] + chunk - 1) / chunk;
+  const int n = (offs_s[e + 1] - offs_s[e] + chunk - 1) / chunk;
   float s = 0.f;
   for (int ch = 0; ch < n; ch += 16) {
     float v[16];
@@ -1397,7 +1404,13 @@ int bwd_zero_grads(float *d_router, size_t n_router, float *d_gate, float *d_up,
 }
 
 size_t bwd_router_part_elems(size_t max_tokens, size_t k, size_t d, size_t E) {
-  return (cdiv(max_tokens * k, kRouterChunk) + E) * d;
+  // The most chunks that any batch of up to max_tokens has.
+  size_t n = 0;
+  for (size_t rows : {(size_t)4096, (size_t)8192, max_tokens * k}) {
+    rows = std::min(rows, max_tokens * k);
+    n = std::max(n, cdiv(rows, router_chunk_rows(rows)));
+  }
+  return (n + E) * d;
 }
 
 int bwd_router_wgrad(const void *xg, const float *dlr, const int32_t *offsets, size_t T, size_t k,
@@ -1405,16 +1418,17 @@ int bwd_router_wgrad(const void *xg, const float *dlr, const int32_t *offsets, s
                      hipStream_t s) {
   if (T == 0) return PRICHS_OK;
   // Every group's chunks fit in cdiv(T*k, chunk) + E workgroups; the rest exit.
-  const unsigned grid = (unsigned)(cdiv(T * k, kRouterChunk) + E);
+  const int chunk = (int)router_chunk_rows(T * k);
+  const unsigned grid = (unsigned)(cdiv(T * k, (size_t)chunk) + E);
   if (dtype == PRICHS_DTYPE_BF16)
     hipLaunchKernelGGL(router_wgrad_part_kernel<bf16_t>, dim3(grid), dim3(256), 0, s,
-                       static_cast<const bf16_t *>(xg), dlr, offsets, (int)E, (int)d, part);
+                       static_cast<const bf16_t *>(xg), dlr, offsets, (int)E, (int)d, chunk, part);
   else
     hipLaunchKernelGGL(router_wgrad_part_kernel<float>, dim3(grid), dim3(256), 0, s,
-                       static_cast<const float *>(xg), dlr, offsets, (int)E, (int)d, part);
+                       static_cast<const float *>(xg), dlr, offsets, (int)E, (int)d, chunk, part);
   PRICHS_LAUNCH_CHECK("moe backward: router weight gradient");
   hipLaunchKernelGGL(router_wgrad_reduce_kernel, dim3(blocks_for((long long)(d * E))), dim3(256),
-                     0, s, part, offsets, (int)E, (int)d, beta, dw);
+                     0, s, part, offsets, (int)E, (int)d, chunk, beta, dw);
   PRICHS_LAUNCH_CHECK("moe backward: router weight gradient reduce");
   return PRICHS_OK;
 }
