@@ -481,14 +481,14 @@ def main():
     if T * k < 64 * E:  # fewer than 64 rows per routed expert on average
         # Decode shape: every touched expert's gate/up weights are streamed once
         # for a handful of rows, so the launch is bound by HBM, not MFMA.  When
-        # one router workgroup covers the batch (T <= 32 here) the engine runs
+        # the batch is decode-sized (T <= 32 here) the engine runs
         # the router inside a gate/up launch over every token of every expert:
         # all E + S experts' weights, x, and the activations of G T rows.
         sel = eng.stash()["selected_experts"].cpu().numpy()
         touched = len(set(sel.reshape(-1).tolist())) + S
         if decode:
             gu_bytes = (E + S) * d * 2 * f * es + T * d * es + (E + S) * T * f * es
-            kernel = ("router workgroup + dense gate/up GEMM + fused SwiGLU, decode launch "
+            kernel = ("router workgroups + dense gate/up GEMM + fused SwiGLU, decode launch "
                       "(skinny::decode_gate_up_router_kernel<4>)")
         else:
             gu_bytes = touched * d * 2 * f * es + rows * d * es + rows * f * es
@@ -565,10 +565,10 @@ def main():
         },
         "stage_ms": {kk: v for kk, v in ms.items() if kk != "n"},
         "stage_ms_flushed": {kk: v for kk, v in ms_cold.items() if kk != "n"},
-        **({"stage_note": "decode path: the router and the permutation run inside the gate/up "
-                          "launch (its first workgroup), so the router and permute intervals hold "
-                          "no kernel, only the gap between event records; gate_up times the "
-                          "router + gate/up launch"} if decode else {}),
+        **({"stage_note": "decode path: the router runs inside the gate/up launch (its first "
+                          "workgroups) and the down launch writes the permutation, so the router "
+                          "and permute intervals hold no kernel, only the gap between event "
+                          "records; gate_up times the router + gate/up launch"} if decode else {}),
         **({"cold_weights": cold} if cold is not None else {}),
         "inputs": inputs_record(f"config{args.config}", inp.digest()),
         "device": torch.cuda.get_device_name(0),

@@ -236,7 +236,7 @@ int prichs_pack_down(const float *down, size_t d, size_t f, int dtype,
  * accumulation.  Requires d % 64 == 0 and f % 64 == 0 for bf16, d % 16 == 0
  * and f % 16 == 0 for f32.  max_rows bounds offsets[G] (sizes the launch);
  * bf16 launches with max_rows <= 64 stream the weights through a skinny
- * (decode) kernel instead of the 256x256-tiled one. */
+ * (decode) kernel instead of the tiled one. */
 int prichs_grouped_gate_up_swiglu(const void *x, const int32_t *row_token,
                                   const int32_t *offsets, size_t G,
                                   size_t max_rows, const void *w_packed,
@@ -449,13 +449,13 @@ int prichs_moe_engine_stash(const prichs_moe_engine *eng,
  * stage_ms waits for those forwards and writes the AVERAGE milliseconds of:
  * [0] router, [1] permute, [2] gate/up GEMM, [3] down GEMM, [4] combine,
  * [5] whole forward; *n_forwards (may be NULL) gets the number averaged.
- * It then re-arms recording for another n forwards.  When one router
- * workgroup covers the batch (decode-sized T, bf16, one shared expert, 5-8
- * routed experts, d % 128 == 0, no backward enabled), the router and the
- * permutation run inside the gate/up launch, which covers every token of
- * every expert, and the down GEMM gathers the routed rows: [0] and [1] then
- * time only event gaps and [2] covers the router too.  The stash's rows and
- * every output are bit-identical either way.  Each event
+ * It then re-arms recording for another n forwards.  At decode sizes (at
+ * most 32 tokens, bf16, one shared expert, 5-8 routed experts, d % 128 == 0,
+ * no backward enabled) the router runs inside the gate/up launch, which
+ * covers every token of every expert, and the down GEMM finds the routed rows
+ * and writes the permutation: [0] and [1] then time only event gaps, [2]
+ * covers the router too and [3] the permutation.  The stash's rows and every
+ * output are bit-identical either way.  Each event
  * costs a few microseconds on the stream, so time throughput with timing
  * off. */
 #define PRICHS_NUM_STAGES 6
