@@ -672,8 +672,8 @@ __global__ __launch_bounds__(wgb::kThreads) void wgrad_bf16_kernel(
   }
 }
 
-// Short items (wgrad_short): most of an item's time is then its epilogue, whose 256 KiB of f32 per 256 x 256 tile leave every CU at
-// the same time.  One workgroup per (group, 128 x 256 tile), the shared group
+// Short items (wgrad_short): most of an item's time is then its epilogue, whose
+// 256 KiB of f32 per 256 x 256 tile leave every CU at the same time.  One workgroup per (group, 128 x 256 tile), the shared group
 // first, three stages of LDS and at most 128 registers, so two share a CU and
 // one's stores run behind the other's products; no group is split, and a
 // group without rows writes its zeros (beta = 0) here, so there is no reduce
