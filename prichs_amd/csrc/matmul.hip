@@ -107,6 +107,99 @@ __global__ __launch_bounds__(T::kThreads) void f32_matmul_kernel(
   f32_matmul_tile<T, OP>(lds, A, B, C, M, N, R, m0, n0, vec_c);
 }
 
+// Short reductions, where a pipelined tile would mostly fill and drain its two
+// stages: one workgroup per 64 x 64 tile (tiles numbered row-major over the
+// grid), 4 waves of 32 x 32 (2 x 2 MFMA blocks of 16 x 16), steps of 16
+// reduction elements through one padded LDS buffer of 8.5 KiB (eight
+// workgroups share a CU and hide each other's loads), loaded with bounds
+// checks so that consecutive threads read consecutive addresses of whichever
+// index is contiguous.
+constexpr int kShortTile = 64;  // output tile (rows and columns)
+constexpr int kShortStep = 16;  // reduction elements per LDS stage
+constexpr int kShortThreads = 256;
+
+template <int OP>
+__global__ __launch_bounds__(kShortThreads) void f32_matmul_short_kernel(
+    const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, long long M,
+    long long N, long long R, long long n_tiles) {
+  __shared__ float As[kShortTile][kShortStep + 1];
+  __shared__ float Bs[kShortTile][kShortStep + 1];
+  const long long tile = blockIdx.x;
+  const long long m0 = (tile / n_tiles) * kShortTile;
+  const long long n0 = (tile % n_tiles) * kShortTile;
+  const int t = threadIdx.x;
+  const int lane = t & 63, wave = t >> 6;
+  const int wm = wave >> 1, wn = wave & 1;
+
+  // Loader coordinates: "rc" = the reduction index is the contiguous one.
+  constexpr bool a_rc = OP != 1, b_rc = OP == 2;
+  const int a_i = a_rc ? t >> 2 : (t & 15) * 4, a_r = a_rc ? (t & 3) * 4 : t >> 4;
+  const int b_j = b_rc ? t >> 2 : (t & 15) * 4, b_r = b_rc ? (t & 3) * 4 : t >> 4;
+
+  f32x4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  float ra[4], rb[4];
+  auto gload = [&](long long r0) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const long long i = m0 + a_i + (a_rc ? 0 : q), ar = r0 + a_r + (a_rc ? q : 0);
+      ra[q] = (i < M && ar < R) ? (OP == 1 ? A[ar * M + i] : A[i * R + ar]) : 0.f;
+      const long long j = n0 + b_j + (b_rc ? 0 : q), br = r0 + b_r + (b_rc ? q : 0);
+      rb[q] = (j < N && br < R) ? (OP == 2 ? B[j * R + br] : B[br * N + j]) : 0.f;
+    }
+  };
+  auto lstore = [&]() {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      As[a_i + (a_rc ? 0 : q)][a_r + (a_rc ? q : 0)] = ra[q];
+      Bs[b_j + (b_rc ? 0 : q)][b_r + (b_rc ? q : 0)] = rb[q];
+    }
+  };
+
+  // MFMA operands (v_mfma_f32_16x16x4f32): lane l holds A[row l%16][k l/16]
+  // and B[k l/16][col l%16]; the result lane holds rows 4 (l/16) + 0..3 of
+  // column l%16.
+  const int fr = lane & 15, fk = lane >> 4;
+  gload(0);
+  for (long long r0 = 0; r0 < R; r0 += kShortStep) {
+    __syncthreads();  // the previous stage's reads are done
+    lstore();
+    __syncthreads();
+    if (r0 + kShortStep < R) gload(r0 + kShortStep);
+#pragma unroll
+    for (int ks = 0; ks < kShortStep / 4; ++ks) {
+      const int kk = ks * 4 + fk;
+      float af[2], bf[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) af[i] = As[wm * 32 + i * 16 + fr][kk];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) bf[j] = Bs[wn * 32 + j * 16 + fr][kk];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i], bf[j], acc[i][j], 0, 0, 0);
+    }
+  }
+
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const long long col = n0 + wn * 32 + j * 16 + fr;
+      if (col >= N) continue;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const long long row = m0 + wm * 32 + i * 16 + 4 * fk + r;
+        if (row < M) C[row * N + col] = acc[i][j][r];
+      }
+    }
+}
+
 // The tile shapes, from large outputs to outputs of a few tiles with a long
 // reduction (waves m x n x k: the last split the reduction).
 template <int CFG, int OP, int W> struct MatmulCfg;
@@ -156,21 +249,38 @@ bool matmul_halves(size_t M, size_t N, int cus, size_t &full) {
   return full > 0 && tail > 0 && 2 * tail <= (size_t)cus;
 }
 
+// Configuration 6: the kernel for short reductions.  Before its first products a
+// pipelined tile fetches and stores its stages, as long as 2 stages of
+// products with 16-byte loads and 4 with single elements; the short kernel has
+// no such start but takes longer per element, 46 ns per 64 x 64 tile of
+// several on a CU and 62 of one alone.  MI355X, us, pipelined -> short: 4096 x
+// 4096 outputs of 16 elements 24.5 -> 18.2, 3000 x 3001 of 17 43.2 -> 15.4, 341
+// x 3005 of 1 13.8 -> 4.7, 1341 x 1245 of 91 21.0 -> 9.8; on small outputs the
+// two meet near 40 elements with single-element loads and near 16 with 16-byte
+// ones (60 x 84 of 64: 3.9 -> 6.0).
+constexpr int kMatmulShort = 6;
+constexpr double kShortAlone = 62.0, kShortShared = 46.0, kFillStages[2] = {2.0, 4.0};
+
 int matmul_cfg(size_t M, size_t N, size_t R, bool vec, int cus) {
-  int best = 0;
-  double best_t = 0;
+  int best = 0, bk = 0;
+  double best_t = 0, per = 0;  // per: ns per reduction element
   for (int c = 0; c < kMatmulCfgs; ++c) {
     const MatmulTileCost &k = kMatmulCost[c];
     const double tiles = (double)cdiv(M, k.bm) * (double)cdiv(N, k.bn);
     if (c > 0 && tiles > (double)INT32_MAX) continue;
-    const double rounds = std::ceil(tiles / cus);
-    const double t = (double)roundup(R, k.bk) * std::max(k.alone[!vec], rounds * k.shared[!vec]);
-    if (c == 0 || t < best_t) best = c, best_t = t;
+    const double e = std::max(k.alone[!vec], std::ceil(tiles / cus) * k.shared[!vec]);
+    const double t = (double)roundup(R, k.bk) * e;
+    if (c == 0 || t < best_t) best = c, best_t = t, per = e, bk = k.bk;
   }
   size_t full = 0;
-  if (vec && matmul_halves(M, N, cus, full) &&
-      (double)roundup(R, 32) * ((double)(full / cus) * kMatmulWhole + kMatmulHalf) < best_t)
-    best = 5;
+  if (vec && matmul_halves(M, N, cus, full)) {
+    const double e = (double)(full / cus) * kMatmulWhole + kMatmulHalf;
+    if ((double)roundup(R, 32) * e < best_t) best = 5, per = e, bk = 32;
+  }
+  const double tiles = (double)cdiv(M, kShortTile) * (double)cdiv(N, kShortTile);
+  if ((double)roundup(R, kShortStep) * std::max(kShortAlone, tiles / cus * kShortShared) <
+      ((double)roundup(R, bk) + kFillStages[!vec] * bk) * per)
+    return kMatmulShort;
   return best;
 }
 
@@ -218,6 +328,15 @@ void launch_matmul_kernel(const float *a, const float *b, float *c, const Matmul
                      vec_c);
 }
 
+template <int OP>
+void launch_matmul_short(const float *a, const float *b, float *c, const MatmulDims &d,
+                         hipStream_t s) {
+  const size_t nt = cdiv(d.N, kShortTile);
+  hipLaunchKernelGGL(f32_matmul_short_kernel<OP>, dim3((unsigned)(cdiv(d.M, kShortTile) * nt)),
+                     dim3(kShortThreads), 0, s, a, b, c, (long long)d.M, (long long)d.N,
+                     (long long)d.R, (long long)nt);
+}
+
 template <int OP, int W>
 void launch_matmul_cfg(int cfg, const float *a, const float *b, float *c, const MatmulDims &d,
                        int vec_c, hipStream_t s) {
@@ -227,6 +346,7 @@ void launch_matmul_cfg(int cfg, const float *a, const float *b, float *c, const 
     case 2: return launch_matmul_kernel<2, OP, W>(a, b, c, d, vec_c, s);
     case 3: return launch_matmul_kernel<3, OP, W>(a, b, c, d, vec_c, s);
     case 5: return launch_matmul_kernel<W == 4 ? 5 : 4, OP, W>(a, b, c, d, vec_c, s);
+    case kMatmulShort: return launch_matmul_short<OP>(a, b, c, d, s);
     default: return launch_matmul_kernel<4, OP, W>(a, b, c, d, vec_c, s);
   }
 }

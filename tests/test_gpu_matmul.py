@@ -201,7 +201,9 @@ def test_matmul_device_entry_on_stream_and_big_reduction(cuda, orc):
                                    (1272, 1000, 68), (500, 1001, 69),     # 32 x 64
                                    (1156, 1152, 100), (1220, 1084, 36),   # 64 x 64, tail in halves
                                    (300, 500, 132), (300, 301, 69),       # 32 x 32
-                                   (36, 68, 260), (17, 45, 257)])         # 16 x 16
+                                   (36, 68, 260), (17, 45, 257),          # 16 x 16
+                                   (1, 1, 1), (64, 128, 16), (65, 127, 1),  # short reductions
+                                   (1000, 1999, 17), (2004, 1000, 8)])
 @pytest.mark.parametrize("op", [L.MATMUL_AB, L.MATMUL_ATB, L.MATMUL_ABT],
                          ids=["ab", "at_b", "a_bt"])
 def test_matmul_tile_shapes(cuda, op, M, N, R):
