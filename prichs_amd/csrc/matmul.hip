@@ -230,14 +230,18 @@ constexpr int kMatmulCfgs = 5;
 // 32), at 4096 x 4096 x 1024 288 against 258 and 356, at 128 x 128 x 4096 72
 // against 256 and 26, and 16 x 16 with the reduction over 8 waves 10.2.
 struct MatmulTileCost {
-  int bm, bn, bk;
+  int bm, bn, bk, threads;
   double alone[2], shared[2];  // [0] 16-byte, [1] single-element loads
 };
 constexpr MatmulTileCost kMatmulCost[kMatmulCfgs] = {
-    {128, 128, 32, {63.0, 78.0}, {63.0, 78.0}}, {64, 64, 64, {18.6, 30.0}, {17.8, 30.0}},
-    {32, 64, 64, {12.7, 18.0}, {9.7, 20.0}},    {32, 32, 64, {7.2, 10.5}, {5.6, 11.0}},
-    {16, 16, 256, {2.5, 5.7}, {2.6, 10.0}},
+    {128, 128, 32, 256, {63.0, 78.0}, {63.0, 78.0}},
+    {64, 64, 64, 512, {18.6, 30.0}, {17.8, 30.0}},
+    {32, 64, 64, 256, {12.7, 18.0}, {9.7, 20.0}},
+    {32, 32, 64, 512, {7.2, 10.5}, {5.6, 11.0}},
+    {16, 16, 256, 512, {2.5, 5.7}, {2.6, 10.0}},
 };
+// A launch has at most 2^32 - 1 threads in x.
+constexpr double kMaxLaunchThreads = 4294967295.0;
 
 // Configuration 5: a last partial round of at most half the CUs in half tiles
 // (2048 x 1280 x 1536: 640 tiles are 2.5 rounds, 71.0 us against 75.0 in 32
@@ -267,18 +271,19 @@ int matmul_cfg(size_t M, size_t N, size_t R, bool vec, int cus) {
   for (int c = 0; c < kMatmulCfgs; ++c) {
     const MatmulTileCost &k = kMatmulCost[c];
     const double tiles = (double)cdiv(M, k.bm) * (double)cdiv(N, k.bn);
-    if (c > 0 && tiles > (double)INT32_MAX) continue;
+    if (c > 0 && tiles * k.threads > kMaxLaunchThreads) continue;
     const double e = std::max(k.alone[!vec], std::ceil(tiles / cus) * k.shared[!vec]);
     const double t = (double)roundup(R, k.bk) * e;
     if (c == 0 || t < best_t) best = c, best_t = t, per = e, bk = k.bk;
   }
   size_t full = 0;
-  if (vec && matmul_halves(M, N, cus, full)) {
+  if (vec && matmul_halves(M, N, cus, full) && (double)(full + cus) * 256 <= kMaxLaunchThreads) {
     const double e = (double)(full / cus) * kMatmulWhole + kMatmulHalf;
     if ((double)roundup(R, 32) * e < best_t) best = 5, per = e, bk = 32;
   }
   const double tiles = (double)cdiv(M, kShortTile) * (double)cdiv(N, kShortTile);
-  if ((double)roundup(R, kShortStep) * std::max(kShortAlone, tiles / cus * kShortShared) <
+  if (tiles * kShortThreads <= kMaxLaunchThreads &&
+      (double)roundup(R, kShortStep) * std::max(kShortAlone, tiles / cus * kShortShared) <
       ((double)roundup(R, bk) + kFillStages[!vec] * bk) * per)
     return kMatmulShort;
   return best;
@@ -319,6 +324,8 @@ void launch_matmul_kernel(const float *a, const float *b, float *c, const Matmul
                           hipStream_t s) {
   typedef typename MatmulCfg<CFG, OP, W>::T T;
   typedef typename MatmulCfg<CFG, OP, W>::TH TH;
+  static_assert(CFG >= kMatmulCfgs || T::kThreads == kMatmulCost[CFG < kMatmulCfgs ? CFG : 0].threads,
+                "the cost table's workgroup");
   const unsigned mt = (unsigned)cdiv(d.M, T::BM), nt = (unsigned)cdiv(d.N, T::BN);
   size_t full = (size_t)mt * nt;
   if (!std::is_same<T, TH>::value) matmul_halves(d.M, d.N, device_cu_count(), full);

@@ -35,3 +35,12 @@ def test_matmul_short_reductions(op):
         assert x.kernel.startswith("f32_matmul_short_kernel<") == (c in short), (c, x.kernel)
         if c in short:
             assert x.grid[0] == -(-c[0] // 64) * -(-c[1] // 64)
+
+
+def test_matmul_largest_launches():
+    # One output column (or row) of 2^27: 2^23 tiles of 16 x 16 with 512
+    # threads would be 2^32 threads, more than a launch may have.
+    for c, x in zip(cases := [("abt", 1 << 27, 1, 256, 0), ("abt", 1, 1 << 27, 256, 0),
+                              ("abt", (1 << 27) - 64, 16, 512, 0), ("atb", 1 << 27, 4, 300, 0)],
+                    _matmul_launches(cases)):
+        assert x.grid[0] * x.block < 1 << 32, (c, x)
