@@ -1136,11 +1136,26 @@ __device__ __forceinline__ void self_permute(const SelfPerm &p, int g, bool writ
     }
   }
   if (write && threadIdx.x == 0) p.offsets[g] = off;
+  // Uniform, but counted behind branches on lane values: said so, the K loop's
+  // branch on the row count is a scalar one instead of an exec mask around
+  // every second MFMA (32 tokens, d = 512, f = 4096: 18.6 -> 17.5 us).
+  off = __builtin_amdgcn_readfirstlane(off);
+  cnt = __builtin_amdgcn_readfirstlane(cnt);
 }
+
+// LDS of a skinny workgroup.
+template <bool GATEUP, int U, int SK, bool SELF> struct SkinnyLds {
+  static constexpr int kRow = 32 * U + 8;  // LDS row (16-byte pad: conflict-free reads)
+  __attribute__((aligned(16))) bf16_t a[SK][2][BM * kRow];
+  f32x4 red[SK > 1 ? SK - 1 : 1][SK > 1 ? 4 * 2 * 64 : 1];  // [slice-1][N-wave, tile, lane]
+  f32x4 gate[GATEUP ? 2 * 2 * 64 : 1];                       // [gate wave, tile, lane]
+  int tok[SELF ? BM : 1];
+};
 
 // The workgroup (N-slab bx, group g, M-tile bz) of a skinny launch.
 template <bool GATEUP, int U, int SK, bool SELF = false>
-__device__ __forceinline__ void skinny_body(const SkinnyArgs &sa, int bx, int g, int bz) {
+__device__ __forceinline__ void skinny_body(SkinnyLds<GATEUP, U, SK, SELF> &lds,
+                                            const SkinnyArgs &sa, int bx, int g, int bz) {
   const bf16_t *__restrict__ A = sa.A;
   const int32_t *__restrict__ a_rows = sa.a_rows;
   const int lda = sa.lda, K = sa.K, ldc = sa.ldc, n_store = sa.n_store, ldp = sa.ldp;
@@ -1148,18 +1163,14 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs &sa, int bx, int g,
   const long long b_stride = sa.b_stride;
   bf16_t *__restrict__ C = sa.C;
   bf16_t *__restrict__ P = sa.P;
-  constexpr int kRow = 32 * U + 8;                 // LDS row (16-byte pad: conflict-free reads)
+  constexpr int kRow = SkinnyLds<GATEUP, U, SK, SELF>::kRow;
   constexpr int kSegs = BM * 4 * U;                // 16-byte segments of one chunk tile
   constexpr int kSegPerThread = kSegs / kThreads;  // U / 2
   static_assert(kSegs % kThreads == 0, "whole segments per thread");
-  __shared__ __attribute__((aligned(16))) bf16_t a_s[SK][2][BM * kRow];
-  __shared__ f32x4 red_s[SK > 1 ? SK - 1 : 1][4][2][64];  // [slice-1][N-wave][tile][lane]
-  __shared__ f32x4 gate_s[2][2][64];                      // [gate wave][tile][lane]
-  __shared__ int tok_s[SELF ? BM : 1];
   const bool dense = sa.dense_T > 0;
   int g0, r1;
   if constexpr (SELF) {
-    self_permute(sa.perm, g, bx == 0, tok_s, g0, r1);
+    self_permute(sa.perm, g, bx == 0, lds.tok, g0, r1);
     r1 += g0;
     __syncthreads();
   } else {
@@ -1192,7 +1203,7 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs &sa, int bx, int g,
     const int r = i / (4 * U), sc = i % (4 * U);
     int src = min(m0 + r, r1 - 1);
     if constexpr (SELF)
-      src = g * sa.perm.T + tok_s[src - g0];
+      src = g * sa.perm.T + lds.tok[src - g0];
     else if (a_rows != nullptr)
       src = a_rows[src];
     else if (dense)
@@ -1213,14 +1224,14 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs &sa, int bx, int g,
   auto store_a = [&](int buf, int c) {
 #pragma unroll
     for (int j = 0; j < kSegPerThread; ++j) {
-      *reinterpret_cast<bf16x8 *>(&a_s[ks][buf][adst[j]]) = areg[j];
+      *reinterpret_cast<bf16x8 *>(&lds.a[ks][buf][adst[j]]) = areg[j];
       if (acpy[j] != nullptr) *reinterpret_cast<bf16x8 *>(acpy[j] + c * 32 * U) = areg[j];
     }
   };
   const int rd = (lane & 15) * kRow + 8 * (lane >> 4);  // fragment read offset, tile 0
   f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
   auto mma = [&](const bf16x8(&w)[U], int buf) {
-    const bf16_t *as = &a_s[ks][buf][rd];
+    const bf16_t *as = &lds.a[ks][buf][rd];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       acc0 = mfma_bf16(w[u], *reinterpret_cast<const bf16x8 *>(as + 32 * u), acc0);
@@ -1256,15 +1267,15 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs &sa, int bx, int g,
 
   if (SK > 1) {
     if (ks > 0) {
-      red_s[ks - 1][wn][0][lane] = acc0;
-      red_s[ks - 1][wn][1][lane] = acc1;
+      lds.red[ks - 1][(2 * wn) * 64 + lane] = acc0;
+      lds.red[ks - 1][(2 * wn + 1) * 64 + lane] = acc1;
     }
     __syncthreads();
     if (ks == 0) {
 #pragma unroll
       for (int j = 0; j < SK - 1; ++j) {
-        acc0 += red_s[j][wn][0][lane];
-        acc1 += red_s[j][wn][1][lane];
+        acc0 += lds.red[j][(2 * wn) * 64 + lane];
+        acc1 += lds.red[j][(2 * wn + 1) * 64 + lane];
       }
     }
   }
@@ -1286,8 +1297,8 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs &sa, int bx, int g,
       }
     }
     if (ks == 0 && wn < 2) {
-      gate_s[wn][0][lane] = acc0;
-      gate_s[wn][1][lane] = acc1;
+      lds.gate[(2 * wn) * 64 + lane] = acc0;
+      lds.gate[(2 * wn + 1) * 64 + lane] = acc1;
     }
     __syncthreads();
     if (ks == 0 && wn >= 2) {
@@ -1296,7 +1307,7 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs &sa, int bx, int g,
       for (int t = 0; t < 2; ++t) {
         const int m = mr + 16 * t;
         if (m < r1 && col < n_store) {
-          const f32x4 gv = gate_s[wn - 2][t][lane];
+          const f32x4 gv = lds.gate[(2 * (wn - 2) + t) * 64 + lane];
           const f32x4 uv = t == 0 ? acc0 : acc1;
           float h[4];
 #pragma unroll
@@ -1321,7 +1332,8 @@ __device__ __forceinline__ void skinny_body(const SkinnyArgs &sa, int bx, int g,
 }
 template <bool GATEUP, int U, int SK, bool SELF = false>
 __global__ __launch_bounds__(kThreads * SK) void skinny_gemm_kernel(SkinnyArgs sa) {
-  skinny_body<GATEUP, U, SK, SELF>(sa, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z);
+  __shared__ SkinnyLds<GATEUP, U, SK, SELF> lds;
+  skinny_body<GATEUP, U, SK, SELF>(lds, sa, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z);
 }
 
 // The router workgroups' arguments in the decode launch (router_chain_body).
@@ -1344,17 +1356,21 @@ __global__ __launch_bounds__(kThreads) void decode_gate_up_router_kernel(SkinnyA
                                                                         RouterArgs ra, int routers,
                                                                         int nx, int ny) {
   static_assert(kThreads == rq::kRouterThreads, "one workgroup size for both roles");
-  extern __shared__ __attribute__((aligned(16))) float router_s[];  // the chain router's products
+  // One buffer for either role: the chain router's products, the GEMM's tiles.
+  extern __shared__ __attribute__((aligned(16))) float decode_s[];
+  using Lds = SkinnyLds<true, U, 1, false>;
+  static_assert(sizeof(Lds) <= rq::kChainLdsBytes, "both roles fit the launch's LDS");
   const int b = (int)blockIdx.x;
   if (b < routers) {
     rq::router_chain_body<bf16_t>(ra.x, ra.w_lds, ra.bias, ra.concept, ra.n_concept, ra.T, ra.d,
                                   ra.E, ra.k, ra.logits, ra.topk_idx, ra.topk_w, ra.block_counts,
                                   rq::FusedPerm{nullptr, nullptr, nullptr, nullptr}, b,
-                                  reinterpret_cast<rq::f32x4 *>(router_s));
+                                  reinterpret_cast<rq::f32x4 *>(decode_s));
     return;
   }
   const int i = b - routers;
-  skinny_body<true, U, 1>(sa, i % nx, (i / nx) % ny, i / (nx * ny));
+  skinny_body<true, U, 1>(*reinterpret_cast<Lds *>(decode_s), sa, i % nx, (i / nx) % ny,
+                          i / (nx * ny));
 }
 }  // namespace skinny
 
@@ -1769,6 +1785,22 @@ bool decode_dense_applies(size_t T, size_t d, size_t f, size_t E, size_t k, size
          d <= (1u << 20) && f <= (1u << 20) && router_chain_applies(T, d, E, x, w_lds);
 }
 
+// LDS of the decode launch.  The router's products, which the GEMM's tiles
+// share, leave room for three workgroups per CU; 56 KiB for two, taken where
+// the launch then has fewer rounds times workgroups: a third place that leaves
+// a last round nearly empty costs more than it hides.  MI355X, us per layer of
+// 1 token, d = 1024, two -> three per CU: f = 2048 (577 workgroups) 28.3 ->
+// 25.9, f = 2816 (793) 32.2 -> 33.7, f = 4096 (1153) 44.6 -> 41.5; d = 256, f =
+// 4096 takes 26.7, and took 28.8 with the LDS of both roles side by side.
+unsigned decode_lds_bytes(size_t workgroups, int cus) {
+  constexpr unsigned kTwo = 56 * 1024;
+  static_assert(rq::kChainLdsBytes <= 52 * 1024 && kTwo > 160 * 1024 / 3 && kTwo <= 64 * 1024,
+                "three per CU, two per CU, no raised LDS limit");
+  const size_t n = (size_t)std::max(cus, 1);
+  return 2 * cdiv(workgroups, 2 * n) < 3 * cdiv(workgroups, 3 * n) ? kTwo
+                                                                  : (unsigned)rq::kChainLdsBytes;
+}
+
 int decode_gate_up_router(const void *x, size_t T, size_t d, size_t f, size_t E, size_t k,
                           const float *w_lds, const float *router_bias,
                           const float *concept_bias, size_t n_concept, float *logits,
@@ -1788,7 +1820,6 @@ int decode_gate_up_router(const void *x, size_t T, size_t d, size_t f, size_t E,
   const int nx = (int)(np / skinny::BN);
   const int mtiles = (int)((T + skinny::BM - 1) / skinny::BM);
   const int routers = (int)cdiv(T, (size_t)rq::kChainTokens);
-  static_assert(rq::kChainLdsBytes <= 64 * 1024, "needs no raised LDS limit");
   const skinny::SkinnyArgs sa{static_cast<const bf16_t *>(x), nullptr, (int)d,
                               static_cast<const bf16_t *>(w_gate_up), (long long)(np * d), (int)d,
                               static_cast<bf16_t *>(act_dense), (int)f, (int)f, nullptr, (int)T,
@@ -1799,7 +1830,8 @@ int decode_gate_up_router(const void *x, size_t T, size_t d, size_t f, size_t E,
                               block_counts};
   const unsigned grid = (unsigned)(routers + nx * G * mtiles);
   hipLaunchKernelGGL((skinny::decode_gate_up_router_kernel<U>), dim3(grid), dim3(skinny::kThreads),
-                     rq::kChainLdsBytes, as_stream(stream), sa, ra, routers, nx, G);
+                     decode_lds_bytes(grid, device_cu_count()), as_stream(stream), sa, ra, routers,
+                     nx, G);
   PRICHS_LAUNCH_CHECK("decode gate/up + router launch");
   return PRICHS_OK;
 }

@@ -97,7 +97,8 @@ def engine(d, f, E, k, dtype, max_tokens, backward=False):
     return h
 
 
-def static_lds(library=os.path.join(ROOT, "prichs_amd", "libprichs_hip.so")):
+def static_lds(library=os.environ.get("PRICHS_HIP_LIB") or os.path.join(
+        ROOT, "prichs_amd", "libprichs_hip.so")):
     """Bytes of LDS that each kernel of the library has at launch (besides its
     dynamic LDS), by symbol, from its code objects' metadata."""
     import msgpack

@@ -44,3 +44,29 @@ def test_matmul_largest_launches():
                               ("abt", (1 << 27) - 64, 16, 512, 0), ("atb", 1 << 27, 4, 300, 0)],
                     _matmul_launches(cases)):
         assert x.grid[0] * x.block < 1 << 32, (c, x)
+
+
+def test_decode_launch_workgroups_per_cu():
+    # The router's and the GEMM's LDS share one buffer: three workgroups of
+    # the decode launch fit a CU's 160 KiB, or two where a third place would
+    # only leave a nearly empty round behind (d = 1024, f = 2816: 792 + 1
+    # workgroups on 768 places).
+    cases = [(256, 4096, 32), (512, 2048, 8), (1536, 1280, 1), (1536, 1280, 32), (1024, 4096, 1),
+             (1024, 2816, 1)]
+    rows = ll.run(f"""
+result = []
+for d, f, T in {cases!r}:
+    h = engine(d, f, 8, 2, L.DTYPE_BF16, 32)
+    L.check(lib.prichs_moe_engine_forward(h, P, T, None, 0, P, L.DTYPE_BF16, None))
+    result += launches()[:1]
+    L.check(lib.prichs_moe_engine_destroy(h))
+""")
+    static = ll.static_lds()
+    for c, x in zip(cases, ll.as_launches(rows)):
+        assert x.kernel.startswith("skinny::decode_gate_up_router_kernel<"), x.kernel
+        per_cu = 160 * 1024 // (x.lds + static[x.symbol])
+        if c[1] == 1280:  # one round on two places per CU
+            assert x.grid[0] <= 512 and per_cu >= 2, (c, x.lds, static[x.symbol])
+        else:
+            assert per_cu == (2 if c[1] == 2816 else 3), (c, x.lds, static[x.symbol])
+        assert x.lds + static[x.symbol] <= 64 * 1024
