@@ -1,5 +1,7 @@
 """Which kernels the library launches, on the CPU (tests/launch_log.py): the
 dispatch rules on sizes, types and alignment."""
+import re
+
 import pytest
 
 from prichs_amd import _lib as L
@@ -70,3 +72,39 @@ for d, f, T in {cases!r}:
         else:
             assert per_cu == (2 if c[1] == 2816 else 3), (c, x.lds, static[x.symbol])
         assert x.lds + static[x.symbol] <= 64 * 1024
+
+
+def _tiles(x):
+    """(rows, columns) of the tiles of a grouped or dense bf16 GEMM launch."""
+    m = re.match(r"bf16_gemm_kernel<Bf16Cfg<(\d+), (\d+)", x.kernel)
+    return (int(m[1]), int(m[2])) if m else None
+
+
+def _forward_gemms(cases, **env):
+    """Launches of the gate/up and down GEMMs of bf16 engine forwards: cases of
+    (E, k, d, f, T)."""
+    rows = ll.run(f"""
+result = []
+for E, k, d, f, T in {cases!r}:
+    h = engine(d, f, E, k, L.DTYPE_BF16, T)
+    L.check(lib.prichs_moe_engine_forward(h, P, T, None, 0, P, L.DTYPE_BF16, None))
+    result += [x for x in launches() if "gemm_kernel" in x[0]]
+    L.check(lib.prichs_moe_engine_destroy(h))
+""", **env)
+    rows = ll.as_launches(rows)
+    assert len(rows) == 2 * len(cases)
+    return list(zip(rows[::2], rows[1::2]))
+
+
+def test_grouped_tiles_near_whole_rounds():
+    # Batches whose groups sit near a multiple of a tile's rows, where the
+    # faster tiles (measured with random routing) were not taken: the larger
+    # ones of gate/up (first three) and down.
+    cases = [(16, 2, 1536, 1280, 3800), (4, 2, 1536, 1280, 1024), (8, 2, 1536, 640, 2048),
+             (8, 2, 1536, 1280, 6860)]
+    for c, g in zip(cases, _forward_gemms(cases)):
+        assert _tiles(g[c[-1] == 6860]) == (256, 256), (c, g)
+    # Few rows keep the smaller tiles.
+    cases = [(8, 2, 1536, 1280, 333), (8, 2, 1536, 1280, 128), (8, 2, 1536, 1280, 8192)]
+    want = [((128, 256), (128, 256)), ((64, 128), (64, 128)), ((256, 256), (256, 256))]
+    assert [tuple(map(_tiles, g)) for g in _forward_gemms(cases)] == want
