@@ -1460,14 +1460,17 @@ using TailCfg = typename std::conditional<
     Bf16Cfg<Cf::BM, Cf::BN / 2, Cf::BN == 256 ? 4 : Cf::WGM, Cf::BN == 256 ? 2 : Cf::WGN,
             Cf::kStages>>::type;
 
-// Persistent grid of a bf16 launch: one workgroup per CU (the LDS ring allows
-// one), fewer when the launch has fewer tiles (twice the tiles when the last
-// round may be split into halves).
+// Persistent grid of a bf16 launch: as many workgroups per CU as the LDS ring
+// allows (kPerCu: two with 64 x 128 tiles, else one), fewer when the launch has
+// fewer tiles (twice the tiles when the last round may be split into halves).
+// Under a cap one per CU at most: nothing would keep two on the same CU.
 template <class Cf, bool GATEUP>
 size_t bf16_grid(size_t max_rows, int G, int Np, int cus) {
   const bool halves = !std::is_same<Cf, TailCfg<Cf, GATEUP>>::value;
   const size_t ub = (max_rows / Cf::BM + G) * (size_t)(Np / Cf::BN) * (halves ? 2 : 1);
-  return std::max<size_t>(1, std::min<size_t>(ub, (size_t)gemm_cu_limit(cus) * Cf::kPerCu));
+  const size_t limit = (size_t)gemm_cu_limit(cus);
+  const size_t places = limit < (size_t)cus ? limit : limit * Cf::kPerCu;
+  return std::max<size_t>(1, std::min<size_t>(ub, places));
 }
 
 template <class Cf, bool GATEUP, bool DSW = false>

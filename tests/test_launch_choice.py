@@ -108,3 +108,16 @@ def test_grouped_tiles_near_whole_rounds():
     cases = [(8, 2, 1536, 1280, 333), (8, 2, 1536, 1280, 128), (8, 2, 1536, 1280, 8192)]
     want = [((128, 256), (128, 256)), ((64, 128), (64, 128)), ((256, 256), (256, 256))]
     assert [tuple(map(_tiles, g)) for g in _forward_gemms(cases)] == want
+
+
+def test_gemm_cu_cap():
+    # PRICHS_GEMM_MAX_CUS bounds the workgroups of every persistent bf16
+    # launch, of 64 x 128 tiles too, two of which fit a CU.
+    cases = [(8, 2, 512, 512, T) for T in (100, 300, 1000, 4096)]
+    tiles = set()
+    for cap in (48, 512):
+        for g in _forward_gemms(cases, PRICHS_GEMM_MAX_CUS=str(cap)):
+            for x in g:
+                tiles.add((cap, _tiles(x)))
+                assert x.grid[0] <= (48 if cap == 48 else 512), x
+    assert (48, (64, 128)) in tiles and (512, (64, 128)) in tiles, tiles
