@@ -1292,14 +1292,10 @@ int bwd_wgrad(bool gateup, const void *A, size_t lda, const void *B, size_t ldb,
       if (n * G > (size_t)INT32_MAX)
         return fail(PRICHS_ERR_UNSUPPORTED, "moe backward: too many tiles");
       auto sk = gateup ? wgrad_bf16_short_kernel<true> : wgrad_bf16_short_kernel<false>;
-      static bool short_attr_set[2] = {false, false};
-      if (!short_attr_set[gateup]) {
-        PRICHS_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(sk),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)wgb::kShortLdsBytes),
-                       "moe backward: set LDS size");
-        short_attr_set[gateup] = true;
-      }
+      static LdsLimit limit[2];
+      if (int rc = raise_lds_limit(limit[gateup], reinterpret_cast<const void *>(sk),
+                                   wgb::kShortLdsBytes, "moe backward: set LDS size"))
+        return rc;
       hipLaunchKernelGGL(sk, dim3((unsigned)(n * G)), dim3(wgb::kThreads), wgb::kShortLdsBytes, s,
                          static_cast<const bf16_t *>(A), (int)lda, (uint32_t)ab,
                          static_cast<const bf16_t *>(B), (int)ldb, (uint32_t)bb, offsets, (int)G,
@@ -1316,14 +1312,10 @@ int bwd_wgrad(bool gateup, const void *A, size_t lda, const void *B, size_t ldb,
     if (items + (size_t)cus > (size_t)INT32_MAX)
       return fail(PRICHS_ERR_UNSUPPORTED, "moe backward: too many tiles");
     auto kern = gateup ? wgrad_bf16_kernel<true, false> : wgrad_bf16_kernel<false, true>;
-    static bool attr_set[2] = {false, false};
-    if (!attr_set[gateup]) {
-      PRICHS_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         (int)wgb::kLdsBytes),
-                     "moe backward: set LDS size");
-      attr_set[gateup] = true;
-    }
+    static LdsLimit limit[2];
+    if (int rc = raise_lds_limit(limit[gateup], reinterpret_cast<const void *>(kern),
+                                 wgb::kLdsBytes, "moe backward: set LDS size"))
+      return rc;
     // The item bound plus half a round: a last round of at most cus / 2
     // items may run as twice as many half-height items.  (Workgroups past
     // the items exit at once, but each still waits for a free CU.)

@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+
 #include <cstddef>
 #include <cstdint>
 #include <cstdio>
@@ -41,6 +43,14 @@ inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s);
 
 // Number of compute units of the current device (cached per device).
 int device_cu_count();
+
+// Raises the current device's limit on a kernel's dynamic LDS to `bytes`, once
+// per device; `raised` is the launcher's record of what it has raised (any
+// number of threads may launch at the same time).
+struct LdsLimit {
+  std::atomic<size_t> bytes[64];
+};
+int raise_lds_limit(LdsLimit &raised, const void *kernel, size_t bytes, const char *who);
 
 // ------------------------------------------------------------------ bf16 --
 typedef uint16_t bf16_t;

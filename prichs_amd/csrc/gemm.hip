@@ -1480,14 +1480,11 @@ int launch_bf16(const void *A, const int32_t *a_rows, int lda, const void *B, lo
                 A2Rows a2 = A2Rows()) {
   using CfT = TailCfg<Cf, GATEUP>;
   const int grid = (int)bf16_grid<Cf, GATEUP>(max_rows, G, Np, cus);
-  static bool attr_set = false;
-  if (!attr_set) {
-    PRICHS_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&bf16_gemm_kernel<Cf, CfT, GATEUP, DSW>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)Cf::kLdsBytes),
-                   "grouped gemm: set LDS size");
-    attr_set = true;
-  }
+  static LdsLimit limit;
+  if (int rc = raise_lds_limit(
+          limit, reinterpret_cast<const void *>(&bf16_gemm_kernel<Cf, CfT, GATEUP, DSW>),
+          Cf::kLdsBytes, "grouped gemm: set LDS size"))
+    return rc;
   // 16-byte epilogue stores (down / dense: rows staged in LDS; gate/up:
   // lane pairs' halves exchanged) need C (and the pre-activations) 16-byte
   // aligned and whole 8-column chunks; otherwise each lane stores its 8-byte

@@ -314,13 +314,10 @@ int launch_quad_t(const XT *x, const float *w, const float *bias, const float *c
                   int nb, hipStream_t s, FusedPerm perm = FusedPerm{nullptr, nullptr, nullptr, nullptr},
                   const float *w_lds = nullptr) {
   const size_t lds = (size_t)8 * (d + 4) * sizeof(float);
-  static int attr_bytes = 0;
-  if ((int)lds > attr_bytes) {
-    PRICHS_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&router_topk_quad_kernel<XT>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
-                   "router: set LDS size");
-    attr_bytes = (int)lds;
-  }
+  static LdsLimit limit;
+  if (int rc = raise_lds_limit(limit, reinterpret_cast<const void *>(&router_topk_quad_kernel<XT>),
+                               lds, "router: set LDS size"))
+    return rc;
   hipLaunchKernelGGL((router_topk_quad_kernel<XT>), dim3(nb), dim3(kRouterThreads), lds, s, x, w,
                      bias, concept, nc, T, d, E, k, logits, idx, wt, bc, perm, w_lds);
   return PRICHS_OK;
@@ -482,14 +479,11 @@ int launch_staged_t(const XT *x, const float *w, const float *bias, const float 
                     int T, int d, int E, int k, float *logits, int32_t *idx, float *wt,
                     int32_t *bc, int nb, hipStream_t s) {
   using Cf = StagedRouter<XT, LPT, KC>;
-  static bool attr_set = false;
-  if (!attr_set) {
-    PRICHS_HIP_TRY(hipFuncSetAttribute(
-                       reinterpret_cast<const void *>(&router_topk_staged_kernel<XT, LPT, KC>),
-                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)Cf::kLds),
-                   "router: set LDS size");
-    attr_set = true;
-  }
+  static LdsLimit limit;
+  if (int rc = raise_lds_limit(
+          limit, reinterpret_cast<const void *>(&router_topk_staged_kernel<XT, LPT, KC>), Cf::kLds,
+          "router: set LDS size"))
+    return rc;
   hipLaunchKernelGGL((router_topk_staged_kernel<XT, LPT, KC>), dim3(nb), dim3(kRouterThreads),
                      Cf::kLds, s, x, w, bias, concept, nc, T, d, E, k, logits, idx, wt, bc);
   return PRICHS_OK;

@@ -40,6 +40,20 @@ int device_cu_count() {
   return n;
 }
 
+int raise_lds_limit(LdsLimit &raised, const void *kernel, size_t bytes, const char *who) {
+  static std::mutex mu;
+  int dev = 0;
+  PRICHS_HIP_TRY(hipGetDevice(&dev), who);
+  const bool known = dev >= 0 && dev < 64;
+  if (known && raised.bytes[dev].load(std::memory_order_acquire) >= bytes) return PRICHS_OK;
+  std::lock_guard<std::mutex> lock(mu);
+  if (known && raised.bytes[dev].load(std::memory_order_relaxed) >= bytes) return PRICHS_OK;
+  PRICHS_HIP_TRY(
+      hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes), who);
+  if (known) raised.bytes[dev].store(bytes, std::memory_order_release);
+  return PRICHS_OK;
+}
+
 }  // namespace prichs
 
 extern "C" const char *prichs_last_error(void) { return prichs::g_last_error; }

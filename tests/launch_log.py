@@ -60,9 +60,14 @@ def start(so):
     return L.load(), L
 
 
-def events(kind):
-    rows = [ln.split("\t") for ln in _log.launch_log_take().decode().splitlines()]
-    return [r[1:] for r in rows if r[0] == kind]
+def hip():
+    """The stand-in library (hipSetDevice)."""
+    return _log
+
+
+def raw_events():
+    """The log since the last call: rows of text, launches and raised limits."""
+    return [ln.split("\t") for ln in _log.launch_log_take().decode().splitlines()]
 
 
 def _short(name):
@@ -79,7 +84,7 @@ def _short(name):
 def launches():
     """The kernels launched since the last call, as Launch rows."""
     return [[_short(r[0]), r[1], [int(v) for v in r[2:5]], int(r[5]), int(r[6]), int(r[7])]
-            for r in events("launch")]
+            for ev, *r in raw_events() if ev == "launch"]
 
 
 def engine(d, f, E, k, dtype, max_tokens, backward=False):
@@ -91,9 +96,9 @@ def engine(d, f, E, k, dtype, max_tokens, backward=False):
     z = (C.c_float * (d * f))()
     ptrs = (C.c_void_p * (E + 1))(*[C.addressof(z)] * (E + 1))
     w, b = (C.c_float * (d * E))(), (C.c_float * E)()
-    L.check(lib.prichs_moe_engine_upload(h, w, b, ptrs, ptrs, ptrs))
     if backward:
         L.check(lib.prichs_moe_engine_enable_backward(h))
+    L.check(lib.prichs_moe_engine_upload(h, w, b, ptrs, ptrs, ptrs))
     return h
 
 

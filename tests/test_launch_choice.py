@@ -121,3 +121,34 @@ def test_gemm_cu_cap():
                 tiles.add((cap, _tiles(x)))
                 assert x.grid[0] <= (48 if cap == 48 else 512), x
     assert (48, (64, 128)) in tiles and (512, (64, 128)) in tiles, tiles
+
+
+def test_lds_limits_on_every_device():
+    # A kernel's limit on dynamic LDS is the device's: every launch with more
+    # than 64 KiB follows a raise of its kernel's limit on that device.
+    rows = ll.run("""
+for dev in (0, 1, 0, 2):
+    hip().hipSetDevice(dev)
+    for M in (64, 1000, 20000):
+        L.check(lib.prichs_gemm(P, 512, M, 512, P, 512, P, 512, L.DTYPE_BF16, None))
+    for E, d in ((8, 4096), (64, 512), (8, 1024)):
+        L.check(lib.prichs_router_topk(P, L.DTYPE_F32, P, P, None, 0, 5000, d, E, 2, P, P, P, P, None))
+    h = engine(256, 256, 8, 2, L.DTYPE_BF16, 6000, backward=True)
+    g = L.MoEGrads(P, P, P, P, 1 << 20, 0)
+    for T in (100, 400, 6000):
+        L.check(lib.prichs_moe_engine_forward(h, P, T, None, 0, P, L.DTYPE_BF16, None))
+        L.check(lib.prichs_moe_engine_backward(h, P, P, T, P, L.DTYPE_BF16, C.byref(g), 2, None))
+result = raw_events()
+""")
+    limit, seen = {}, set()
+    for r in rows:
+        if r[0] == "attribute":
+            limit[r[1], r[3]] = int(r[2])
+        elif int(r[7]) > 64 * 1024:
+            name, lds, dev = r[1], int(r[7]), r[8]
+            assert limit.get((name, dev), 0) >= lds, (name, lds, dev)
+            seen.add((name, dev))
+    assert {dev for _, dev in seen} == {"0", "1", "2"}
+    kinds = {n.split("<")[0].split("::")[-1] for n, _ in seen}
+    assert {"bf16_gemm_kernel", "wgrad_bf16_kernel", "wgrad_bf16_short_kernel",
+            "router_topk_quad_kernel"} <= kinds, kinds
