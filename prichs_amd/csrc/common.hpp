@@ -52,6 +52,13 @@ struct LdsLimit {
 };
 int raise_lds_limit(LdsLimit &raised, const void *kernel, size_t bytes, const char *who);
 
+// LDS writes done, then the workgroup barrier.  Unlike __syncthreads it leaves
+// global loads in flight.  One statement: nothing can come between the wait and
+// the barrier.
+__device__ __forceinline__ void lds_write_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // ------------------------------------------------------------------ bf16 --
 typedef uint16_t bf16_t;
 

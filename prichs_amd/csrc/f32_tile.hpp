@@ -43,12 +43,6 @@ namespace f32t {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// LDS writes done, then the workgroup barrier.  Unlike __syncthreads it does
-// not wait for the global loads in flight, which go to registers only.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 // Wrapper: a builtin called with template-dependent arguments fails silently
 // in the host pass.
 __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
@@ -250,7 +244,7 @@ struct Tile {
       if (sl + 1 < kSlices) {
         read(f[(sl + 1) & 1], cur, sl + 1);
       } else {
-        lds_barrier();
+        lds_write_barrier();
         read(f[(sl + 1) & 1], nx, 0);
       }
       products(f[sl & 1]);
@@ -275,7 +269,7 @@ struct Tile {
       ob.template store<false>(lds + OpA::kElems, t);
       oa.template fetch<false>(BK, R, a_step, t);
       ob.template fetch<false>(BK, R, b_step, t);
-      lds_barrier();
+      lds_write_barrier();
       Frags f[2];
       read(f[0], lds, 0);
       long long r0 = 0;
@@ -288,7 +282,7 @@ struct Tile {
                              a_step, b_step, t);
     }
     if (WGK == 1) return true;
-    lds_barrier();  // the last stage's reads ahead are done
+    lds_write_barrier();  // the last stage's reads ahead are done
     float *part = lds + ((wm * WGN + wn) * 64 + lane) * 4;
     constexpr int kBlock = WGM * WGN * 64 * 4, kWave = MI * NJ * kBlock;
     if (wk > 0) {
@@ -298,7 +292,7 @@ struct Tile {
         for (int j = 0; j < NJ; ++j)
           *reinterpret_cast<f32x4 *>(part + (wk - 1) * kWave + (i * NJ + j) * kBlock) = acc[i][j];
     }
-    lds_barrier();
+    lds_write_barrier();
     if (wk > 0) return false;
 #pragma unroll
     for (int k = 0; k < WGK - 1; ++k)

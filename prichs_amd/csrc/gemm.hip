@@ -196,20 +196,24 @@ __device__ __forceinline__ void static_for(std::integer_sequence<int, Is...>, F 
   (f(std::integral_constant<int, Is>{}), ...);
 }
 
-// Workgroup barrier without a memory fence: LDS-DMA completion is tracked by
-// the explicit vmcnt waits, and a fence would force vmcnt(0).
-__device__ inline void lds_barrier() {
+// Workgroup barrier without a memory fence or a wait (a fence would force
+// vmcnt(0)): LDS-DMA completion is tracked by the explicit vmcnt waits.  It does
+// not wait for the wave's own LDS writes; before other waves read those,
+// tile_write_barrier.
+__device__ inline void bare_barrier() {
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 }
 
-// The same between LDS writes and other waves' reads of them: the bare barrier
-// does not wait for the writes (the LDS queues of the SIMDs drain on their
-// own), so the wave waits for its own first.
-__device__ inline void lds_write_barrier() {
+// lds_write_barrier in builtins, which tell the compiler that nothing is left to
+// wait for: the epilogue's row reads then wait for one another only.  The first
+// fence keeps the LDS writes before the wait.
+__device__ inline void tile_write_barrier() {
+  asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-  lds_barrier();
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
 }
 
 #ifndef PRICHS_BF16_STAGES
@@ -403,7 +407,7 @@ __device__ __forceinline__ void bf16_tile(
   // The previous tile's stores drain and every wave is past its last LDS
   // read before the ring is refilled.
   wait_vmcnt(0);
-  lds_barrier();
+  bare_barrier();
 
   // DMA instruction `which` of stage kt_: A rows first, then B fragments.
   auto issue_one = [&](int kt_, int which) {
@@ -458,7 +462,7 @@ __device__ __forceinline__ void bf16_tile(
       PRICHS_WAIT_VMCNT(kInst2);
     else
       PRICHS_WAIT_VMCNT(0);
-    lds_barrier();
+    bare_barrier();
     read_frags(f0, 0);
     auto mma = [&](const Frags &F) {
 #pragma unroll
@@ -478,7 +482,7 @@ __device__ __forceinline__ void bf16_tile(
       else
         PRICHS_WAIT_VMCNT(0);
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): own reads of step s done
-      lds_barrier();
+      bare_barrier();
       if (kFull || s_ + R < NS) {
         issue_stage(2 * (s_ + R));
         issue_stage(2 * (s_ + R) + 1);
@@ -496,7 +500,7 @@ __device__ __forceinline__ void bf16_tile(
     mma(f0);
     mma(f1);
     __builtin_amdgcn_s_waitcnt(0xc07f);
-    lds_barrier();  // every wave is done reading the ring
+    bare_barrier();  // every wave is done reading the ring
   } else {
   // Ping-pong K loop over a ring of S = kStages LDS stages, S - 1 of them in
   // flight.  Waves 0-3 (group 0) and 4-7 (group 1) sit one per SIMD each, so
@@ -524,7 +528,7 @@ __device__ __forceinline__ void bf16_tile(
   // memory clobber alone would let the scheduler move them over it).
   auto pp_barrier = [] {
     __builtin_amdgcn_sched_barrier(0);
-    lds_barrier();
+    bare_barrier();
     __builtin_amdgcn_sched_barrier(0);
   };
   Frags F;
@@ -588,7 +592,7 @@ __device__ __forceinline__ void bf16_tile(
     // 32-byte pieces of 16 rows).  C is 16-byte aligned and ldc, n_store
     // are multiples of 8.
     constexpr int kS = Cf::kStgStride;
-    lds_barrier();  // every wave is done reading the ring
+    bare_barrier();  // every wave is done reading the ring
     const int tcol = wn * WN + cq;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
@@ -600,7 +604,7 @@ __device__ __forceinline__ void bf16_tile(
             u32x2{pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3])};
       }
     }
-    lds_write_barrier();
+    tile_write_barrier();
     constexpr int kChunksRow = BN / 8;  // 16-byte chunks per tile row
     if constexpr (DSW) {
       // SwiGLU backward on the staged (bf16-rounded) dA: chunk ch of row r
@@ -709,7 +713,7 @@ __device__ __forceinline__ void bf16_tile(
       // the forward's weights and activations (training forward 335.5 ->
       // 328.8 us, step -6.9 us).
       constexpr int kS = Cf::kStgStride;
-      lds_barrier();  // every wave is done reading the ring
+      bare_barrier();  // every wave is done reading the ring
       const int tcol = wn * WN + cq;
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
@@ -721,7 +725,7 @@ __device__ __forceinline__ void bf16_tile(
               u32x2{pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3])};
         }
       }
-      lds_write_barrier();
+      tile_write_barrier();
       constexpr int kChunksRow = BN / 8;  // 16-byte chunks per tile row
 #pragma unroll 4
       for (int c = tid; c < BM * kChunksRow; c += Cf::kThreads) {
@@ -752,7 +756,7 @@ __device__ __forceinline__ void bf16_tile(
       // pre-activation copy of the training forward the extra barrier costs
       // more than it gains there).
       constexpr int kSa = BN / 2 + 8;
-      lds_barrier();  // every wave is done reading the ring
+      bare_barrier();  // every wave is done reading the ring
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
         bf16_t *srow = lds + (wm * WM + fr + 16 * i) * kSa;
@@ -770,7 +774,7 @@ __device__ __forceinline__ void bf16_tile(
           }
         }
       }
-      lds_write_barrier();
+      tile_write_barrier();
       constexpr int kChunksRow = BN / 16;  // 16-byte chunks per activation row
 #pragma unroll 4
       for (int c = tid; c < BM * kChunksRow; c += Cf::kThreads) {
@@ -907,7 +911,7 @@ __global__ __launch_bounds__(T::kThreads) void grouped_gemm_kernel(
   const int fr = tile.lane & 15, fc = 4 * (tile.lane >> 4);
 
   for (unsigned b = blockIdx.x; b < total; b += gridDim.x) {
-    if (b != blockIdx.x) f32t::lds_barrier();  // the tile before is out of the LDS
+    if (b != blockIdx.x) lds_write_barrier();  // the tile before is out of the LDS
     int mt, nt;
     tile_coords((int)f32t::xcd_run(b, total), tm.m_tiles, n_tiles, mt, nt);
     const int g = wave_find_group(tm, mt);

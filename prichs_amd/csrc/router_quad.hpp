@@ -216,12 +216,6 @@ __device__ inline void finish_block(const int *cnt_s, const int32_t *idx_s, cons
                 perm.token_row);
 }
 
-// LDS writes done, then the workgroup barrier; unlike __syncthreads it leaves
-// global loads in flight.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 // ---------------------------------------------------------------------------
 // Quad-broadcast router (E <= 8, eight lanes per token, d % 128 == 0).  The
 // block's router weights sit transposed in LDS for the whole kernel (staged
@@ -497,11 +491,11 @@ __device__ inline void router_chain_body(
       for (int i = 0; i < kAhead; ++i) {
         if (r0 + i < rounds) {
           produce(r0 + i, i);
-          lds_barrier();
+          lds_write_barrier();
         }
       }
     }
-    lds_barrier();
+    lds_write_barrier();
   } else {
     float acc = 0.0f;
     f32x4 held[kChainK / 4];
@@ -520,7 +514,7 @@ __device__ inline void router_chain_body(
     // again only after barrier r + 1, which this wave reaches with its reads
     // of round r done.
     for (int r = 0; r < rounds; ++r) {
-      lds_barrier();
+      lds_write_barrier();
       f32x4 v0[kChainK / 4], v1[kChainK / 4];
       read(r, 0, v0);
       if (r > 0) add(held);  // always a whole round before
@@ -529,7 +523,7 @@ __device__ inline void router_chain_body(
       add(v0);
       if (kChainProd * r + 1 < nch) add(v1);
     }
-    lds_barrier();
+    lds_write_barrier();
     if (kChainProd * (rounds - 1) + 2 < nch) add(held);
 
     const int e = lane & 7, t = bid * kChainTokens + (lane >> 3);
