@@ -99,9 +99,6 @@ def test_backward_f32_matches_oracle(cuda, orc, T, d, f, E, k, weighting):
 
 
 # ------------------------------------------------------------- bf16 engine --
-# Config-1 shapes in bf16, a padded f (192: packed columns 384..511 are
-# padding), a decode-sized batch whose groups take the skinny GEMM, and a
-# batch whose shared group (3000 rows) the weight-gradient kernels split over K.
 # The f32 weight gradients' 128 x 128 and 64 x 64 tiles (the cases above take
 # 32 x 64), with gradients ending inside a tile.
 @pytest.mark.parametrize("T,d,f", [(40, 1536, 1296), (37, 656, 624)])
@@ -112,6 +109,9 @@ def test_backward_f32_tile_shapes(cuda, orc, T, d, f):
     check_against_oracle(orc, inp, d_out, 2, d_x, grads, TOL["f32"])
 
 
+# Config-1 shapes in bf16, a padded f (192: packed columns 384..511 are
+# padding), a decode-sized batch whose groups take the skinny GEMM, and a
+# batch whose shared group (3000 rows) the weight-gradient kernels split over K.
 @pytest.mark.parametrize("T,d,f,E,k", [(512, 256, 128, 8, 2), (300, 128, 192, 8, 2),
                                        (32, 256, 128, 8, 2), (3000, 256, 128, 4, 2)])
 @pytest.mark.parametrize("weighting", [1, 2])

@@ -50,68 +50,38 @@ def test_dense_gemm(cuda, orc, M, K, N):
     assert not hw[:, :32].any() and not hw[:, 32 + N:].any()
 
 
-def _tile_times(tiles, grid, split):
-    full, tail = divmod(tiles, grid)
-    if tail == 0:
-        return full
-    return full + (0.6 if split and 2 * tail <= grid else 1.0)
-
-
-def _dense_cfg(M, N, cus):
-    """Mirror of the dense launcher's choice: ("square" | "wide" | "tall", tail
-    split).  Square = 256 x 256 tiles on a grid of min(2 (M/256 + 1) N/256,
-    CUs) whose last partial round of t tiles is split into half-width tiles
-    when 2 t fits the grid; wide = 128 x 384 tiles (N a multiple of 384) on
-    min((M/128 + 1) N/384, CUs), never split, each 0.75 of a square tile's
-    work at 0.96 of its rate; tall = 256 x 288 tiles (N a multiple of 288) on
-    min((M/256 + 1) N/288, CUs), never split, 1.125 of a square tile's work.
-    The fastest estimate wins (ties keep the earlier shape)."""
-    sq_tiles = -(-M // 256) * (N // 256)
-    sq_grid = min(2 * (M // 256 + 1) * (N // 256), cus)
-    tail = sq_tiles % sq_grid
-    split = 0 < tail and 2 * tail <= sq_grid
-    best, cfg = _tile_times(sq_tiles, sq_grid, True), ("square", split)
-    if N % 384 == 0:
-        wd_tiles = -(-M // 128) * (N // 384)
-        wd_grid = min((M // 128 + 1) * (N // 384), cus)
-        t = _tile_times(wd_tiles, wd_grid, False) * 0.75 / 0.96
-        if t < best:
-            best, cfg = t, ("wide", False)
-    if N % 288 == 0:
-        tl_tiles = -(-M // 256) * (N // 288)
-        tl_grid = min((M // 256 + 1) * (N // 288), cus)
-        t = _tile_times(tl_tiles, tl_grid, False) * 1.125
-        if t < best:
-            best, cfg = t, ("tall", False)
-    return cfg
+# (M, N) -> tile of the dense bf16 GEMM's launch on 256 CUs and whether its last
+# round runs in half-width tiles (tests/test_launch_choice.py checks them).
+DENSE_TILES = {
+    (777, 1536): ((64, 128), False), (2048, 1536): ((128, 256), True),
+    (4096, 1536): ((256, 256), True), (8192, 1536): ((128, 384), False),
+    (12000, 1536): ((128, 384), False), (12288, 1536): ((128, 384), False),
+    (20000, 1536): ((256, 256), False), (2048, 2304): ((256, 256), True),
+    (4096, 2304): ((128, 384), False), (8192, 2304): ((256, 288), False),
+    (300, 320): ((64, 128), False), (1024, 2304): ((128, 256), True),
+}
 
 
 def test_gemm_tail_round_halves_bit_identical(cuda):
     """The last partial round of the down / dense GEMM runs as half-width
-    tiles, and some dense launches run as 128 x 384 tiles: every output
-    element is the same MFMA chain over K, so rows computed either way are
-    bit-identical to the same rows of a launch that computes them as whole
-    256 x 256 tiles, and within the 1e-2 bar of float64."""
+    tiles, and some dense launches run as 128 x 384, 128 x 256 or 64 x 128
+    tiles: every output element is the same MFMA chain over K, so rows
+    computed either way are bit-identical to the same rows of a launch that
+    computes them as whole 256 x 256 tiles, and within the 1e-2 bar of
+    float64."""
     K = N = 1536
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
     rng = np.random.default_rng(11)
     a = synth.round_bf16(rng.standard_normal((20000, K)))
     w = synth.round_bf16(0.05 * rng.standard_normal((K, N)))
     wp = ops.to_device_packed([ops.pack_weight(w, "bf16")], "bf16")
-    assert _dense_cfg(20000, N, cus) == ("square", False)
     whole = host(ops.gemm(dev(a), wp, N))
-    seen = set()
-    for M in (4096, 8192, 12000, 12288):
-        cfg = _dense_cfg(M, N, cus)
-        seen.add(cfg)
-        say(f"dense gemm M={M}: tiles {cfg[0]}, tail split {cfg[1]} on {cus} CUs")
+    for M in sorted(m for m, n in DENSE_TILES if n == N and m < 20000):
+        say(f"dense gemm M={M}: {DENSE_TILES[M, N]}")
         c = host(ops.gemm(dev(a[:M]), wp, N))
         np.testing.assert_array_equal(c, whole[:M])
         lo = max(0, M - 2048)  # the tail tiles hold the last M-tiles
         ref = a[lo:M].astype(np.float64) @ w.astype(np.float64)
         assert rel_err(c[lo:], ref) <= 1e-2
-    if cus == 256:
-        assert ("square", True) in seen and ("wide", False) in seen, seen
 
 
 def test_dense_gemm_qkv_shape_tiles(cuda, orc):
@@ -119,13 +89,10 @@ def test_dense_gemm_qkv_shape_tiles(cuda, orc):
     256 x 288 tiles on 256 CUs (one round; 18 B blocks per stage dealt
     unevenly over the 8 waves): against the oracle's matmul_2d on row slices,
     and bit-identical to the rows of launches that pick 128 x 384 tiles (4096
-    rows) and 256 x 256 tiles with a half-width tail (2048 rows)."""
+    rows), 256 x 256 and 128 x 256 tiles with a half-width tail (2048 and 1024
+    rows)."""
     M, K, N = 8192, 1536, 2304
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
-    cfgs = {m: _dense_cfg(m, N, cus)[0] for m in (M, 4096, 2048)}
-    say(f"dense gemm {N}x{K}: tiles by rows {cfgs} on {cus} CUs")
-    if cus == 256:
-        assert cfgs == {M: "tall", 4096: "wide", 2048: "square"}, cfgs
+    say(f"dense gemm {N}x{K}: " + str([DENSE_TILES[m, N] for m in (M, 4096, 2048, 1024)]))
     rng = np.random.default_rng(5)
     a = synth.round_bf16(rng.standard_normal((M, K)))
     w = synth.round_bf16(0.05 * rng.standard_normal((K, N)))
@@ -134,7 +101,7 @@ def test_dense_gemm_qkv_shape_tiles(cuda, orc):
     for lo in (0, 4000, M - 256):
         ref = orc.matmul_2d(a[lo:lo + 256], w)
         assert rel_err(c[lo:lo + 256], ref) <= 1e-2, lo
-    for m2 in (4096, 2048):
+    for m2 in (4096, 2048, 1024):
         np.testing.assert_array_equal(host(ops.gemm(dev(a[:m2]), wp, N)), c[:m2])
 
 

@@ -193,17 +193,44 @@ def test_matmul_device_entry_on_stream_and_big_reduction(cuda, orc):
     assert rel_err(out.cpu().numpy(), orc.matmul_2d(a, b)) <= TOL
 
 
-# (M, N, R) of the output and the reduction: each tile shape of the kernel
-# with 16-byte loads (every row start a multiple of 4 elements) and with
-# single-element ones, ending inside a tile and inside a reduction step.
-@pytest.mark.parametrize("M,N,R", [(2044, 2040, 36), (1999, 2001, 33),    # 128 x 128
-                                   (1000, 1020, 100), (1001, 777, 101),   # 64 x 64
-                                   (1272, 1000, 68), (500, 1001, 69),     # 32 x 64
-                                   (1156, 1152, 100), (1220, 1084, 36),   # 64 x 64, tail in halves
-                                   (300, 500, 132), (300, 301, 69),       # 32 x 32
-                                   (36, 68, 260), (17, 45, 257),          # 16 x 16
-                                   (1, 1, 1), (64, 128, 16), (65, 127, 1),  # short reductions
-                                   (1000, 1999, 17), (2004, 1000, 8)])
+# (M, N, R) of the output and the reduction, and the kernels that take them (all
+# ops; tests/test_launch_choice.py checks them) from 16-byte aligned operands and
+# from operands 4 bytes past: tile shape, "+halves" for a last round in half
+# tiles, elements per load, or the kernel for short reductions.  They end inside
+# a tile and inside a reduction step.
+MATMUL_TILES = [
+    (2044, 2040, 36, "128x128/4", "short"),
+    (2044, 2040, 132, "128x128/4", "128x128/1"),
+    (1999, 2001, 333, "128x128/1", "128x128/1"),
+    (1999, 2001, 33, "short", "short"),
+    (1000, 1020, 100, "64x64/4", "short"),
+    (1000, 1020, 356, "64x64/4", "64x64/1"),
+    (1001, 777, 401, "64x64/1", "64x64/1"),
+    (1001, 777, 101, "short", "short"),
+    (1236, 788, 100, "32x64/4", "short"),
+    (1236, 788, 1004, "32x64/4", "32x64/1"),
+    (500, 1001, 301, "32x64/1", "32x64/1"),
+    (500, 1001, 69, "short", "short"),
+    (1156, 1152, 100, "64x64+halves/4", "short"),
+    (1220, 1084, 136, "64x64+halves/4", "short"),
+    (1272, 1000, 68, "64x64+halves/4", "short"),
+    (1220, 1084, 36, "short", "short"),
+    (300, 500, 132, "32x32/4", "32x32/1"),
+    (300, 301, 301, "32x32/1", "32x32/1"),
+    (300, 301, 69, "32x32/1", "32x32/1"),
+    (144, 56, 1892, "16x16/4", "16x16/1"),
+    (145, 58, 1895, "16x16/1", "16x16/1"),
+    (36, 68, 260, "16x16/4", "32x32/1"),
+    (17, 45, 257, "32x32/1", "32x32/1"),
+    (1, 1, 1, "short", "short"),
+    (64, 128, 16, "short", "short"),
+    (65, 127, 1, "short", "short"),
+    (1000, 1999, 17, "short", "short"),
+    (2004, 1000, 8, "short", "short"),
+]
+
+
+@pytest.mark.parametrize("M,N,R", [c[:3] for c in MATMUL_TILES])
 @pytest.mark.parametrize("op", [L.MATMUL_AB, L.MATMUL_ATB, L.MATMUL_ABT],
                          ids=["ab", "at_b", "a_bt"])
 def test_matmul_tile_shapes(cuda, op, M, N, R):

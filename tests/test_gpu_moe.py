@@ -112,6 +112,43 @@ def test_router_ties_nan_and_concept_bias(cuda, orc, d):
             assert np.abs(gw[ok] - rw[ok]).max() <= 1e-6
 
 
+# The same through the engine, whose batches of up to 2048 tokens take the chain
+# router: inside the decode launch (16), in one workgroup with its permutation
+# (5, f32), and in several.
+@pytest.mark.parametrize("T,dtype", [(16, "bf16"), (64, "bf16"), (5, "f32"), (70, "f32")])
+def test_chain_router_ties_nan_and_concept_bias(cuda, orc, T, dtype):
+    d, f, E, k = 128, 64, 8, 2
+    rng = np.random.default_rng(12)
+    x = synth.round_bf16(rng.standard_normal((T, d)))
+    x[:4] = 0.0
+    wr = (0.2 * rng.standard_normal((d, E))).astype(np.float32)
+    wr_nan = wr.copy()
+    wr_nan[3, 5] = np.nan
+    b = np.array([0.5, 0.5, -0.0, 0.0, 0.5, 0.1, -1, 0.5], np.float32)
+    cb = np.array([0.0, 0.0, 0.25], np.float32)
+    gate = [synth.round_bf16(0.1 * rng.standard_normal((d, f))) for _ in range(E + 1)]
+    down = [np.ascontiguousarray(g.T) for g in gate]
+    say("chain router", T, dtype)
+    for w_r in (wr, wr_nan):
+        eng = moe.MoEEngine(d, f, E, k, 1, dtype, max_tokens=T)
+        eng.upload(w_r, b, gate, gate, down)
+        for concept in (None, cb):
+            eng.forward(dev(x, dtype), concept_bias=None if concept is None else dev(concept))
+            st = eng.stash()
+            rl, rs, rw = orc.route(x, w_r, b, k, concept_bias=concept)
+            o_off, o_rt, _, o_tr = orc.bin_tokens(rs, rw, E)
+            assert np.array_equal(host(st["router_logits"]).view(np.uint32), rl.view(np.uint32))
+            assert np.array_equal(host(st["selected_experts"]), rs)
+            assert np.array_equal(host(st["offsets"])[:E + 1], o_off)
+            assert np.array_equal(host(st["row_token"])[:T * k], o_rt)
+            assert np.array_equal(host(st["token_row"]), o_tr)
+            gw = host(st["gating_weights"])
+            assert np.array_equal(np.isnan(gw), np.isnan(rw))
+            ok = ~np.isnan(rw)
+            assert np.abs(gw[ok] - rw[ok]).max(initial=0) <= 1e-6
+        eng.close()
+
+
 # ------------------------------------------------------------ permutation --
 @pytest.mark.parametrize("cfg", [1, 2, 3, 4])
 def test_permutation_bit_exact(cuda, orc, cfg):
@@ -204,20 +241,30 @@ def test_gate_up_unaligned_output_bit_identical(cuda):
     assert int(flat[:4].view(torch.int16).abs().sum()) == 0  # nothing written before it
 
 
-# Launches with few rows take 128 x 256 tiles (whole ones, or all as 128 x 128
-# halves where those fill at most half the CUs) or 64 x 128 ones: ragged, empty, one-row and
-# exactly full groups.  The extra group of the second launch makes the same
-# rows take 256 x 256 tiles; every output element is one MFMA chain over K, so
-# the shared rows agree bit for bit.
-@pytest.mark.parametrize("d,f,counts", [(1536, 1280, [83, 0, 129, 300, 1]),      # halves
-                                        (1536, 1280, [64, 0, 65, 1, 63, 70]),     # 64 x 128
-                                        (64, 192, [100, 33]),      # 64 x 128, 1 and 3 K-steps
-                                        (1536, 1280, [256, 128, 700, 384, 513]),  # whole
-                                        (320, 192, [65, 255, 1000])])
+# Launches with few rows take 128 x 256 tiles or 64 x 128 ones: ragged, empty,
+# one-row and exactly full groups.  Per case the (tile, whole rounds, last round
+# in halves) of the gate/up and the down launch on 256 CUs, which
+# tests/test_launch_choice.py checks.  With one more group, REF_ROWS rows in
+# all, both take 256 x 256 tiles; every output element is one MFMA chain over
+# K, so the shared rows agree bit for bit.
+MID, SMALL, BIG = (128, 256), (64, 128), (256, 256)
+MID_TILES = [
+    (1536, 1280, [83, 0, 129, 200, 1, 128, 127, 140, 92], (MID, 0, True), (SMALL, 0, False)),
+    (1536, 1280, [256, 128, 700, 384, 513], (MID, 0, False), (MID, 0, True)),
+    (1536, 1280, [6500, 100], (MID, 2, True), (BIG, 0, False)),
+    (1536, 1280, [64, 0, 65, 1, 63, 70], (SMALL, 0, False), (SMALL, 0, False)),
+    (64, 192, [100, 33], (SMALL, 0, False), (SMALL, 0, False)),  # 1 and 3 K-steps
+    (320, 192, [900, 3000, 100, 0, 1000], (MID, 0, True), (MID, 0, True)),
+]
+REF_ROWS = {1536: 15600, 320: 20000, 64: 30000}
+
+
+@pytest.mark.parametrize("d,f,counts", [c[:3] for c in MID_TILES])
 @pytest.mark.parametrize("aligned", [True, False])
 def test_mid_tiles_bit_identical(cuda, orc, d, f, counts, aligned):
     rng = np.random.default_rng(d + f + len(counts))
-    G, rows, extra, Tx = len(counts), sum(counts), 9000, 400
+    G, rows, Tx = len(counts), sum(counts), 400
+    extra = REF_ROWS[d] - rows
     x = dev(synth.round_bf16(rng.standard_normal((Tx, d))), "bf16")
     w = [synth.round_bf16(0.03 * rng.standard_normal((d, f))) for _ in range(3)]
     gu = ops.to_device_packed([ops.pack_gate_up(w[g % 2], w[(g + 1) % 3], "bf16")
@@ -428,18 +475,26 @@ def test_engine_permutation_across_batch_sizes(cuda, d, Ts):
 
 
 # ------------------------------------------------------------ decode path --
-@pytest.mark.parametrize("T,E,k,concept", [(32, 8, 2, False), (17, 8, 2, True), (1, 8, 2, False),
-                                           (5, 6, 3, False), (32, 5, 1, True)],
-                         ids=["T32", "T17_concept", "T1", "T5_E6_k3", "T32_E5_k1_concept"])
-def test_decode_path_bit_identical_to_routed_path(cuda, orc, T, E, k, concept):
-    # When one router workgroup covers the batch, the engine runs the router
-    # (and the permutation) inside a gate/up launch that covers every token
-    # of every expert, and the down GEMM gathers the routed rows.  An engine
+# T k selections above 64, 128 and 192: two to four windows of a wave in the down
+# launch's search for its rows.  f = 64 (2 j + 1), 128 j and (few tokens) 256 j: 2,
+# 4 and 8 K-steps per chunk there.
+@pytest.mark.parametrize("T,E,k,concept,f", [(32, 8, 2, False, 1280), (17, 8, 2, True, 1280),
+                                             (1, 8, 2, False, 1280), (5, 6, 3, False, 128),
+                                             (32, 5, 1, True, 128), (32, 8, 3, False, 192),
+                                             (29, 7, 5, True, 64), (32, 8, 8, False, 128),
+                                             (7, 8, 4, False, 320), (8, 6, 6, True, 256)],
+                         ids=["T32", "T17_concept", "T1", "T5_E6_k3", "T32_E5_k1_concept",
+                              "T32_k3_f192", "T29_E7_k5_f64", "T32_k8", "T7_k4_f320",
+                              "T8_E6_k6_f256"])
+def test_decode_path_bit_identical_to_routed_path(cuda, orc, T, E, k, concept, f):
+    # At most 32 tokens: the engine runs the router inside a gate/up launch
+    # that covers every token of every expert, and the down GEMM finds its
+    # rows and writes the permutation.  An engine
     # with the backward enabled keeps the routed stages (router, permutation,
     # routed gate/up, down).  Routing, the permutation, the stash's act and y
     # rows and the output are the same bits on both; the output is within
     # 2e-2 of the oracle.
-    d, f = (1536, 1280) if E == 8 and k == 2 else (256, 128)
+    d = 1536 if f == 1280 else 256
     inp = synth.make_moe_inputs(T=T, d=d, f=f, E=E, k=k, dtype="bf16", seed=100 + T + E,
                                 name=f"decode-T{T}-E{E}-k{k}")
     say("decode vs routed", T, E, k, concept)

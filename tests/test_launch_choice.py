@@ -39,6 +39,28 @@ def test_matmul_short_reductions(op):
             assert x.grid[0] == -(-c[0] // 64) * -(-c[1] // 64)
 
 
+def _matmul_kernel(x):
+    """Tile shape / elements per load of an f32 product's launch, or "short"."""
+    if x.kernel.startswith("f32_matmul_short_kernel<"):
+        return "short"
+    t = re.findall(r"Tile<(\d+), (\d+),[^>]*, (\d)>", x.kernel)
+    return f"{t[0][0]}x{t[0][1]}{'+halves' if t[0] != t[1] else ''}/{t[0][2]}"
+
+
+def test_cases_of_the_matmul_tiles():
+    # What the GPU test of the products' kernels launches; together every
+    # kernel with either kind of loads it has.
+    from tests.test_gpu_matmul import MATMUL_TILES
+
+    cases = [(op, M, N, R, by) for M, N, R, _, _ in MATMUL_TILES for by in (0, 4)
+             for op in sorted(OPS)]
+    want = [k for *_, k0, k1 in MATMUL_TILES for k in (k0, k1) for _ in OPS]
+    got = [_matmul_kernel(x) for x in _matmul_launches(cases)]
+    assert got == want, [(c, g, w) for c, g, w in zip(cases, got, want) if g != w]
+    shapes = {f"{t}/{w}" for t in ("128x128", "64x64", "32x64", "32x32", "16x16") for w in (1, 4)}
+    assert shapes | {"64x64+halves/4", "short"} == set(want)
+
+
 def test_matmul_largest_launches():
     # One output column (or row) of 2^27: 2^23 tiles of 16 x 16 with 512
     # threads would be 2^32 threads, more than a launch may have.
@@ -152,3 +174,85 @@ result = raw_events()
     kinds = {n.split("<")[0].split("::")[-1] for n, _ in seen}
     assert {"bf16_gemm_kernel", "wgrad_bf16_kernel", "wgrad_bf16_short_kernel",
             "router_topk_quad_kernel"} <= kinds, kinds
+
+
+def _rounds(x, counts, Np):
+    """(tile, whole rounds, last round in halves) of a grouped bf16 launch over
+    groups of `counts` rows and Np packed columns."""
+    bm, bn = _tiles(x)
+    tiles = sum(-(-c // bm) for c in counts) * (Np // bn)
+    whole, tail = divmod(tiles, x.grid[0])
+    cfgs = re.findall(r"Bf16Cfg<[^>]*>", x.kernel)
+    return (bm, bn), whole, cfgs[0] != cfgs[1] and 0 < 2 * tail <= x.grid[0]
+
+
+def test_cases_of_the_smaller_tiles():
+    # What the GPU tests of the 128 x 256 and 64 x 128 tiles launch, and that
+    # their reference launches take 256 x 256 tiles.
+    from tests.test_gpu_moe import MID_TILES, REF_ROWS
+
+    calls = []
+    for d, f, counts, _, _ in MID_TILES:
+        calls += [(d, f, len(counts), sum(counts)), (d, f, len(counts) + 1, REF_ROWS[d])]
+    rows = ll.as_launches(ll.run(f"""
+result = []
+for d, f, G, rows in {calls!r}:
+    L.check(lib.prichs_grouped_gate_up_swiglu(P, P, P, G, rows, P, d, f, L.DTYPE_BF16, P, None))
+    L.check(lib.prichs_grouped_down(P, P, G, rows, P, d, f, L.DTYPE_BF16, P, None))
+    result += launches()
+"""))
+    assert len(rows) == 4 * len(MID_TILES)
+    for (d, f, counts, gu, dn), (a, b, ra, rb) in zip(MID_TILES, zip(*[iter(rows)] * 4)):
+        np_gu, np_dn = -(-2 * f // 256) * 256, -(-d // 256) * 256
+        assert _rounds(a, counts, np_gu) == gu, (d, f, counts, a)
+        assert _rounds(b, counts, np_dn) == dn, (d, f, counts, b)
+        assert _tiles(ra) == _tiles(rb) == (256, 256), (d, f, counts)
+
+
+def test_cases_of_the_dense_tiles():
+    from tests.test_gpu_block import DENSE_TILES
+
+    rows = ll.as_launches(ll.run(f"""
+result = []
+for M, N in {sorted(DENSE_TILES)!r}:
+    L.check(lib.prichs_gemm(P, 1536, M, 1536, P, N, P, N, L.DTYPE_BF16, None))
+    result += launches()
+"""))
+    got = {}
+    for (M, N), x in zip(sorted(DENSE_TILES), rows):
+        tile, _, halves = _rounds(x, [M], -(-N // 256) * 256)
+        got[M, N] = (tile, halves)
+    assert got == DENSE_TILES
+
+
+def test_cases_of_the_f32_and_weight_gradient_kernels():
+    # The tiles and kernels that the GPU tests of the f32 grouped GEMMs and of
+    # the weight gradients say they take (gate/up and down; dW_down and
+    # dW_gate/up).
+    got = ll.run("""
+result = []
+for d, f, G, rows in [(48, 1008, 2, 1700), (2000, 48, 2, 1700), (80, 496, 2, 850), (112, 80, 6, 105)]:
+    L.check(lib.prichs_grouped_gate_up_swiglu(P, P, P, G, rows, P, d, f, L.DTYPE_F32, P, None))
+    L.check(lib.prichs_grouped_down(P, P, G, rows, P, d, f, L.DTYPE_F32, P, None))
+    result.append([x[0] for x in launches()])
+for T, d, f, E, k, dt in [(40, 1536, 1296, 3, 2, 0), (37, 656, 624, 3, 2, 0), (512, 256, 128, 8, 2, 0),
+                          (130, 448, 128, 2, 1, 1), (2600, 1536, 1280, 8, 2, 1),
+                          (3000, 256, 128, 4, 2, 1)]:
+    h = engine(d, f, E, k, dt, T, backward=True)
+    g = L.MoEGrads(P, P, P, P, d * f, 0)
+    L.check(lib.prichs_moe_engine_forward(h, P, T, None, 0, P, 0, None))
+    launches()
+    L.check(lib.prichs_moe_engine_backward(h, P, P, T, P, 0, C.byref(g), 2, None))
+    result.append([x[0] for x in launches() if x[0].startswith("wgrad_") and "reduce" not in x[0]])
+    L.check(lib.prichs_moe_engine_destroy(h))
+""")
+
+    def short(name):
+        t = re.search(r"Tile<(\d+), (\d+)", name)
+        return f"{t[1]}x{t[2]}" if t else name.split("<")[0]
+
+    assert [[short(n) for n in pair] for pair in got] == [
+        ["128x128", "32x64"], ["32x64", "128x128"], ["64x64", "32x64"], ["32x64", "32x64"],
+        ["128x128", "128x128"], ["64x64", "64x64"], ["32x64", "32x64"],
+        ["wgrad_bf16_short_kernel"] * 2, ["wgrad_bf16_kernel", "wgrad_bf16_short_kernel"],
+        ["wgrad_bf16_kernel"] * 2]
