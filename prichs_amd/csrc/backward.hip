@@ -494,10 +494,10 @@ __device__ __forceinline__ void wgrad_item(
   // of the wave's (BPT / 2) x 64 block.
   //
   // The tile leaves through the stage ring (idle after the last K-step), 128
-  // (S = 3: 64) rows of 1 KiB at a time: the waves holding them write their fragments to
-  // LDS (float4 chunk c of row r at c ^ (r & 15), no bank conflicts either
-  // way), then each wave stores 16 whole rows, one 1 KiB row per
-  // instruction, instead of 16 rows x 64 bytes per instruction.
+  // (S = 3: 64) rows of 1 KiB at a time: the waves holding them write their
+  // fragments to LDS (float4 chunk c of row r at c ^ (r & 15), no bank conflicts
+  // either way), then each wave stores 16 (S = 3: 8) whole rows, one 1 KiB row
+  // per instruction, instead of 16 rows x 64 bytes per instruction.
   const long long base = (long long)slot_of(g, E) * slot_stride;
   float *const pbase = pslot >= 0 ? part + (long long)pslot * P * Q : nullptr;
   const bool rmw = pslot < 0 && beta != 0;  // dW += tile (beta = 1, an unsplit group)
@@ -673,11 +673,12 @@ __global__ __launch_bounds__(wgb::kThreads) void wgrad_bf16_kernel(
 }
 
 // Short items (wgrad_short): most of an item's time is then its epilogue, whose
-// 256 KiB of f32 per 256 x 256 tile leave every CU at the same time.  One workgroup per (group, 128 x 256 tile), the shared group
-// first, three stages of LDS and at most 128 registers, so two share a CU and
-// one's stores run behind the other's products; no group is split, and a
-// group without rows writes its zeros (beta = 0) here, so there is no reduce
-// pass.  The same MFMA chain per element as the items above.
+// 256 KiB of f32 per 256 x 256 tile leave every CU at the same time.  One
+// workgroup per (group, 128 x 256 tile), the shared group first, three stages of
+// LDS and at most 128 registers, so two share a CU and one's stores run behind
+// the other's products; no group is split, and a group without rows writes its
+// zeros (beta = 0) here, so there is no reduce pass.  The same MFMA chain per
+// element as the items above.
 template <bool GATEUP>
 __global__ __launch_bounds__(wgb::kThreads, 4) void wgrad_bf16_short_kernel(
     const bf16_t *__restrict__ A, int lda, uint32_t a_bytes, const bf16_t *__restrict__ B,

@@ -174,7 +174,7 @@ extern "C" int prichs_moe_engine_create(size_t d, size_t f, size_t E, size_t k, 
   const size_t o_tr = c.take(sizeof(int32_t) * Tm * k);
   const size_t o_act = c.take(es * rows * f);
   const size_t o_y = c.take(es * rows * d);
-  // Decode buffers for batches one router workgroup covers (32 tokens).
+  // Decode buffers for batches of up to 32 tokens (decode_dense_applies).
   const size_t Td = (dtype == PRICHS_DTYPE_BF16 && n_shared == 1) ? std::min<size_t>(Tm, 32) : 0;
   const size_t o_actd = c.take(es * (E + 1) * Td * f + 1);
 

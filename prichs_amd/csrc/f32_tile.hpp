@@ -8,10 +8,11 @@
 //
 // Pipeline: global -> registers two stages of BK reduction elements ahead of
 // the products, registers -> one of two LDS buffers one stage ahead, one
-// barrier per stage; fragments LDS -> registers one 16-element slice ahead.  Loads are unpredicated (an address past the reduction
-// is replaced by the operand's first one and its value by zero at the LDS
-// store), so the compiler's waits stay exact and a stage's loads stay in
-// flight behind the whole of the previous stage's products.
+// barrier per stage; fragments LDS -> registers one 16-element slice ahead.
+// Loads are unpredicated (an address past the reduction is replaced by the
+// operand's first one and its value by zero at the LDS store), so the
+// compiler's waits stay exact and a stage's loads stay in flight behind the
+// whole of the previous stage's products.
 //
 // LDS: an RC operand keeps [row][BK] with 16-byte chunk c of row r at slot
 // c ^ (r & 7), so a fragment is read as one ds_read_b128 per lane (rows 0..7

@@ -20,7 +20,9 @@
 // through a ring of 4 LDS stages that global_load_lds_dwordx4 fills directly
 // (no staging registers), 3 stages ahead of the MFMAs; the two halves of the
 // workgroup ping-pong, one wave per SIMD multiplying while the other reads
-// its fragments and issues loads.  Workgroups are persistent and walk an
+// its fragments and issues loads.  Dense launches also take 128x384 and 256x288
+// tiles, launches with few rows 128x256 ones and, on a pipelined K loop of four
+// waves, 64x128 ones.  Workgroups are persistent and walk an
 // XCD-aware tile order.  The epilogues stage the finished tile in LDS and
 // write whole rows with 16-byte lanes (down / dense: the tile; gate/up: the
 // activations, or in the training forward the pre-activations, whose
@@ -296,8 +298,8 @@ using Bf16Small = Bf16Cfg<64, 128, 2, 2, 6>;
 // as its first operand, so each lane's accumulator holds 4 consecutive
 // output columns of one row (D[n][m] of v_mfma_f32_16x16x32_bf16), stored as
 // one 8-byte write.
-// Both bf16 configurations run the same number of waves, so the launch bound
-// is a constant (a bound that depends on a template parameter fails to
+// The bf16 configurations run 8 waves, 64 x 128 tiles 4: one constant launch
+// bound for all (a bound that depends on a template parameter fails to
 // substitute in the host pass).
 constexpr int kBf16Threads = 64 * PRICHS_BF16_WGM * PRICHS_BF16_WGN;
 
@@ -981,7 +983,10 @@ typedef f32t::Tile<64, 64, 32, 4, 1, 1, true, true> Medium;
 typedef f32t::Tile<32, 64, 64, 2, 1, 2, true, true> Small;
 
 // The shape with the least whole rounds of the chip x time.  The groups' last
-// M-tiles are half full on average (their row counts are on the device).
+// M-tiles are half full on average (their row counts are on the device).  Whole
+// rounds overrate shapes of which several share a CU: the 6144 rows of 9 groups
+// and 512 columns of a 2048-token training step (53 us per product) take 128 x
+// 128 tiles, 64 x 64 ones counting 3.2 rounds as 4.
 int tile_choice(size_t max_rows, int G, int Np, int cus) {
   int best = 0;
   double best_t = 0;
