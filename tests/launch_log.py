@@ -102,18 +102,45 @@ def engine(d, f, E, k, dtype, max_tokens, backward=False):
     return h
 
 
+def _unpack(b, i):
+    """The MessagePack value at b[i] and the index past it (what code object
+    metadata holds: maps, arrays, texts, whole numbers, truth values)."""
+    t = b[i]
+    i += 1
+
+    def number(n):
+        return int.from_bytes(b[i:i + n], "big"), i + n
+
+    if t < 0x80:
+        return t, i
+    if t in (0xc2, 0xc3):
+        return t == 0xc3, i
+    if 0xcc <= t <= 0xcf:
+        return number(1 << (t - 0xcc))
+    if t >> 5 == 5:
+        n = t & 31
+    elif t >> 5 == 4:
+        n = t & 15
+    else:
+        n, i = number({0xd9: 1, 0xda: 2, 0xdb: 4, 0xdc: 2, 0xdd: 4, 0xde: 2, 0xdf: 4}[t])
+    if t >> 5 == 5 or 0xd9 <= t <= 0xdb:
+        return b[i:i + n].decode(), i + n
+    is_map, items = t >> 4 == 8 or t >= 0xde, []
+    for _ in range(2 * n if is_map else n):
+        v, i = _unpack(b, i)
+        items.append(v)
+    return (dict(zip(items[::2], items[1::2])) if is_map else items), i
+
+
 def static_lds(library=os.environ.get("PRICHS_HIP_LIB") or os.path.join(
         ROOT, "prichs_amd", "libprichs_hip.so")):
     """Bytes of LDS that each kernel of the library has at launch (besides its
     dynamic LDS), by symbol, from its code objects' metadata."""
-    import msgpack
-
     data, out, at = open(library, "rb").read(), {}, 0
     key = b"\xaeamdhsa.kernels"
     while (at := data.find(key, at)) >= 0:
-        u = msgpack.Unpacker(strict_map_key=False)
-        u.feed(data[at - 1:at + (8 << 20)])
-        for k in u.unpack()["amdhsa.kernels"]:
+        kernels, _ = _unpack(data, at + len(key))
+        for k in kernels:
             out[k[".name"]] = k[".group_segment_fixed_size"]
         at += len(key)
     return out
