@@ -254,16 +254,18 @@ bool matmul_halves(size_t M, size_t N, int cus, size_t &full) {
 }
 
 // Configuration 6: the kernel for short reductions.  Before its first products a
-// pipelined tile fetches and stores its stages, as long as 2 stages of
-// products with 16-byte loads and 4 with single elements; the short kernel has
-// no such start but takes longer per element, 46 ns per 64 x 64 tile of
-// several on a CU and 62 of one alone.  MI355X, us, pipelined -> short: 4096 x
-// 4096 outputs of 16 elements 24.5 -> 18.2, 3000 x 3001 of 17 43.2 -> 15.4, 341
-// x 3005 of 1 13.8 -> 4.7, 1341 x 1245 of 91 21.0 -> 9.8; on small outputs the
+// pipelined tile fetches and stores its stages, as long as the products of 98
+// reduction elements with 16-byte loads and of 224 with single ones; the short
+// kernel has no such start but takes longer per element, 9 ns and 42.5 for each
+// 64 x 64 tile on a CU (partly filled rounds count three quarters as whole ones).
+// Fitted to 2919 measured sizes; the choice is the slower one by more than 8% on
+// 3 of them.  MI355X, us, pipelined -> short: 4096 x 4096 outputs of 16 elements
+// 24.5 -> 18.2, 3000 x 3001 of 17 43.2 -> 15.4, 341 x 3005 of 1 13.8 -> 4.7, 1341
+// x 1245 of 91 21.0 -> 9.8, 936 x 1140 of 613 31.2 -> 46.6; on small outputs the
 // two meet near 40 elements with single-element loads and near 16 with 16-byte
 // ones (60 x 84 of 64: 3.9 -> 6.0).
 constexpr int kMatmulShort = 6;
-constexpr double kShortAlone = 62.0, kShortShared = 46.0, kFillStages[2] = {2.0, 4.0};
+constexpr double kShortBase = 9.0, kShortTileCost = 42.5, kFillElems[2] = {98.0, 224.0};
 
 int matmul_cfg(size_t M, size_t N, size_t R, bool vec, int cus) {
   int best = 0, bk = 0;
@@ -282,9 +284,10 @@ int matmul_cfg(size_t M, size_t N, size_t R, bool vec, int cus) {
     if ((double)roundup(R, 32) * e < best_t) best = 5, per = e, bk = 32;
   }
   const double tiles = (double)cdiv(M, kShortTile) * (double)cdiv(N, kShortTile);
+  const double rounds = std::max(1.0, 0.25 * tiles / cus + 0.75 * std::ceil(tiles / cus));
   if (tiles * kShortThreads <= kMaxLaunchThreads &&
-      (double)roundup(R, kShortStep) * std::max(kShortAlone, tiles / cus * kShortShared) <
-      ((double)roundup(R, bk) + kFillStages[!vec] * bk) * per)
+      (double)roundup(R, kShortStep) * (kShortBase + kShortTileCost * rounds) <
+          ((double)roundup(R, bk) + kFillElems[!vec]) * per)
     return kMatmulShort;
   return best;
 }

@@ -199,8 +199,8 @@ def test_matmul_device_entry_on_stream_and_big_reduction(cuda, orc):
 # tiles, elements per load, or the kernel for short reductions.  They end inside
 # a tile and inside a reduction step.
 MATMUL_TILES = [
-    (2044, 2040, 36, "128x128/4", "short"),
-    (2044, 2040, 132, "128x128/4", "128x128/1"),
+    (2044, 2040, 36, "short", "short"),
+    (2044, 2040, 132, "128x128/4", "short"),
     (1999, 2001, 333, "128x128/1", "128x128/1"),
     (1999, 2001, 33, "short", "short"),
     (1000, 1020, 100, "64x64/4", "short"),

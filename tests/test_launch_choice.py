@@ -31,7 +31,8 @@ def test_matmul_short_reductions(op):
     short = [(4096, 4096, 16, 0), (3000, 3001, 17, 0), (1341, 1245, 91, 0), (341, 3005, 1, 0),
              (16, 16, 16, 0), (1, 1, 1, 0), (2044, 2040, 8, 4)]
     tiles = [(2048, 1280, 1536, 0), (60, 84, 64, 0), (2000, 2000, 64, 0), (1024, 1024, 1024, 4),
-             (101, 103, 151, 0), (16, 16, 512, 0)]
+             (101, 103, 151, 0), (16, 16, 512, 0), (936, 1140, 613, 0), (3645, 379, 601, 0),
+             (1721, 826, 662, 0)]
     got = _matmul_launches([(op, *c) for c in short + tiles])
     for c, x in zip(short + tiles, got):
         assert x.kernel.startswith("f32_matmul_short_kernel<") == (c in short), (c, x.kernel)
